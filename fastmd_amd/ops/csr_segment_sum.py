@@ -41,15 +41,55 @@ class Csr:
         return int(self.off.shape[0]) - 1
 
 
-def csr_from_segment(segment: Tensor, num_segment: int) -> Csr:
-    """The CSR of an arbitrary segment index (stable order within a segment). Host plumbing:
-    torch's stable sort and a count; the hot path gets its CSRs from the neighbour list."""
+def _csr_by_sort(segment: Tensor, num_segment: int) -> Csr:
+    """The CSR by torch's stable sort and a count (tensors that the kernels do not take)."""
     segment = segment.long()
     perm = torch.argsort(segment, stable=True).to(torch.int32)
     counts = torch.bincount(segment, minlength=num_segment)[:num_segment]
     off = torch.zeros(num_segment + 1, dtype=torch.int64, device=segment.device)
     torch.cumsum(counts, 0, out=off[1:])
     return Csr(off, perm)
+
+
+def csr_from_segments(pairs) -> tuple[list[Csr], Tensor | None]:
+    """The CSRs of up to two ``(segment, num_segment)`` pairs by fmd_csr_from_index (shared launches,
+    no host read), and the device flags of negative indices, which the caller gives to
+    ``refuse_negative`` once its other launches are queued (None: nothing left to check)."""
+    if not all(s.is_cuda and s.dim() == 1 and s.dtype in (torch.int32, torch.int64) and s.device == pairs[0][0].device
+               and max(s.numel(), n) < 2 ** 31 - 1 and n >= 0 for s, n in pairs):
+        return [_csr_by_sort(s, n) for s, n in pairs], None
+    dev = pairs[0][0].device
+    out, work, perms, offs = [], [], [], []
+    sizes = [int(_abi.load().fmd_csr_work_size(s.numel())) for s, _ in pairs]
+    scratch = torch.empty(sum(sizes) + len(pairs), dtype=torch.int32, device=dev)
+    flags = scratch[sum(sizes):]
+    for (s, n), start in zip(pairs, (0, sizes[0])):
+        off = torch.empty(n + 1, dtype=torch.int64, device=dev)
+        perm = torch.empty(s.numel(), dtype=torch.int32, device=dev)
+        out.append(Csr(off, perm))
+        perms.append(perm.data_ptr())
+        offs.append(off.data_ptr())
+        work.append(scratch.data_ptr() + 4 * start)
+    _abi.call("fmd_csr_from_index", len(pairs), _abi.ptr_array([s.data_ptr() for s, _ in pairs]),
+              _abi.array(_abi._i32, [s.dtype == torch.int64 for s, _ in pairs]),
+              _abi.array(_abi._i64, [s.stride(0) for s, _ in pairs]),
+              _abi.array(_abi._i64, [s.numel() for s, _ in pairs]), _abi.array(_abi._i64, [n for _, n in pairs]),
+              _abi.ptr_array(perms), _abi.ptr_array(offs), _abi.ptr_array(work), flags.data_ptr(), stream())
+    return out, flags
+
+
+def refuse_negative(flags: Tensor | None) -> None:
+    """RuntimeError for a negative segment index (one host read of the flags)."""
+    if flags is not None and any(flags.tolist()):
+        raise RuntimeError("a segment index must be non-negative")
+
+
+def csr_from_segment(segment: Tensor, num_segment: int) -> Csr:
+    """The CSR of an arbitrary segment index (stable order within a segment). The hot path gets
+    its CSRs from the neighbour list; this one serves the operators called with a plain index."""
+    (csr,), flags = csr_from_segments([(segment, int(num_segment))])
+    refuse_negative(flags)
+    return csr
 
 
 def _prep_off(off: Tensor) -> Tensor:
@@ -197,11 +237,14 @@ def csr_segment_sum(value: Tensor, segment: Tensor | None, num_segment: int, per
     require_cuda(value, weight, segment, perm, off)
     if value.dtype != torch.float32:
         raise ValueError("csr_segment_sum: float32 values only")
+    flags = None
     if identity_perm:
         perm = None
     elif perm is None or off is None:
         if segment is None:
             raise ValueError("a segment index or a CSR is required")
-        csr = csr_from_segment(segment, num_segment)
+        (csr,), flags = csr_from_segments([(segment, num_segment)])
         perm, off = csr.perm, csr.off
-    return _CsrSegmentSum.apply(value, weight, num_segment, _prep_off(off), _prep_perm(perm), skip_segment)
+    out = _CsrSegmentSum.apply(value, weight, num_segment, _prep_off(off), _prep_perm(perm), skip_segment)
+    refuse_negative(flags)
+    return out

@@ -21,7 +21,7 @@ from torch.autograd import Function
 
 from fastmd_amd import _abi
 from fastmd_amd._device import require_cuda, rows_view, stream
-from fastmd_amd.ops.csr_segment_sum import Csr, csr_from_segment, segment_sum_csr
+from fastmd_amd.ops.csr_segment_sum import Csr, csr_from_segments, refuse_negative, segment_sum_csr
 
 
 def _launch(parts, rows: int, out: Tensor) -> None:
@@ -51,10 +51,6 @@ def _launch(parts, rows: int, out: Tensor) -> None:
     _abi.call("fmd_gather_cat_f32", len(parts), _abi.ptr_array(srcs), _abi.ptr_array(idx),
               _abi.array(_abi._i64, strides), _abi.array(_abi._i64, lds), _abi.array(_abi._i32, widths), rows, out.data_ptr(), out.stride(0),
               stream())
-
-
-def _csr_for(index: Tensor, num_rows: int, csr: Csr | None) -> Csr:
-    return csr if csr is not None else csr_from_segment(index, num_rows)
 
 
 class _GatherCat(Function):
@@ -93,6 +89,7 @@ class _GatherCat(Function):
             indices.append(saved.pop(0) if kind == "g" else None)
         # group gathered blocks by source tensor identity so a shared source sums both blocks
         results: dict[int, Tensor] = {}
+        flags = []
         cols = []
         for kind, shape in zip(ctx.kinds, ctx.shapes):
             cols.append(col)
@@ -108,15 +105,22 @@ class _GatherCat(Function):
             if sid in results:
                 grads += [None, None]  # already summed into the first block of this source
                 continue
-            terms = []
-            for q, (kq, sq) in enumerate(zip(ctx.kinds, ctx.shapes)):
-                if kq == "g" and ctx.src_ids[q] == sid:
-                    terms.append((gout, _csr_for(indices[q], sq[0], ctx.csrs[q]), cols[q], 1.0, None))
+            blocks = [q for q, kq in enumerate(ctx.kinds) if kq == "g" and ctx.src_ids[q] == sid]
+            csrs = {q: ctx.csrs[q] for q in blocks if ctx.csrs[q] is not None}
+            plain = [q for q in blocks if q not in csrs]
+            for start in range(0, len(plain), 2):  # the CSRs of plain indices, two per launch sequence
+                pair = plain[start:start + 2]
+                made, negative = csr_from_segments([(indices[q], ctx.shapes[q][0]) for q in pair])
+                csrs.update(zip(pair, made))
+                flags.append(negative)
+            terms = [(gout, csrs[q], cols[q], 1.0, None) for q in blocks]
             out = None
             for start in range(0, len(terms), 2):
                 out = segment_sum_csr(terms[start:start + 2], shape[0], shape[1], out=out, accumulate=start > 0)
             results[sid] = out
             grads += [out, None]
+        for negative in flags:
+            refuse_negative(negative)
         return (None, None, *grads)
 
 

@@ -9,7 +9,7 @@
 * ``aggregate(data, segment, bin_count=None, average=True, num_segment=None)``: the segment sum of
   the rows, divided by the (zero-clamped-to-one) counts when ``average`` (segment.py:97-133).
 
-Every sum runs through a CSR of ``segment`` (a stable sort; rows of a segment in index order) and
+Every sum runs through a CSR of ``segment`` (in stable order: rows of a segment in index order) and
 the fixed-order segment-sum kernel, so results are bitwise reproducible run to run. GPU tensors
 only, like the rest of the operator layer.
 """
@@ -19,7 +19,7 @@ import torch
 from torch import Tensor
 
 from fastmd_amd._device import require_cuda
-from fastmd_amd.ops.csr_segment_sum import csr_from_segment, csr_segment_sum
+from fastmd_amd.ops.csr_segment_sum import csr_from_segments, csr_segment_sum, refuse_negative
 
 
 def _offsets(segment: Tensor, num_segment: int) -> Tensor:
@@ -49,8 +49,10 @@ def weighted_segment_sum(weight: Tensor, value: Tensor, segment: Tensor, num_seg
             raise ValueError(f"weight must be {tuple(value.shape)} or ({value.shape[0]}, 1), got {tuple(weight.shape)}")
         weight = weight.expand_as(value).contiguous()
     num_segment = int(num_segment)
-    csr = csr_from_segment(segment, num_segment)
-    return csr_segment_sum(value, segment, num_segment, perm=csr.perm, off=csr.off, weight=weight)
+    (csr,), flags = csr_from_segments([(segment, num_segment)])
+    out = csr_segment_sum(value, segment, num_segment, perm=csr.perm, off=csr.off, weight=weight)
+    refuse_negative(flags)
+    return out
 
 
 def aggregate(data: Tensor, segment: Tensor, bin_count: Tensor | None = None, average: bool = True,
@@ -64,8 +66,9 @@ def aggregate(data: Tensor, segment: Tensor, bin_count: Tensor | None = None, av
         if bin_count is not None:
             num_segment = max(num_segment, int(bin_count.shape[0]))
     num_segment = int(num_segment)
-    csr = csr_from_segment(segment, num_segment)
+    (csr,), flags = csr_from_segments([(segment, num_segment)])
     out = csr_segment_sum(data, segment, num_segment, perm=csr.perm, off=csr.off)
+    refuse_negative(flags)
     if not average:
         return out
     if bin_count is None:

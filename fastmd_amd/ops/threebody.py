@@ -29,7 +29,7 @@ from torch.autograd import Function
 
 from fastmd_amd import _abi
 from fastmd_amd._device import require_cuda, rows_view, stream
-from fastmd_amd.ops.csr_segment_sum import csr_from_segment, segment_sum_csr
+from fastmd_amd.ops.csr_segment_sum import csr_from_segments, refuse_negative, segment_sum_csr
 
 MAX_FREQ = 16
 
@@ -107,8 +107,9 @@ def fourier_basis_vjp(gout: Tensor, unit_vec: Tensor, target_index: Tensor, sour
     contrib = torch.empty((rows, 6), dtype=torch.float32, device=device)
     _abi.call("fmd_threebody_fourier_bwd_rows_f32", g.data_ptr(), u.data_ptr(), ld, tgt.data_ptr(), src.data_ptr(),
               rows, f.data_ptr(), f.numel(), float(scale), contrib.data_ptr(), stream())
-    segment_sum_csr([(contrib, csr_from_segment(tgt, n_vec), 0, 1.0, None),
-                     (contrib, csr_from_segment(src, n_vec), 3, 1.0, None)], n_vec, 3, out=grad)
+    (by_target, by_source), flags = csr_from_segments([(tgt, n_vec), (src, n_vec)])
+    segment_sum_csr([(contrib, by_target, 0, 1.0, None), (contrib, by_source, 3, 1.0, None)], n_vec, 3, out=grad)
+    refuse_negative(flags)
     return grad
 
 
