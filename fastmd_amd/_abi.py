@@ -64,7 +64,7 @@ SIGNATURES: dict[str, tuple] = {
     "fmd_segsum_csr_f32": (ctypes.c_int, [_i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i32,
                                           _p, _i64, _p]),
     "fmd_csr_work_size": (_i64, [_i64]),
-    "fmd_csr_from_index": (ctypes.c_int, [_i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
+    "fmd_csr_from_index": (ctypes.c_int, [_i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "fmd_segsum_csr_t_f32": (ctypes.c_int, [_p, _i64, _p, _p, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, _p,
                                             _p]),
     "fmd_gemm_f32": (ctypes.c_int, [_p, _i64, _p, _i64, _i32, _p, _p, _i64, _i64, _i64, _i64, _i32, _i32, _p]),

@@ -12,9 +12,12 @@
 //     (each scatter workgroup sums the chunk histograms itself, so there is no scan launch), then
 //     one search per segment over the sorted keys. Up to two indices share the launches.
 // Bound by launches and dependent loads, not by bytes (160 000 rows: 8 MB in all): the two CSRs of a
-// gather-cat VJP at 160 000 rows, 10 000 segments are 5 launches where torch's sort, bincount and
-// cumsum were 44. Measured: that forward and VJP at F = 128 523 -> 279 us, the Fourier basis and
-// its VJP at 107 520 triplets 512 -> 236 us, one edge block at 135 atoms (three CSRs) 679 -> 444 us.
+// gather-cat VJP at 160 000 rows, 10 000 segments are 5 launches (45 us) where torch's sort, bincount
+// and cumsum were 44 (275 us). Measured whole: that forward and VJP at F = 128 453 -> 222 us, the Fourier
+// basis and its VJP at 107 520 triplets 511 -> 213 us, one edge block at 135 atoms (three CSRs)
+// 751 -> 419 us. The flag of negative indices goes to host memory from the first kernel, behind an
+// event of its own: waiting for the whole sequence instead left the GPU idle between calls (279, 236
+// and 444 us).
 #include "common.h"
 
 namespace {
@@ -37,11 +40,10 @@ struct Job {
   int32_t nseg;
   int32_t* perm;
   int64_t* off;
-  int32_t* negative;   // [1]: some index is negative
+  int32_t* negative;   // set to 1 if some index is negative (host memory the device can write)
   uint32_t* key[2];    // [rows] each
   int32_t* row[2];     // [rows] each
   uint32_t* hist;      // [chunks][kDigits]
-  int32_t* chunk_neg;  // [chunks]
   int chunks;
   int32_t chunk_rows;  // a multiple of kThreads
   int passes;
@@ -61,6 +63,12 @@ __device__ __forceinline__ uint32_t row_key(const Job& j, int64_t r, bool& neg) 
   return v < 0 || v > j.nseg ? (uint32_t)j.nseg : (uint32_t)v;
 }
 
+// The flag is the caller's to read once the first launch has run: a store past the caches, to host
+// memory, only from workgroups that saw a negative index.
+__device__ __forceinline__ void flag_negative(const Job& j) {
+  __hip_atomic_store(j.negative, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // the lanes of the wave (among `active`) whose digit is this lane's
 __device__ __forceinline__ uint64_t same_digit(uint32_t digit, int bits, uint64_t active) {
   uint64_t m = active;
@@ -76,10 +84,8 @@ __global__ void __launch_bounds__(kThreads) csr_hist_kernel(const Jobs jobs, int
   const Job& j = jobs.j[blockIdx.y];
   if (pass >= j.passes || (int)blockIdx.x >= j.chunks) return;
   __shared__ uint32_t s_hist[kDigits];
-  __shared__ int s_neg;
   const int t = threadIdx.x;
   s_hist[t] = 0;
-  if (t == 0) s_neg = 0;
   __syncthreads();
   const int shift = pass * j.bits;
   const uint32_t mask = (1u << j.bits) - 1;
@@ -97,10 +103,9 @@ __global__ void __launch_bounds__(kThreads) csr_hist_kernel(const Jobs jobs, int
     for (int g = 0; g < kGroups; ++g)
       if (r0 + g * kThreads < hi) atomicAdd(&s_hist[(key[g] >> shift) & mask], 1u);
   }
-  if (neg) s_neg = 1;
+  if (neg) flag_negative(j);
   __syncthreads();
   j.hist[(int64_t)blockIdx.x * kDigits + t] = s_hist[t];
-  if (pass == 0 && t == 0) j.chunk_neg[blockIdx.x] = s_neg;
 }
 
 // Scatter of one chunk: the digit bases from the chunk histograms (thread d: digit d), the waves'
@@ -130,15 +135,19 @@ __global__ void __launch_bounds__(kThreads) csr_scatter_kernel(const Jobs jobs, 
       if (r0 + g * FMD_WAVE < end) atomicAdd(&s_base[wave][(key[g] >> shift) & mask], 1u);
   }
   uint32_t before = 0, total = 0;
-  constexpr int kLoads = 8;  // histogram rows in flight per thread
+  // histogram rows in flight per thread (8 left 20 dependent round trips at 160 000 rows)
+  constexpr int kLoads = 32;
   for (int c0 = 0; c0 < j.chunks; c0 += kLoads) {
     uint32_t v[kLoads];
 #pragma unroll
-    for (int u = 0; u < kLoads; ++u) v[u] = c0 + u < j.chunks ? j.hist[(int64_t)(c0 + u) * kDigits + t] : 0;
+    for (int u = 0; u < kLoads; ++u) {  // clamped, not predicated: no branch between the loads
+      const int c = c0 + u < j.chunks ? c0 + u : j.chunks - 1;
+      v[u] = j.hist[c * kDigits + t];
+    }
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
-      total += v[u];
-      if (c0 + u < (int)blockIdx.x) before += v[u];
+      total += c0 + u < j.chunks ? v[u] : 0;
+      before += c0 + u < (int)blockIdx.x ? v[u] : 0;
     }
   }
   uint32_t all;
@@ -197,12 +206,6 @@ __global__ void __launch_bounds__(kThreads) csr_offsets_kernel(const Jobs jobs) 
   const Job& j = jobs.j[blockIdx.y];
   const int64_t s = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (s <= j.nseg) j.off[s] = lower_bound(j.key[(j.passes - 1) & 1], j.rows, (uint32_t)s);
-  if (blockIdx.x == 0 && threadIdx.x < FMD_WAVE) {
-    int neg = 0;
-    for (int c = threadIdx.x; c < j.chunks; c += FMD_WAVE) neg |= j.chunk_neg[c];
-    const uint64_t any = __ballot(neg != 0);
-    if (threadIdx.x == 0) j.negative[0] = any != 0;
-  }
 }
 
 // One workgroup per index: the same passes on (key, row) pairs in LDS.
@@ -212,17 +215,14 @@ __global__ void __launch_bounds__(kSmallThreads) csr_small_kernel(const Jobs job
   __shared__ uint16_t s_row[2][kSmallRows];
   __shared__ uint32_t s_base[kSmallWaves][kDigits];
   __shared__ uint32_t s_scan[17];
-  __shared__ int s_neg;
   const int t = threadIdx.x, lane = t & (FMD_WAVE - 1), wave = t / FMD_WAVE;
   const int rows = j.rows;
-  if (t == 0) s_neg = 0;
-  __syncthreads();
   bool neg = false;
   for (int r = t; r < rows; r += kSmallThreads) {
     s_key[0][r] = row_key(j, r, neg);
     s_row[0][r] = (uint16_t)r;
   }
-  if (neg) s_neg = 1;
+  if (neg) flag_negative(j);
   // a wave's contiguous share, in groups of 64 rows
   const int wave_rows = (int)fmd_cdiv(rows, kSmallThreads) * FMD_WAVE;
   const int lo = wave * wave_rows, end = lo + wave_rows < rows ? lo + wave_rows : rows;
@@ -264,7 +264,6 @@ __global__ void __launch_bounds__(kSmallThreads) csr_small_kernel(const Jobs job
   const int fin = j.passes & 1;
   for (int r = t; r < rows; r += kSmallThreads) j.perm[r] = s_row[fin][r];
   for (int64_t s = t; s <= j.nseg; s += kSmallThreads) j.off[s] = lower_bound(s_key[fin], rows, (uint32_t)s);
-  if (t == 0) j.negative[0] = s_neg;
 }
 
 }  // namespace
@@ -272,12 +271,12 @@ __global__ void __launch_bounds__(kSmallThreads) csr_small_kernel(const Jobs job
 extern "C" {
 
 int64_t fmd_csr_work_size(int64_t rows) {
-  return 4 * (rows > 0 ? rows : 0) + kMaxChunks * (kDigits + 1);
+  return 4 * (rows > 0 ? rows : 0) + kMaxChunks * kDigits;
 }
 
 int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* is64, const int64_t* stride,
                        const int64_t* rows, const int64_t* num_segment, int32_t* const* perm, int64_t* const* off,
-                       uint32_t* const* work, int32_t* negative, hipStream_t stream) {
+                       uint32_t* const* work, int32_t* negative, hipEvent_t checked, hipStream_t stream) {
   FMD_REQUIRE(count >= 1 && count <= 2 && index && is64 && stride && rows && num_segment && perm && off && work);
   FMD_REQUIRE(negative);
   Jobs jobs{};
@@ -307,7 +306,7 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
   if (small) {
     hipLaunchKernelGGL(csr_small_kernel, dim3(1, (unsigned)count), dim3(kSmallThreads), 0, stream, jobs);
     FMD_CHECK_LAUNCH();
-    return FMD_OK;
+    return checked ? (int)hipEventRecord(checked, stream) : FMD_OK;
   }
   for (int q = 0; q < count; ++q) {
     Job& j = jobs.j[q];
@@ -324,12 +323,15 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
     j.row[0] = reinterpret_cast<int32_t*>(work[q] + 2 * n);
     j.row[1] = reinterpret_cast<int32_t*>(work[q] + 3 * n);
     j.hist = work[q] + 4 * n;
-    j.chunk_neg = reinterpret_cast<int32_t*>(j.hist + kMaxChunks * kDigits);
     chunks = j.chunks > chunks ? j.chunks : chunks;
   }
   for (int p = 0; p < passes; ++p) {
     hipLaunchKernelGGL(csr_hist_kernel, dim3((unsigned)chunks, (unsigned)count), dim3(kThreads), 0, stream, jobs, p);
     FMD_CHECK_LAUNCH();
+    if (p == 0 && checked) {  // every index has been read
+      const hipError_t err = hipEventRecord(checked, stream);
+      if (err != hipSuccess) return (int)err;
+    }
     hipLaunchKernelGGL(csr_scatter_kernel, dim3((unsigned)chunks, (unsigned)count), dim3(kThreads), 0, stream, jobs, p);
     FMD_CHECK_LAUNCH();
   }

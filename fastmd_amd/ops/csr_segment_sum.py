@@ -51,18 +51,42 @@ def _csr_by_sort(segment: Tensor, num_segment: int) -> Csr:
     return Csr(off, perm)
 
 
-def csr_from_segments(pairs) -> tuple[list[Csr], Tensor | None]:
+class _NegativeCheck:
+    """Whether an index of a CSR launch is negative: flags in pinned host memory that its first kernel
+    writes, and the event behind that kernel. ``refuse`` waits for that kernel only, with the rest of
+    the caller's launches queued; the flags outlive the kernel in any case."""
+
+    __slots__ = ("flags", "event")
+
+    def __init__(self, count: int) -> None:
+        self.flags = torch.zeros(count, dtype=torch.int32, pin_memory=True)
+        self.event = torch.cuda.Event()
+        self.event.record()  # creates the event; the launch records it again where it belongs
+
+    def refuse(self) -> None:
+        """RuntimeError for a negative segment index."""
+        self.event.synchronize()
+        if any(self.flags.tolist()):
+            raise RuntimeError("a segment index must be non-negative")
+
+    def __del__(self) -> None:
+        event = getattr(self, "event", None)
+        if event is not None and not event.query():
+            event.synchronize()
+
+
+def csr_from_segments(pairs) -> tuple[list[Csr], _NegativeCheck | None]:
     """The CSRs of up to two ``(segment, num_segment)`` pairs by fmd_csr_from_index (shared launches,
-    no host read), and the device flags of negative indices, which the caller gives to
-    ``refuse_negative`` once its other launches are queued (None: nothing left to check)."""
+    no host read), and their check, which the caller passes to ``refuse_negative`` once its other
+    launches are queued (None: nothing left to check)."""
     if not all(s.is_cuda and s.dim() == 1 and s.dtype in (torch.int32, torch.int64) and s.device == pairs[0][0].device
                and max(s.numel(), n) < 2 ** 31 - 1 and n >= 0 for s, n in pairs):
         return [_csr_by_sort(s, n) for s, n in pairs], None
     dev = pairs[0][0].device
     out, work, perms, offs = [], [], [], []
     sizes = [int(_abi.load().fmd_csr_work_size(s.numel())) for s, _ in pairs]
-    scratch = torch.empty(sum(sizes) + len(pairs), dtype=torch.int32, device=dev)
-    flags = scratch[sum(sizes):]
+    scratch = torch.empty(sum(sizes), dtype=torch.int32, device=dev)
+    check = _NegativeCheck(len(pairs))
     for (s, n), start in zip(pairs, (0, sizes[0])):
         off = torch.empty(n + 1, dtype=torch.int64, device=dev)
         perm = torch.empty(s.numel(), dtype=torch.int32, device=dev)
@@ -74,21 +98,21 @@ def csr_from_segments(pairs) -> tuple[list[Csr], Tensor | None]:
               _abi.array(_abi._i32, [s.dtype == torch.int64 for s, _ in pairs]),
               _abi.array(_abi._i64, [s.stride(0) for s, _ in pairs]),
               _abi.array(_abi._i64, [s.numel() for s, _ in pairs]), _abi.array(_abi._i64, [n for _, n in pairs]),
-              _abi.ptr_array(perms), _abi.ptr_array(offs), _abi.ptr_array(work), flags.data_ptr(), stream())
-    return out, flags
+              _abi.ptr_array(perms), _abi.ptr_array(offs), _abi.ptr_array(work), check.flags.data_ptr(),
+              check.event.cuda_event, stream())
+    return out, check
 
 
-def refuse_negative(flags: Tensor | None) -> None:
-    """RuntimeError for a negative segment index (one host read of the flags)."""
-    if flags is not None and any(flags.tolist()):
-        raise RuntimeError("a segment index must be non-negative")
+def refuse_negative(check: _NegativeCheck | None) -> None:
+    if check is not None:
+        check.refuse()
 
 
 def csr_from_segment(segment: Tensor, num_segment: int) -> Csr:
     """The CSR of an arbitrary segment index (stable order within a segment). The hot path gets
     its CSRs from the neighbour list; this one serves the operators called with a plain index."""
-    (csr,), flags = csr_from_segments([(segment, int(num_segment))])
-    refuse_negative(flags)
+    (csr,), check = csr_from_segments([(segment, int(num_segment))])
+    refuse_negative(check)
     return csr
 
 
@@ -237,14 +261,14 @@ def csr_segment_sum(value: Tensor, segment: Tensor | None, num_segment: int, per
     require_cuda(value, weight, segment, perm, off)
     if value.dtype != torch.float32:
         raise ValueError("csr_segment_sum: float32 values only")
-    flags = None
+    check = None
     if identity_perm:
         perm = None
     elif perm is None or off is None:
         if segment is None:
             raise ValueError("a segment index or a CSR is required")
-        (csr,), flags = csr_from_segments([(segment, num_segment)])
+        (csr,), check = csr_from_segments([(segment, num_segment)])
         perm, off = csr.perm, csr.off
     out = _CsrSegmentSum.apply(value, weight, num_segment, _prep_off(off), _prep_perm(perm), skip_segment)
-    refuse_negative(flags)
+    refuse_negative(check)
     return out

@@ -89,7 +89,7 @@ class _GatherCat(Function):
             indices.append(saved.pop(0) if kind == "g" else None)
         # group gathered blocks by source tensor identity so a shared source sums both blocks
         results: dict[int, Tensor] = {}
-        flags = []
+        checks = []
         cols = []
         for kind, shape in zip(ctx.kinds, ctx.shapes):
             cols.append(col)
@@ -110,17 +110,17 @@ class _GatherCat(Function):
             plain = [q for q in blocks if q not in csrs]
             for start in range(0, len(plain), 2):  # the CSRs of plain indices, two per launch sequence
                 pair = plain[start:start + 2]
-                made, negative = csr_from_segments([(indices[q], ctx.shapes[q][0]) for q in pair])
+                made, check = csr_from_segments([(indices[q], ctx.shapes[q][0]) for q in pair])
                 csrs.update(zip(pair, made))
-                flags.append(negative)
+                checks.append(check)
             terms = [(gout, csrs[q], cols[q], 1.0, None) for q in blocks]
             out = None
             for start in range(0, len(terms), 2):
                 out = segment_sum_csr(terms[start:start + 2], shape[0], shape[1], out=out, accumulate=start > 0)
             results[sid] = out
             grads += [out, None]
-        for negative in flags:
-            refuse_negative(negative)
+        for check in checks:
+            refuse_negative(check)
         return (None, None, *grads)
 
 

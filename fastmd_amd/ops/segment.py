@@ -49,9 +49,9 @@ def weighted_segment_sum(weight: Tensor, value: Tensor, segment: Tensor, num_seg
             raise ValueError(f"weight must be {tuple(value.shape)} or ({value.shape[0]}, 1), got {tuple(weight.shape)}")
         weight = weight.expand_as(value).contiguous()
     num_segment = int(num_segment)
-    (csr,), flags = csr_from_segments([(segment, num_segment)])
+    (csr,), check = csr_from_segments([(segment, num_segment)])
     out = csr_segment_sum(value, segment, num_segment, perm=csr.perm, off=csr.off, weight=weight)
-    refuse_negative(flags)
+    refuse_negative(check)
     return out
 
 
@@ -66,9 +66,9 @@ def aggregate(data: Tensor, segment: Tensor, bin_count: Tensor | None = None, av
         if bin_count is not None:
             num_segment = max(num_segment, int(bin_count.shape[0]))
     num_segment = int(num_segment)
-    (csr,), flags = csr_from_segments([(segment, num_segment)])
+    (csr,), check = csr_from_segments([(segment, num_segment)])
     out = csr_segment_sum(data, segment, num_segment, perm=csr.perm, off=csr.off)
-    refuse_negative(flags)
+    refuse_negative(check)
     if not average:
         return out
     if bin_count is None:

@@ -98,18 +98,18 @@ def fourier_basis_vjp(gout: Tensor, unit_vec: Tensor, target_index: Tensor, sour
     src = _index(source_index, rows, "source_index")
     f = _freqs(freqs, device)
     n_vec = int(u.shape[0])
-    grad = torch.zeros((n_vec, 3), dtype=torch.float32, device=device)
     if rows == 0 or n_vec == 0:
-        return grad
+        return torch.zeros((n_vec, 3), dtype=torch.float32, device=device)
+    grad = torch.empty((n_vec, 3), dtype=torch.float32, device=device)
     g = gout.to(torch.float32).contiguous()
     if g.shape != (rows, 1 + 2 * f.numel()):
         raise ValueError(f"gout must be [{rows}, {1 + 2 * f.numel()}], got {tuple(g.shape)}")
     contrib = torch.empty((rows, 6), dtype=torch.float32, device=device)
     _abi.call("fmd_threebody_fourier_bwd_rows_f32", g.data_ptr(), u.data_ptr(), ld, tgt.data_ptr(), src.data_ptr(),
               rows, f.data_ptr(), f.numel(), float(scale), contrib.data_ptr(), stream())
-    (by_target, by_source), flags = csr_from_segments([(tgt, n_vec), (src, n_vec)])
+    (by_target, by_source), check = csr_from_segments([(tgt, n_vec), (src, n_vec)])
     segment_sum_csr([(contrib, by_target, 0, 1.0, None), (contrib, by_source, 3, 1.0, None)], n_vec, 3, out=grad)
-    refuse_negative(flags)
+    refuse_negative(check)
     return grad
 
 

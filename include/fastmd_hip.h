@@ -363,7 +363,9 @@ int fmd_segsum_csr_t_f32(const float* gout, int64_t ld_gout, const float* value,
 /* The CSR of one or two segment indices (int32, or int64 where is64; element stride `stride`):
  * perm[q] [rows] = the rows in stable order of their segment, off[q] [num_segment + 1] = the run
  * of every segment. Rows with an index outside [0, num_segment) follow every run and belong to
- * none; negative[q] [1] = whether some index was negative (the caller refuses the call then).
+ * none. negative[q] (host memory that the device can write, cleared by the caller) is set to 1
+ * if some index is negative; `checked` (may be null) is recorded on the stream once every index
+ * has been read, so the caller can refuse the call without waiting for the rest of it.
  * work[q]: fmd_csr_work_size(rows) uint32 of scratch (nothing in it has to be set). One launch
  * for at most 8192 rows per index, else two per 8 bits of num_segment and one for the offsets,
  * shared by both indices.
@@ -372,7 +374,7 @@ int fmd_segsum_csr_t_f32(const float* gout, int64_t ld_gout, const float* value,
 int64_t fmd_csr_work_size(int64_t rows);
 int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* is64, const int64_t* stride,
                        const int64_t* rows, const int64_t* num_segment, int32_t* const* perm, int64_t* const* off,
-                       uint32_t* const* work, int32_t* negative, hipStream_t stream);
+                       uint32_t* const* work, int32_t* negative, hipEvent_t checked, hipStream_t stream);
 
 /* ----------------------------------------------------------------------------------------
  * (d) Edge GEMM on MFMA

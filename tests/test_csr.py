@@ -44,8 +44,8 @@ def test_two_indices_share_the_launches(rows):
     sizes = (300, 70000)
     index = [rng.integers(0, n, r) for r, n in zip(rows, sizes)]
     pairs = [(torch.tensor(i, dtype=torch.int32, device="cuda"), n) for i, n in zip(index, sizes)]
-    csrs, flags = csr_from_segments(pairs)
-    refuse_negative(flags)
+    csrs, check = csr_from_segments(pairs)
+    refuse_negative(check)
     for csr, i, n in zip(csrs, index, sizes):
         perm, off = stable_csr(i, n)
         assert csr.off.cpu().numpy().tolist() == off.tolist() and csr.perm.cpu().numpy().tolist() == perm.tolist()
