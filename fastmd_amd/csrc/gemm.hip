@@ -651,31 +651,32 @@ constexpr int X3_PL = 128 * 16, X3_OP = 3 * X3_PL, X3_BUF = 2 * X3_OP;
   } while (0)
 
 // six products per block, the small ones first: (0,2) (1,1) (2,0) (0,1) (1,0) (0,0)
-#define X3_COMPUTE(BUFI, MBV)                                                                       \
+#define X3_COMPUTE(BUFI, MBV) X3_COMPUTE_N(BUFI, MBV, 2)
+#define X3_COMPUTE_N(BUFI, MBV, NBV)                                                                \
   do {                                                                                              \
     const __bf16* as_ = lds + (BUFI) * X3_BUF;                                                      \
     const __bf16* bs_ = as_ + X3_OP;                                                                \
-    bf16x8 av_[3][2], bv_[3][2];                                                                    \
+    bf16x8 av_[3][MBV], bv_[3][NBV];                                                                    \
     _Pragma("unroll") for (int p = 0; p < 3; ++p) {                                                 \
       _Pragma("unroll") for (int i = 0; i < (MBV); ++i)                                             \
         av_[p][i] = *reinterpret_cast<const bf16x8*>(as_ + p * X3_PL + (wm * 32 * (MBV) + i * 32) * 16 + rd); \
-      _Pragma("unroll") for (int j = 0; j < 2; ++j)                                                 \
-        bv_[p][j] = *reinterpret_cast<const bf16x8*>(bs_ + p * X3_PL + (wn * 64 + j * 32) * 16 + rd); \
+      _Pragma("unroll") for (int j = 0; j < (NBV); ++j)                                                 \
+        bv_[p][j] = *reinterpret_cast<const bf16x8*>(bs_ + p * X3_PL + (wn * 32 * (NBV) + j * 32) * 16 + rd); \
     }                                                                                               \
     /* product-major: consecutive MFMAs go to the four accumulators in turn (four independent   \
        chains in flight); each accumulator still takes its six products in the same order */     \
     _Pragma("unroll") for (int pr = 0; pr < 6; ++pr) {                                              \
       const int pa_ = pr == 0 ? 0 : pr == 1 ? 1 : pr == 2 ? 2 : pr == 3 ? 0 : pr == 4 ? 1 : 0;      \
       const int pb_ = pr == 0 ? 2 : pr == 1 ? 1 : pr == 2 ? 0 : pr == 3 ? 1 : pr == 4 ? 0 : 0;      \
-      _Pragma("unroll") for (int i = 0; i < (MBV); ++i) _Pragma("unroll") for (int j = 0; j < 2; ++j) \
+      _Pragma("unroll") for (int i = 0; i < (MBV); ++i) _Pragma("unroll") for (int j = 0; j < (NBV); ++j) \
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av_[pa_][i], bv_[pb_][j], acc[i][j], 0, 0, 0); \
     }                                                                                               \
   } while (0)
 
 // The end of a split-plane tile: C (+)= acc (+ radd[radd.idx[r]]) (+ bias), then the activation;
 // interior wave tiles without bias / accumulate / activation store straight from the accumulators.
-template <int MB>
-__device__ __forceinline__ void x3_finish(f32x16 (&acc)[MB][2], const X3Part& radd, const float* __restrict__ bias,
+template <int MB, int NB = 2>
+__device__ __forceinline__ void x3_finish(f32x16 (&acc)[MB][NB], const X3Part& radd, const float* __restrict__ bias,
                                           float* c, int64_t ldc, int64_t m, int64_t n, int accumulate, int act,
                                           int64_t row0, int64_t col0, int h, int rr) {
   if (radd.src) {
@@ -687,31 +688,31 @@ __device__ __forceinline__ void x3_finish(f32x16 (&acc)[MB][2], const X3Part& ra
         const int64_t row = min(row0 + bi * 32 + (v / 4) * 8 + h * 4 + (v % 4), m - 1);
         const float* qr = radd.src + (radd.idx ? (int64_t)radd.idx[row * radd.istride] : row) * radd.ld;
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj) {
+        for (int bj = 0; bj < NB; ++bj) {
           const int64_t col = min(col0 + bj * 32 + rr, n - 1);
           acc[bi][bj][v] += qr[col];
         }
       }
   }
-  if (!bias && act == 0 && row0 + 32 * MB <= m && col0 + 64 <= n) {
+  if (!bias && act == 0 && row0 + 32 * MB <= m && col0 + 32 * NB <= n) {
     float* base = c + (row0 + h * 4) * ldc + col0 + rr;
     if (accumulate) {
       // every old value loaded before any store: one memory round trip, not one per row (the
       // stores could alias the loads, so the compiler keeps a load-add-store chain in order)
 #pragma unroll
       for (int bi = 0; bi < MB; ++bi) {
-        float old[16][2];
+        float old[16][NB];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const float* rp = base + (int64_t)(bi * 32 + (v / 4) * 8 + (v % 4)) * ldc;
-          old[v][0] = rp[0];
-          old[v][1] = rp[32];
+#pragma unroll
+          for (int bj = 0; bj < NB; ++bj) old[v][bj] = rp[32 * bj];
         }
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           float* rp = base + (int64_t)(bi * 32 + (v / 4) * 8 + (v % 4)) * ldc;
-          rp[0] = old[v][0] + acc[bi][0][v];
-          rp[32] = old[v][1] + acc[bi][1][v];
+#pragma unroll
+          for (int bj = 0; bj < NB; ++bj) rp[32 * bj] = old[v][bj] + acc[bi][bj][v];
         }
       }
       return;
@@ -721,12 +722,12 @@ __device__ __forceinline__ void x3_finish(f32x16 (&acc)[MB][2], const X3Part& ra
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         float* rp = base + (int64_t)(bi * 32 + (v / 4) * 8 + (v % 4)) * ldc;
-        store_stream(rp, acc[bi][0][v]);
-        store_stream(rp + 32, acc[bi][1][v]);
+#pragma unroll
+        for (int bj = 0; bj < NB; ++bj) store_stream(rp + 32 * bj, acc[bi][bj][v]);
       }
     return;
   }
-  epilogue<MB, 2>(acc, row0, col0, m, n, bias, c, ldc, accumulate, act);
+  epilogue<MB, NB>(acc, row0, col0, m, n, bias, c, ldc, accumulate, act);
 }
 
 // One 128 x BN tile of C at (row_blk, col_blk): A as up to three gathered column parts (K order
@@ -830,42 +831,105 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     const float* base_ = q2_ ? fa2 : q1_ ? fa1 : fa0;                                               \
     const int64_t kin_ = q2_ ? k0_ - ks2 : q1_ ? k0_ - ks1 : k0_;                                   \
     const int w_ = q2_ ? w2 : q1_ ? w1 : w0;                                                        \
-    _Pragma("unroll") for (int q = 0; q < MB; ++q) {                                                \
+    _Pragma("unroll") for (int q = 0; q < AQ; ++q) {                                                \
       const int64_t o_ = q2_ ? ao2[q] : q1_ ? ao1[q] : ao0[q];                                      \
       ra##S[q] = (kin_ + kc < w_) ? *reinterpret_cast<const float4*>(base_ + o_ + kin_)             \
                                   : make_float4(0.f, 0.f, 0.f, 0.f);                                \
     }                                                                                               \
-    _Pragma("unroll") for (int j = 0; j < 3; ++j)                                                   \
-      pb##S[j] = *reinterpret_cast<const u32x4*>(bp + bo[j] + k0_ * 3);                            \
+    if (BN == 128 || t < 2 * BN)                                                                    \
+      _Pragma("unroll") for (int j = 0; j < 3; ++j)                                                 \
+        pb##S[j] = *reinterpret_cast<const u32x4*>(bp + bo[j] + k0_ * 3);                            \
   } while (0)
 
 #define XP_STORE(BUFI, S)                                                                           \
   do {                                                                                              \
     __bf16* sb_ = lds + (BUFI) * X3_BUF;                                                            \
-    _Pragma("unroll") for (int q = 0; q < MB; ++q) {                                                \
+    _Pragma("unroll") for (int q = 0; q < AQ; ++q) {                                                \
       bf16x4 x0_, x1_, x2_;                                                                         \
       split3(ra##S[q], x0_, x1_, x2_);                                                              \
       *reinterpret_cast<bf16x4*>(sb_ + 0 * X3_PL + soff[q]) = x0_;                                  \
       *reinterpret_cast<bf16x4*>(sb_ + 1 * X3_PL + soff[q]) = x1_;                                  \
       *reinterpret_cast<bf16x4*>(sb_ + 2 * X3_PL + soff[q]) = x2_;                                  \
     }                                                                                               \
-    _Pragma("unroll") for (int j = 0; j < 3; ++j)                                                   \
-      *reinterpret_cast<u32x4*>(sb_ + X3_OP + (t + j * kThreads) * 8) = pb##S[j];                  \
+    if (BN == 128 || t < 2 * BN)                                                                    \
+      _Pragma("unroll") for (int j = 0; j < 3; ++j)                                                 \
+        *reinterpret_cast<u32x4*>(sb_ + X3_OP + (t + j * kThreads) * 8) = pb##S[j];                  \
   } while (0)
 
-// One (64 MB) x 128 tile with fp32 A (MB as in x3_tile) and B's planes. Two register stages
+// Elements of a finished tile that are NaN, formed again as an fp32 FMA chain over the unsplit A and
+// B's planes added up: a plane product cannot carry an infinity (inf - inf in the split, inf * 0
+// between planes), so an operand that is infinite, or rounds to an infinite bf16, shows as a NaN
+// here and gets the value of an fp32 product; a sum that is NaN ends its chain. Outputs of finite
+// operands never come here.
+template <int MB, int NB>
+__device__ __forceinline__ void x3p_nonfinite(f32x16 (&acc)[MB][NB], const X3PPart& P0, const X3PPart& P1,
+                                              const X3PPart& P2, int np, const __bf16* __restrict__ bp, int64_t ldb,
+                                              int64_t m, int64_t n, int64_t k, int64_t row0, int64_t col0, int h,
+                                              int rr) {
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN if an element is NaN or infinite
+#pragma unroll
+  for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) zero[v & 3] = fmaf(acc[bi][bj][v], 0.f, zero[v & 3]);
+  const float all = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+  if (!__any(all != all)) return;
+  uint64_t mask = 0;
+#pragma unroll
+  for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (acc[bi][bj][v] != acc[bi][bj][v]) mask |= 1ull << ((bi * NB + bj) * 16 + v);
+  while (__any(mask != 0)) {
+    const int id = mask ? __ffsll((unsigned long long)mask) - 1 : -1;
+    float sum = 0.f;
+    if (id >= 0) {
+      const int v = id & 15, bj = (id >> 4) % NB, bi = (id >> 4) / NB;
+      const int64_t row = min(row0 + bi * 32 + (v / 4) * 8 + h * 4 + (v % 4), m - 1);
+      const int64_t col = min(col0 + bj * 32 + rr, n - 1);
+      const __bf16* b = bp + col * ldb;
+      int64_t kk = 0;
+      for (int p = 0; p < np && sum == sum; ++p) {
+        const X3PPart& P = p == 0 ? P0 : p == 1 ? P1 : P2;
+        const float* a = static_cast<const float*>(P.src) + (P.idx ? (int64_t)P.idx[row * P.istride] : row) * P.ld;
+        for (int q = 0; q < P.width && kk < k && sum == sum; ++q, ++kk) {
+          const __bf16* e = b + (kk >> 4) * 48 + (kk & 15);
+          sum = fmaf(a[q], (float)e[0] + ((float)e[16] + (float)e[32]), sum);
+        }
+      }
+    }
+#pragma unroll
+    for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[bi][bj][v] = (bi * NB + bj) * 16 + v == id ? sum : acc[bi][bj][v];
+    mask &= mask - 1;
+  }
+}
+
+// One (32 MB WM) x BN tile with fp32 A and B's planes, in `lds` (2 X3_BUF elements). BN = 128: waves
+// 2 x 2 (WM = 2), each 32 MB x 64; BN = 64 or 32: waves 4 x 1 (WM = 4, MB = 1), each 32 x BN: the last
+// column tile of an N that is not a multiple of 128 (K = 2F + 8 as the output width of an input
+// gradient leaves 8 columns, of which a 128-wide tile would compute 120 for nothing: 160 000 rows, N = 136,
+// 264, 520 with K = 256, 512, 1 024: 125, 357, 1 132 -> 110, 315, 1 060 us; a narrow tile still stages all of
+// A). FIX: form NaN elements again (x3p_nonfinite). Two register stages
 // (loads issued two slices ahead) measured no faster than one at two waves per SIMD instead of
 // three, so the tile keeps one stage: slice kt + 1 is stored into LDS and slice kt + 2 loaded into
 // the stage while the MFMAs of slice kt run.
-template <int MB>
-__device__ __forceinline__ void x3p_tile(const X3PPart& P0, const X3PPart& P1, const X3PPart& P2, int np,
+template <int MB, int BN, bool FIX>
+__device__ __forceinline__ void x3p_tile(__bf16* lds, const X3PPart& P0, const X3PPart& P1, const X3PPart& P2, int np,
                                          const __bf16* __restrict__ bp, int64_t ldb, const X3Part& radd,
                                          const float* __restrict__ bias, float* c, int64_t ldc, int64_t m, int64_t n,
                                          int64_t k, int accumulate, int act, int64_t row_blk, int64_t col_blk) {
-  __shared__ __attribute__((aligned(16))) __bf16 lds[2 * X3_BUF];
+  constexpr int WM = BN == 128 ? 2 : 4, NB = BN == 128 ? 2 : BN / 32, AQ = MB * WM / 2;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = wave >> 1, wn = wave & 1, h = lane >> 5, rr = lane & 31;
+  const int wm = BN == 128 ? wave >> 1 : wave, wn = BN == 128 ? wave & 1 : 0, h = lane >> 5, rr = lane & 31;
   const int64_t ks1 = P0.width, ks2 = ks1 + (np > 1 ? P1.width : 0);
   const int w0 = P0.width, w1 = P1.width, w2 = P2.width;
   const float *fa0 = static_cast<const float*>(P0.src), *fa1 = static_cast<const float*>(P1.src),
@@ -879,10 +943,10 @@ __device__ __forceinline__ void x3p_tile(const X3PPart& P0, const X3PPart& P1, c
   }
   // fp32 A: row (t + 256 q) / 4, k (t % 4) * 4
   const int kc = (t & 3) * 4;
-  int64_t ao0[2], ao1[2], ao2[2];
-  int soff[2];
+  int64_t ao0[AQ], ao1[AQ], ao2[AQ];
+  int soff[AQ];
 #pragma unroll
-  for (int q = 0; q < MB; ++q) {
+  for (int q = 0; q < AQ; ++q) {
     const int r = (t + q * kThreads) >> 2;
     const int64_t gr = min(row_blk + r, m - 1);
     ao0[q] = (P0.idx ? (int64_t)P0.idx[gr * P0.istride] : gr) * P0.ld + kc;
@@ -892,12 +956,12 @@ __device__ __forceinline__ void x3p_tile(const X3PPart& P0, const X3PPart& P1, c
   }
   const int rd = rr * 16 + ((h ^ ((rr >> 3) & 1)) * 8);  // this lane's 8 k of its MFMA row
   u32x4 pb0[3];
-  float4 ra0[MB];
-  f32x16 acc[MB][2];
+  float4 ra0[AQ];
+  f32x16 acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
@@ -912,11 +976,12 @@ __device__ __forceinline__ void x3p_tile(const X3PPart& P0, const X3PPart& P1, c
       XP_STORE(cur ^ 1, 0);                       // slice kt + 1 (loaded one iteration ago)
       if (kt + 2 < nk) XP_LOAD((kt + 2) * 16, 0);  // slice kt + 2 stays in flight over these MFMAs
     }
-    X3_COMPUTE(cur, MB);
+    X3_COMPUTE_N(cur, MB, NB);
     __syncthreads();  // buffer cur is free, buffer cur ^ 1 is complete
   }
-  const int64_t row0 = row_blk + wm * 32 * MB, col0 = col_blk + wn * 64;
-  x3_finish<MB>(acc, radd, bias, c, ldc, m, n, accumulate, act, row0, col0, h, rr);
+  const int64_t row0 = row_blk + wm * 32 * MB, col0 = col_blk + wn * 32 * NB;
+  if constexpr (FIX) x3p_nonfinite<MB, NB>(acc, P0, P1, P2, np, bp, ldb, m, n, k, row0, col0, h, rr);
+  x3_finish<MB, NB>(acc, radd, bias, c, ldc, m, n, accumulate, act, row0, col0, h, rr);
 }
 
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) gemm_x3p_kernel(
@@ -924,8 +989,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     const float* __restrict__ bias, float* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int accumulate, int act,
     int64_t n_tiles) {
   const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  x3p_tile<2>(P0, P1, P2, np, bp, ldb, radd, bias, c, ldc, m, n, k, accumulate, act, (tile / n_tiles) * 128,
-                    (tile % n_tiles) * 128);
+  __shared__ __attribute__((aligned(16))) __bf16 lds[2 * X3_BUF];
+  const int64_t row = (tile / n_tiles) * 128, col = (tile % n_tiles) * 128;
+  if (n - col > 64)
+    x3p_tile<2, 128, true>(lds, P0, P1, P2, np, bp, ldb, radd, bias, c, ldc, m, n, k, accumulate, act, row, col);
+  else if (n - col > 32)
+    x3p_tile<1, 64, true>(lds, P0, P1, P2, np, bp, ldb, radd, bias, c, ldc, m, n, k, accumulate, act, row, col);
+  else
+    x3p_tile<1, 32, true>(lds, P0, P1, P2, np, bp, ldb, radd, bias, c, ldc, m, n, k, accumulate, act, row, col);
 }
 
 // The product with both operands as planes, copied straight into LDS by the memory system
@@ -1280,12 +1351,30 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3
     if (q < grp.count && w >= grp.d[q].tile0) g = q;
   const X3PGroupDesc& d = grp.d[g];
   const int64_t t = w - d.tile0;
-  x3p_tile<MB>(d.p0, d.p1, d.p1, d.np, d.b, d.ldb, d.radd, d.bias, d.c, d.ldc, d.m, d.n, d.k, d.accumulate,
+  __shared__ __attribute__((aligned(16))) __bf16 lds[2 * X3_BUF];
+  x3p_tile<MB, 128, false>(lds, d.p0, d.p1, d.p1, d.np, d.b, d.ldb, d.radd, d.bias, d.c, d.ldc, d.m, d.n, d.k, d.accumulate,
                grp.act, (t / d.n_tiles) * (64 * MB), (t % d.n_tiles) * 128);
 }
 
 #undef XP_LOAD
 #undef XP_STORE
+
+// split3 of a value stored as planes: an infinity or a NaN is its first plane alone, and a finite
+// value that rounds to an infinite bf16 takes the largest bf16 first, so the planes always add up to
+// the value (split3's own planes for every other value).
+__device__ __forceinline__ void split3_stored(float4 v, bf16x4& p0, bf16x4& p1, bf16x4& p2) {
+  split3(v, p0, p1, p2);
+  const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool finite = fabsf(x[e]) <= 3.402823466e38f;
+    if (finite && fabsf((float)p0[e]) <= 3.402823466e38f) continue;
+    const float big = copysignf(3.389531390e38f, x[e]), r1 = x[e] - big;
+    p0[e] = finite ? (__bf16)big : p0[e];
+    p1[e] = finite ? (__bf16)r1 : (__bf16)0.f;
+    p2[e] = finite ? (__bf16)(r1 - (float)p1[e]) : (__bf16)0.f;
+  }
+}
 
 // planes[r][s][p][0, 16) = the bf16 planes of src[r][16 s, 16 s + 16) (split3), zero past the
 // width (the slice-interleaved operand format of gemm_x3p_kernel); one thread per 8 elements
@@ -1301,9 +1390,32 @@ __global__ void split3_kernel(const float* __restrict__ src, int64_t ld, int64_t
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = k0 + e < width ? s[e] : 0.f;
   bf16x4 p[3][2];
-  split3(make_float4(x[0], x[1], x[2], x[3]), p[0][0], p[1][0], p[2][0]);
-  split3(make_float4(x[4], x[5], x[6], x[7]), p[0][1], p[1][1], p[2][1]);
+  split3_stored(make_float4(x[0], x[1], x[2], x[3]), p[0][0], p[1][0], p[2][0]);
+  split3_stored(make_float4(x[4], x[5], x[6], x[7]), p[0][1], p[1][1], p[2][1]);
   __bf16* d = planes + r * slices * 48 + (c >> 1) * 48 + (c & 1) * 8;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    *reinterpret_cast<bf16x4*>(d + q * 16) = p[q][0];
+    *reinterpret_cast<bf16x4*>(d + q * 16 + 4) = p[q][1];
+  }
+}
+
+// The planes of src^T, src [rows, cols] (a [K, N] weight as the N x K operand of the kernels above):
+// planes[c][s][p][0, 16) from src[16 s .. 16 s + 16)[c], zero past the rows. One thread per column
+// and 8 rows, consecutive threads on consecutive columns (coalesced reads; the writes of a weight,
+// some MB, stay in L2).
+__global__ void split3_t_kernel(const float* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, __bf16* planes,
+                                int64_t slices) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= cols) return;
+  const int64_t half = blockIdx.y, k0 = half * 8;
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = k0 + e < rows ? src[(k0 + e) * ld + c] : 0.f;
+  bf16x4 p[3][2];
+  split3_stored(make_float4(x[0], x[1], x[2], x[3]), p[0][0], p[1][0], p[2][0]);
+  split3_stored(make_float4(x[4], x[5], x[6], x[7]), p[0][1], p[1][1], p[2][1]);
+  __bf16* d = planes + (c * slices + (half >> 1)) * 48 + (half & 1) * 8;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     *reinterpret_cast<bf16x4*>(d + q * 16) = p[q][0];
@@ -1314,6 +1426,7 @@ __global__ void split3_kernel(const float* __restrict__ src, int64_t ld, int64_t
 #undef X3_LOAD
 #undef X3_STORE
 #undef X3_COMPUTE
+#undef X3_COMPUTE_N
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -1434,6 +1547,17 @@ int fmd_split3_f32(const float* src, int64_t ld, int64_t rows, int32_t width, ui
   const int64_t slices = fmd_cdiv(width, 16), threads = rows * slices * 2;
   hipLaunchKernelGGL(split3_kernel, dim3((unsigned)fmd_cdiv(threads, 256)), dim3(256), 0, stream, src, ld, rows, width,
                      reinterpret_cast<__bf16*>(planes), slices);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_split3_t_f32(const float* src, int64_t ld, int64_t rows, int64_t cols, uint16_t* planes, hipStream_t stream) {
+  FMD_REQUIRE(rows >= 0 && cols >= 0 && ld >= cols);
+  if (rows == 0 || cols == 0) return FMD_OK;
+  const int64_t slices = fmd_cdiv(rows, 16);
+  FMD_REQUIRE(src && planes && aligned16(planes) && 2 * slices < 65536);
+  hipLaunchKernelGGL(split3_t_kernel, dim3((unsigned)fmd_cdiv(cols, 64), (unsigned)(2 * slices)), dim3(64), 0, stream,
+                     src, ld, rows, cols, reinterpret_cast<__bf16*>(planes), slices);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

@@ -7,7 +7,8 @@ Reference signatures (fastmd/engine/kernels/triton_wide_gemm.py:482-553):
 The reference's 3xTF32 kernels decline K % 16 != 0 (:235), i.e. the configs' K = 2F + 8, and fall
 back to cuBLAS SGEMM. Here large K-contiguous ("NT") GEMMs run fp32-accurate on the bf16 matrix
 cores (each operand split into three bf16 planes, six MFMA products: CDNA4's counterpart of
-3xTF32), the rest on fp32 MFMA (v_mfma_f32_32x32x2_f32); ``edge_gemm(a, w, dtype=torch.bfloat16)``
+3xTF32), and so do large ``[K, N]`` ones with the weight's planes formed transposed; the rest on fp32
+MFMA (v_mfma_f32_32x32x2_f32); ``edge_gemm(a, w, dtype=torch.bfloat16)``
 runs plain bf16 operands (v_mfma_f32_32x32x16_bf16, fp32 out). ``gemm_gather`` fuses the edge-row
 gather-cat into the GEMM's operand load. ``epilogue="silu"`` fuses SiLU into the store.
 """
@@ -21,6 +22,24 @@ from fastmd_amd import _abi
 from fastmd_amd._device import require_cuda, rows_view, stream
 
 _EPILOGUES = {None: 0, "none": 0, "silu": 1}
+
+
+# A float32 gemm splits its B into the bf16 planes beforehand (one launch, about 11 us) and runs on the
+# split-plane kernel with fp32 A:
+# * b [K, N]: from 256 tiles of 128 x 128, as the b [N, K] kernel that splits both operands (the fp32
+#   MFMA form takes 2 217 us at [160 000, 1 024] x [1 024, 520], this one 1 060, 153 against 100 us with
+#   10 000 rows; with 125 tiles, [16 000, 384] x [384, 128], 29 against 37);
+# * b [N, K]: from PLANES_MIN_WORK multiply-adds, where splitting B once instead of once per row tile
+#   saves more than the launch (1 110 against 985 us at [160 000, 520] x [520, 1 024], 265 against 260 with
+#   40 000 rows, 94 against 100 with 10 000).
+PLANES_MIN_TILES = 256
+PLANES_MIN_WORK = 2 ** 34
+
+
+def _takes_planes(m: int, n: int, k: int, b_layout: int) -> bool:
+    if k % 4 or k <= 16 or n <= 16 or k > 65536 or -(-m // 128) * -(-n // 128) < PLANES_MIN_TILES:
+        return False
+    return b_layout == 1 or m * n * k >= PLANES_MIN_WORK
 
 
 def gemm(a: Tensor, b: Tensor, *, b_layout: int, bias: Tensor | None = None, out: Tensor | None = None,
@@ -52,6 +71,9 @@ def gemm(a: Tensor, b: Tensor, *, b_layout: int, bias: Tensor | None = None, out
     b, ldb = rows_view(b)
     if m == 0 or n == 0:
         return out
+    if name == "fmd_gemm_f32" and _takes_planes(m, n, k, b_layout) and lda % 4 == 0 and a.data_ptr() % 16 == 0:
+        return gemm_planes([(a, None)], split_planes(b, transpose=b_layout == 1), a_planes=False, out=out, bias=bias,
+                           accumulate=accumulate, epilogue=epilogue)
     _abi.call(name, a.data_ptr(), lda, b.data_ptr(), ldb, b_layout, _abi.ptr(bias), out.data_ptr(),
               out.stride(0) if m > 1 else n, m, n, k, 1 if accumulate else 0, _EPILOGUES[epilogue], stream())
     return out
@@ -280,19 +302,21 @@ class Planes:
         return self.data.permute(0, 2, 1, 3).reshape(rows, 3, slices * 16)
 
 
-def split_planes(x: Tensor, *, out: Planes | None = None) -> Planes:
-    """The bf16 planes of a 2-D float32 ``x`` (fmd_split3_f32)."""
+def split_planes(x: Tensor, *, out: Planes | None = None, transpose: bool = False) -> Planes:
+    """The bf16 planes of a 2-D float32 ``x`` (fmd_split3_f32), or of its transpose (fmd_split3_t_f32)."""
     require_cuda(x)
     if x.dim() != 2 or x.dtype != torch.float32:
         raise ValueError("split_planes takes a 2-D float32 tensor")
     x, ld = rows_view(x)
-    rows, width = x.shape
+    rows, width = reversed(x.shape) if transpose else x.shape
     slices = -(-width // 16)
     if out is None:
         out = Planes(torch.empty((rows, slices, 3, 16), dtype=torch.bfloat16, device=x.device), width)
     elif out.data.shape != (rows, slices, 3, 16) or out.width != width:
         raise ValueError("split_planes: out does not match")
-    if rows:
+    if transpose:
+        _abi.call("fmd_split3_t_f32", x.data_ptr(), ld, width, rows, out.data.data_ptr(), stream())
+    elif rows:
         _abi.call("fmd_split3_f32", x.data_ptr(), ld, rows, width, out.data.data_ptr(), stream())
     return out
 

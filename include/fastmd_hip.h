@@ -496,6 +496,9 @@ int fmd_gemm_gather_f32(int32_t n_parts, const float* const* srcs, const int32_t
  * once-per-weight-version operand split (_split_kernel / _split, triton_wide_gemm.py:12-15,
  * 131-199: hi/lo TF32 pairs there, three bf16 planes here). */
 int fmd_split3_f32(const float* src, int64_t ld, int64_t rows, int32_t width, uint16_t* planes, hipStream_t stream);
+/* The same planes of src^T for a weight stored [rows = K, cols = N] (row stride ld): planes
+ * [cols, ceil(rows / 16), 3, 16], zero past the rows. rows at most 524 280. */
+int fmd_split3_t_f32(const float* src, int64_t ld, int64_t rows, int64_t cols, uint16_t* planes, hipStream_t stream);
 /* fmd_gemm_gather_f32 with pre-split operands: B [N, K] as planes (fmd_split3_f32, ldb =
  * 48 ceil(K / 16)), and with a_planes the parts as planes too (srcs_p planes of width widths_p,
  * lds_p = 48 ceil(widths_p / 16); widths multiples of 8, all but the last of 16); a_planes 0: the

@@ -1,0 +1,74 @@
+"""float32 gemm whose B is split into bf16 planes by the call itself (b [K, N], and large b [N, K]):
+every width of the last column tile against float64, and non-finite operands."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(a, b, b_layout):
+    return a.double() @ (b.double().t() if b_layout == 0 else b.double())
+
+
+# last column tiles of 8, 32, 33, 64, 65 and 128 columns; K of one partial slice, of an odd number of 16-k slices
+# and of exact ones; the smallest row counts of the route
+@pytest.mark.parametrize("m,n,k", [(32641, 40, 20), (16257, 136, 264), (10900, 288, 36), (10900, 289, 48),
+                                   (8129, 448, 64), (8129, 449, 100), (6600, 520, 1024), (32700, 128, 260)])
+@pytest.mark.parametrize("form", ["plain", "bias_silu", "accumulate"])
+def test_b_layout_1(m, n, k, form):
+    from fastmd_amd.ops import wide_gemm
+
+    assert wide_gemm._takes_planes(m, n, k, 1)
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k + 4, generator=gen, device="cuda")[:, :k]  # a row stride of its own
+    b = torch.randn(k, n + 3, generator=gen, device="cuda")[:, :n]
+    want = reference(a, b, 1)
+    if form == "bias_silu":
+        bias = torch.randn(n, generator=gen, device="cuda")
+        got = wide_gemm.gemm(a, b, b_layout=1, bias=bias, epilogue="silu")
+        want = torch.nn.functional.silu(want + bias.double())
+    elif form == "accumulate":
+        out = torch.randn(m, n, generator=gen, device="cuda")
+        want = want + out.double()
+        got = wide_gemm.gemm(a, b, b_layout=1, out=out, accumulate=True)
+    else:
+        got = wide_gemm.gemm(a, b, b_layout=1)
+    # three planes per operand: 2^-24 per product, K products summed in fp32; 1e-5 of the largest element as
+    # for every float32 gemm here
+    assert float((got.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
+def test_large_b_layout_0_equals_the_kernel_that_splits_both():
+    """The same planes and K order: bitwise gemm_gather, which splits B in the kernel."""
+    from fastmd_amd.ops import wide_gemm
+
+    m, n, k = 160000, 392, 280  # a last column tile of 8
+    assert wide_gemm._takes_planes(m, n, k, 0)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a, b = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(n, k, generator=gen, device="cuda")
+    assert torch.equal(wide_gemm.gemm(a, b, b_layout=0), wide_gemm.gemm_gather([(a, None)], b))
+
+
+@pytest.mark.parametrize("n", [128, 136])
+def test_non_finite_operands_follow_the_fp32_product(n):
+    """Infinities, NaN and values that round to an infinite bf16 give what float64 gives (an infinity
+    kept, inf - inf and inf * 0 NaN), and leave the other rows and columns alone."""
+    from fastmd_amd.ops import wide_gemm
+
+    m, k = 32700, 64
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    a, b = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(k, n, generator=gen, device="cuda")
+    b[:, 3] = b[:, 3].to(torch.bfloat16).float()  # its lower planes are zero
+    a[:, 5] *= 1e-3  # the products of the large finite values stay finite
+    b[2] *= 1e-3
+    a[5, 7], a[6, 7], a[6, 9], a[7, 1], a[8, 2] = float("inf"), float("inf"), float("-inf"), float("nan"), 3.4e38
+    b[4, n - 1], b[5, n - 2] = float("inf"), 3.4e38
+    a[9, 4] = 0.0  # times that infinity
+    want = reference(a, b, 1)
+    got = wide_gemm.gemm(a, b, b_layout=1).double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    fine = torch.isfinite(want) & (want.abs() < 1e30)
+    assert float((got - want)[fine].abs().max()) <= 1e-5 * float(want[fine].abs().max())
+    big = torch.isfinite(want) & ~fine
+    assert float(((got - want)[big] / want[big]).abs().max()) <= 1e-5
