@@ -20,6 +20,8 @@ _i32 = ctypes.c_int32
 _i64 = ctypes.c_int64
 _f32 = ctypes.c_float
 _u8 = ctypes.c_uint8
+# FMD_NL_PAD_* of the candidate search
+NL_PAD_ALL, NL_PAD_STALE, NL_PAD_NONE = 0, 1, 2
 
 # name -> (restype, argtypes); mirrors include/fastmd_hip.h
 SIGNATURES: dict[str, tuple] = {
@@ -27,6 +29,9 @@ SIGNATURES: dict[str, tuple] = {
     "fmd_error_string": (ctypes.c_char_p, [ctypes.c_int]),
     "fmd_nl_candidates": (ctypes.c_int, [_p, _p, _p, _i64, _f32, _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64,
                                          _i64, _p]),
+    "fmd_nl_candidates_pad": (ctypes.c_int, [_p, _p, _p, _i64, _f32, _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64,
+                                             _i64, _i32, _p]),
+    "fmd_nl_atom_order": (ctypes.c_int, [_p, _i64, _p, _p, _p]),
     "fmd_nl_wrap": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "fmd_nl_build_work_size": (_i64, [_i64]),
     "fmd_nl_build": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _p, _p, _p, _i32, _p, _p, _p, _f32, _f32, _i32,

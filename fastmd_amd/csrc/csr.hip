@@ -11,6 +11,8 @@
 //   * above: per pass a histogram launch and a scatter launch over at most 256 contiguous chunks
 //     (each scatter workgroup sums the chunk histograms itself, so there is no scan launch), then
 //     one search per segment over the sorted keys. Up to two indices share the launches.
+// The same passes order the atoms along a Morton curve for the builders (fmd_nl_atom_order: 30-bit
+// keys formed from the fractional coordinates in the first pass; four passes).
 // Bound by launches and dependent loads, not by bytes (160 000 rows: 8 MB in all): the two CSRs of a
 // gather-cat VJP at 160 000 rows, 10 000 segments are 5 launches (45 us) where torch's sort, bincount
 // and cumsum were 44 (275 us). Measured whole: that forward and VJP at F = 128 453 -> 222 us, the Fourier
@@ -40,6 +42,7 @@ struct Job {
   int32_t nseg;
   int32_t* perm;
   int64_t* off;
+  const float* frac;   // Morton keys of [rows, 3] fractional coordinates instead of an index (null: none)
   int32_t* negative;   // set to 1 if some index is negative (host memory the device can write)
   uint32_t* key[2];    // [rows] each
   int32_t* row[2];     // [rows] each
@@ -54,9 +57,28 @@ struct Jobs {
   Job j[2];
 };
 
+// 10 bits of v at every third position
+__device__ __forceinline__ uint32_t spread3(uint32_t v) {
+  v = (v | (v << 16)) & 0x030000FFu;
+  v = (v | (v << 8)) & 0x0300F00Fu;
+  v = (v | (v << 4)) & 0x030C30C3u;
+  return (v | (v << 2)) & 0x09249249u;
+}
+
+__device__ __forceinline__ uint32_t morton_key(const float* f) {
+  uint32_t code = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float x = fminf(fmaxf(f[a], 0.f), 0.99999988f) * 1024.f;  // the largest float below 1
+    code |= spread3((uint32_t)x & 1023u) << a;
+  }
+  return code;
+}
+
 // key of a row: its segment, or num_segment for an index outside [0, num_segment) (such rows follow
 // every run and belong to none)
 __device__ __forceinline__ uint32_t row_key(const Job& j, int64_t r, bool& neg) {
+  if (j.frac) return morton_key(j.frac + 3 * r);
   const int64_t v = j.is64 ? static_cast<const int64_t*>(j.index)[r * j.stride]
                            : (int64_t)static_cast<const int32_t*>(j.index)[r * j.stride];
   neg = neg || v < 0;
@@ -263,7 +285,24 @@ __global__ void __launch_bounds__(kSmallThreads) csr_small_kernel(const Jobs job
   }
   const int fin = j.passes & 1;
   for (int r = t; r < rows; r += kSmallThreads) j.perm[r] = s_row[fin][r];
-  for (int64_t s = t; s <= j.nseg; s += kSmallThreads) j.off[s] = lower_bound(s_key[fin], rows, (uint32_t)s);
+  if (j.off)
+    for (int64_t s = t; s <= j.nseg; s += kSmallThreads) j.off[s] = lower_bound(s_key[fin], rows, (uint32_t)s);
+}
+
+// The chunks of a job above kSmallRows and its buffers in `work`.
+void job_chunks(Job& j, uint32_t* work) {
+  const int64_t n = j.rows;
+  int64_t c = fmd_cdiv(n, kChunkRows);
+  c = c < 1 ? 1 : (c > kMaxChunks ? kMaxChunks : c);
+  const int64_t per = fmd_cdiv(fmd_cdiv(n, c), kThreads) * kThreads;
+  j.chunk_rows = (int32_t)(per < kThreads ? kThreads : per);
+  j.chunks = (int)fmd_cdiv(n, j.chunk_rows);
+  j.chunks = j.chunks < 1 ? 1 : j.chunks;
+  j.key[0] = work;
+  j.key[1] = work + n;
+  j.row[0] = reinterpret_cast<int32_t*>(work + 2 * n);
+  j.row[1] = reinterpret_cast<int32_t*>(work + 3 * n);
+  j.hist = work + 4 * n;
 }
 
 }  // namespace
@@ -309,21 +348,9 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
     return checked ? (int)hipEventRecord(checked, stream) : FMD_OK;
   }
   for (int q = 0; q < count; ++q) {
-    Job& j = jobs.j[q];
     FMD_REQUIRE(work[q]);
-    const int64_t n = rows[q];
-    int64_t c = fmd_cdiv(n, kChunkRows);
-    c = c < 1 ? 1 : (c > kMaxChunks ? kMaxChunks : c);
-    const int64_t per = fmd_cdiv(fmd_cdiv(n, c), kThreads) * kThreads;
-    j.chunk_rows = (int32_t)(per < kThreads ? kThreads : per);
-    j.chunks = (int)fmd_cdiv(n, j.chunk_rows);
-    j.chunks = j.chunks < 1 ? 1 : j.chunks;
-    j.key[0] = work[q];
-    j.key[1] = work[q] + n;
-    j.row[0] = reinterpret_cast<int32_t*>(work[q] + 2 * n);
-    j.row[1] = reinterpret_cast<int32_t*>(work[q] + 3 * n);
-    j.hist = work[q] + 4 * n;
-    chunks = j.chunks > chunks ? j.chunks : chunks;
+    job_chunks(jobs.j[q], work[q]);
+    chunks = jobs.j[q].chunks > chunks ? jobs.j[q].chunks : chunks;
   }
   for (int p = 0; p < passes; ++p) {
     hipLaunchKernelGGL(csr_hist_kernel, dim3((unsigned)chunks, (unsigned)count), dim3(kThreads), 0, stream, jobs, p);
@@ -338,6 +365,30 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
   hipLaunchKernelGGL(csr_offsets_kernel, dim3((unsigned)fmd_cdiv(nseg + 1, kThreads), (unsigned)count), dim3(kThreads),
                      0, stream, jobs);
   FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_nl_atom_order(const float* frac, int64_t n_atoms, uint32_t* work, int32_t* order, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms > 0 && n_atoms < (int64_t(1) << 31) - 1 && frac && work && order);
+  Jobs jobs{};
+  Job& j = jobs.j[0];
+  j.frac = frac;
+  j.rows = (int32_t)n_atoms;
+  j.perm = order;
+  j.passes = 4;
+  j.bits = 8;
+  if (n_atoms <= kSmallRows) {
+    hipLaunchKernelGGL(csr_small_kernel, dim3(1, 1), dim3(kSmallThreads), 0, stream, jobs);
+    FMD_CHECK_LAUNCH();
+    return FMD_OK;
+  }
+  job_chunks(j, work);
+  for (int p = 0; p < j.passes; ++p) {
+    hipLaunchKernelGGL(csr_hist_kernel, dim3((unsigned)j.chunks, 1), dim3(kThreads), 0, stream, jobs, p);
+    FMD_CHECK_LAUNCH();
+    hipLaunchKernelGGL(csr_scatter_kernel, dim3((unsigned)j.chunks, 1), dim3(kThreads), 0, stream, jobs, p);
+    FMD_CHECK_LAUNCH();
+  }
   return FMD_OK;
 }
 

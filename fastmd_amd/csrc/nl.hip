@@ -155,27 +155,17 @@ __global__ void cells_count_kernel(const float* frac, int64_t n, int n0, int n1,
   atomicAdd(&cell_count[(c0 * n1 + c1) * n2 + c2], 1);
 }
 
-// Exclusive scan of the cell counts (one workgroup); leaves the counts zeroed as cursors.
-__global__ void cells_scan_kernel(int32_t* cell_count, int32_t* cell_start, int64_t ncell) {
-  __shared__ int32_t partial[1024];
+// Exclusive scan of the cell counts (one workgroup of 1024); leaves the counts zeroed as cursors.
+__global__ void __launch_bounds__(1024) cells_scan_kernel(int32_t* cell_count, int32_t* cell_start, int64_t ncell) {
+  __shared__ int32_t s_wave[17];
   const int t = threadIdx.x, T = blockDim.x;
   const int64_t chunk = fmd_cdiv(ncell, T);
-  const int64_t lo = t * chunk, hi = lo + chunk < ncell ? lo + chunk : ncell;
+  const int64_t lo = t * chunk < ncell ? t * chunk : ncell, hi = lo + chunk < ncell ? lo + chunk : ncell;
   int32_t s = 0;
   for (int64_t c = lo; c < hi; ++c) s += cell_count[c];
-  partial[t] = s;
-  __syncthreads();
-  if (t == 0) {
-    int32_t run = 0;
-    for (int k = 0; k < T; ++k) {
-      int32_t v = partial[k];
-      partial[k] = run;
-      run += v;
-    }
-    cell_start[ncell] = run;
-  }
-  __syncthreads();
-  int32_t run = partial[t];
+  int32_t total;
+  int32_t run = block_exclusive_scan<int32_t>(s, s_wave, &total);
+  if (t == 0) cell_start[ncell] = total;
   for (int64_t c = lo; c < hi; ++c) {
     int32_t v = cell_count[c];
     cell_start[c] = run;
@@ -199,57 +189,83 @@ __device__ __forceinline__ uint64_t cand_key(int32_t j, int sx, int sy, int sz) 
          (uint64_t)(sz + 128);
 }
 
-// One workgroup per atom: test every atom of the cells within reach (all periodic images),
+struct QueryArgs {
+  const float* wrapped;
+  const float* frac;
+  const float* cell;
+  int64_t n;
+  float cutoff2;
+  int n0, n1, n2, r0, r1, r2;
+  int32_t bmax;
+  int lcap;      // LDS keys of the workgroup form
+  int pad_mode;  // which unused slots are written, see query_slots
+  const int32_t* cell_start;
+  const int32_t* cell_atoms;
+  int32_t* neighbor_matrix;
+  int32_t* neighbor_shifts;
+  int32_t* num_neighbors;
+  uint8_t* capacity_valid;
+  int64_t system_size;
+  int64_t index_offset;
+};
+
+// The slots of atom i that a search writes, [0, end): its candidates and then the pad value, up to
+//   FMD_NL_PAD_ALL    the whole row (24 KB at the 1 504 slots of an 8 A candidate cutoff, of which a
+//                     crystal uses 50: 962 MB at 40 000 atoms, 487 us);
+//   FMD_NL_PAD_STALE  the row's previous candidates: slots past num_neighbors' old value hold the pad
+//                     value already;
+//   FMD_NL_PAD_NONE   the candidates alone (rows of a caller that reads no further than its count).
+__device__ __forceinline__ int query_slots(const QueryArgs& a, int64_t i, int stored, int pad_mode) {
+  const int used = stored < a.bmax ? stored : a.bmax;
+  if (pad_mode == FMD_NL_PAD_NONE) return used;
+  if (pad_mode == FMD_NL_PAD_ALL) return a.bmax;
+  const int old = a.num_neighbors[i] < a.bmax ? a.num_neighbors[i] : a.bmax;
+  return old > used ? old : used;
+}
+
+// A workgroup searches for one atom: test every atom of the cells within reach (all periodic images),
 // collect the candidate keys in LDS, bitonic-sort them and write the row.
-__global__ void __launch_bounds__(256) cells_query_kernel(const float* wrapped, const float* frac, const float* cell,
-                                                          int64_t n, float cutoff2, int n0, int n1, int n2, int r0,
-                                                          int r1, int r2, int32_t bmax, int lcap,
-                                                          const int32_t* cell_start, const int32_t* cell_atoms,
-                                                          int32_t* neighbor_matrix, int32_t* neighbor_shifts,
-                                                          int32_t* num_neighbors, uint8_t* capacity_valid,
-                                                          int64_t system_size, int64_t index_offset) {
-  extern __shared__ uint64_t keys[];
+__device__ __forceinline__ void query_atom(const QueryArgs& a, int64_t i, uint64_t* keys) {
   __shared__ int counter;
-  const int64_t i = blockIdx.x;
   const int t = threadIdx.x;
   if (t == 0) counter = 0;
   __syncthreads();
-  Mat3 cm = load_mat3(cell);
-  const float xi = wrapped[3 * i], yi = wrapped[3 * i + 1], zi = wrapped[3 * i + 2];
-  const int c0 = cell_coord(frac[3 * i], n0), c1 = cell_coord(frac[3 * i + 1], n1), c2 = cell_coord(frac[3 * i + 2], n2);
-  const int span0 = 2 * r0 + 1, span1 = 2 * r1 + 1, span2 = 2 * r2 + 1;
+  Mat3 cm = load_mat3(a.cell);
+  const float xi = a.wrapped[3 * i], yi = a.wrapped[3 * i + 1], zi = a.wrapped[3 * i + 2];
+  const int c0 = cell_coord(a.frac[3 * i], a.n0), c1 = cell_coord(a.frac[3 * i + 1], a.n1), c2 = cell_coord(a.frac[3 * i + 2], a.n2);
+  const int span0 = 2 * a.r0 + 1, span1 = 2 * a.r1 + 1, span2 = 2 * a.r2 + 1;
   const int noff = span0 * span1 * span2;
   for (int q = t; q < noff; q += blockDim.x) {
-    const int d0 = q / (span1 * span2) - r0;
-    const int d1 = (q / span2) % span1 - r1;
-    const int d2 = q % span2 - r2;
+    const int d0 = q / (span1 * span2) - a.r0;
+    const int d1 = (q / span2) % span1 - a.r1;
+    const int d2 = q % span2 - a.r2;
     int t0 = c0 + d0, t1 = c1 + d1, t2 = c2 + d2;
     // floor division into (cell, image shift)
-    int s0 = (t0 >= 0) ? t0 / n0 : -((-t0 + n0 - 1) / n0);
-    int s1 = (t1 >= 0) ? t1 / n1 : -((-t1 + n1 - 1) / n1);
-    int s2 = (t2 >= 0) ? t2 / n2 : -((-t2 + n2 - 1) / n2);
-    t0 -= s0 * n0;
-    t1 -= s1 * n1;
-    t2 -= s2 * n2;
-    const int cid = (t0 * n1 + t1) * n2 + t2;
+    int s0 = (t0 >= 0) ? t0 / a.n0 : -((-t0 + a.n0 - 1) / a.n0);
+    int s1 = (t1 >= 0) ? t1 / a.n1 : -((-t1 + a.n1 - 1) / a.n1);
+    int s2 = (t2 >= 0) ? t2 / a.n2 : -((-t2 + a.n2 - 1) / a.n2);
+    t0 -= s0 * a.n0;
+    t1 -= s1 * a.n1;
+    t2 -= s2 * a.n2;
+    const int cid = (t0 * a.n1 + t1) * a.n2 + t2;
     const float sx = (float)s0, sy = (float)s1, sz = (float)s2;
-    for (int p = cell_start[cid]; p < cell_start[cid + 1]; ++p) {
-      const int32_t j = cell_atoms[p];
+    for (int p = a.cell_start[cid]; p < a.cell_start[cid + 1]; ++p) {
+      const int32_t j = a.cell_atoms[p];
       if (j == i && s0 == 0 && s1 == 0 && s2 == 0) continue;
       // replicas of one system side by side (atoms [k S, (k+1) S) each): no pair across them
-      if (system_size > 0 && (int64_t)j / system_size != i / system_size) continue;
-      const float d2v = pair_d2(xi, yi, zi, wrapped[3 * j], wrapped[3 * j + 1], wrapped[3 * j + 2], sx, sy, sz, cm);
-      if (d2v < cutoff2) {
+      if (a.system_size > 0 && (int64_t)j / a.system_size != i / a.system_size) continue;
+      const float d2v = pair_d2(xi, yi, zi, a.wrapped[3 * j], a.wrapped[3 * j + 1], a.wrapped[3 * j + 2], sx, sy, sz, cm);
+      if (d2v < a.cutoff2) {
         int slot = atomicAdd(&counter, 1);
-        if (slot < lcap) keys[slot] = cand_key(j, s0, s1, s2);
+        if (slot < a.lcap) keys[slot] = cand_key(j, s0, s1, s2);
       }
     }
   }
   __syncthreads();
   const int count = counter;
   // a row whose candidates overflowed the LDS keys holds an arrival-order subset of them: it is
-  // stored empty instead (deterministic; the row is flagged invalid below since lcap >= bmax)
-  const int stored = count <= lcap ? count : 0;
+  // stored empty instead (deterministic; the row is flagged invalid below since a.lcap >= a.bmax)
+  const int stored = count <= a.lcap ? count : 0;
   int P = 1;
   while (P < stored) P <<= 1;
   for (int k = stored + t; k < P; k += blockDim.x) keys[k] = ~0ull;
@@ -261,23 +277,24 @@ __global__ void __launch_bounds__(256) cells_query_kernel(const float* wrapped, 
         const int lo = 2 * k - (k & (stride - 1));
         const int hi = lo + stride;
         const bool up = ((lo & size) == 0);
-        const uint64_t a = keys[lo], b = keys[hi];
-        if ((a > b) == up) {
-          keys[lo] = b;
-          keys[hi] = a;
+        const uint64_t x = keys[lo], y = keys[hi];
+        if ((x > y) == up) {
+          keys[lo] = y;
+          keys[hi] = x;
         }
       }
       __syncthreads();
     }
   }
-  int32_t* nrow = neighbor_matrix + i * bmax;
-  int32_t* srow = neighbor_shifts + i * bmax * 3;
-  for (int s = t; s < bmax; s += blockDim.x) {
-    int32_t j = (int32_t)(n + index_offset);
+  const int end = query_slots(a, i, stored, a.pad_mode);
+  int32_t* nrow = a.neighbor_matrix + i * a.bmax;
+  int32_t* srow = a.neighbor_shifts + i * a.bmax * 3;
+  for (int s = t; s < end; s += blockDim.x) {
+    int32_t j = (int32_t)(a.n + a.index_offset);
     int sx = 0, sy = 0, sz = 0;
     if (s < stored) {
       const uint64_t key = keys[s];
-      j = (int32_t)((int64_t)(key >> 24) + index_offset);
+      j = (int32_t)((int64_t)(key >> 24) + a.index_offset);
       sx = (int)((key >> 16) & 0xff) - 128;
       sy = (int)((key >> 8) & 0xff) - 128;
       sz = (int)(key & 0xff) - 128;
@@ -287,9 +304,155 @@ __global__ void __launch_bounds__(256) cells_query_kernel(const float* wrapped, 
     srow[3 * s + 1] = sy;
     srow[3 * s + 2] = sz;
   }
+  __syncthreads();  // the old count has been read
   if (t == 0) {
-    num_neighbors[i] = count;
-    if (count > bmax) capacity_valid[0] = 0;
+    a.num_neighbors[i] = count;
+    if (count > a.bmax) a.capacity_valid[0] = 0;
+  }
+}
+
+// The workgroup form for every atom, or (SPARSE) for those whose candidates overflowed the wave form's
+// keys, 16 atoms per workgroup (all of them past it cost no more than a workgroup each).
+constexpr int kWaveKeys = 256;  // candidate keys of a wave
+constexpr int kSparseAtoms = 16;
+
+template <bool SPARSE>
+__global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a) {
+  extern __shared__ uint64_t keys[];
+  if (!SPARSE) {
+    query_atom(a, blockIdx.x, keys);
+    return;
+  }
+  const int64_t i0 = (int64_t)blockIdx.x * kSparseAtoms;
+  const int64_t mine = i0 + (threadIdx.x & (kSparseAtoms - 1));
+  const int count = mine < a.n ? a.num_neighbors[mine] : 0;
+  if (!__any(count > kWaveKeys)) return;  // every wave of the workgroup sees the same 16 counts
+  for (int k = 0; k < kSparseAtoms; ++k) {
+    __syncthreads();  // keys and counter are free
+    if (__shfl(count, k, FMD_WAVE) > kWaveKeys) query_atom(a, i0 + k, keys);
+  }
+}
+
+// One wave per atom: 64 cells at a time (a scan of their atom counts), then their atoms 64 at a time,
+// each lane finding its cell in the scanned counts, so that every lane tests an atom and the loads of
+// a pass go out together; candidate keys appended to the wave's LDS list by ballot. The list is put in
+// order by rank: a key's slot is the number of smaller keys (up to four keys per lane against the list,
+// read as LDS broadcasts), written straight to the row. More than kWaveKeys candidates: the count alone,
+// for the workgroup form. Bound by the latency of its loads (27 cells, 320 atoms per atom at 40 000):
+// 40 000 atoms 487 -> 65 us with the rows' unused slots no longer written.
+__global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a) {
+  __shared__ uint64_t s_keys[256 / FMD_WAVE][kWaveKeys];
+  __shared__ int32_t s_first[256 / FMD_WAVE][FMD_WAVE];  // scanned atom counts of the wave's 64 cells
+  __shared__ int32_t s_start[256 / FMD_WAVE][FMD_WAVE];
+  __shared__ uint32_t s_shift[256 / FMD_WAVE][FMD_WAVE];
+  const int lane = threadIdx.x & (FMD_WAVE - 1), wave = threadIdx.x / FMD_WAVE;
+  const int64_t i = (int64_t)blockIdx.x * (256 / FMD_WAVE) + wave;
+  if (i >= a.n) return;  // no barrier below: every wave works on its own share of the LDS
+  uint64_t* keys = s_keys[wave];
+  int32_t *first = s_first[wave], *start = s_start[wave];
+  uint32_t* shift = s_shift[wave];
+  const Mat3 cm = load_mat3(a.cell);
+  const float xi = a.wrapped[3 * i], yi = a.wrapped[3 * i + 1], zi = a.wrapped[3 * i + 2];
+  const int c0 = cell_coord(a.frac[3 * i], a.n0), c1 = cell_coord(a.frac[3 * i + 1], a.n1),
+            c2 = cell_coord(a.frac[3 * i + 2], a.n2);
+  const int span1 = 2 * a.r1 + 1, span2 = 2 * a.r2 + 1, noff = (2 * a.r0 + 1) * span1 * span2;
+  int count = 0;
+  for (int q0 = 0; q0 < noff; q0 += FMD_WAVE) {
+    const int q = q0 + lane;
+    int from = 0, atoms = 0;
+    uint32_t packed = 0;
+    if (q < noff) {
+      int t0 = c0 + q / (span1 * span2) - a.r0, t1 = c1 + (q / span2) % span1 - a.r1, t2 = c2 + q % span2 - a.r2;
+      // floor division into (cell, image shift)
+      const int s0 = t0 >= 0 ? t0 / a.n0 : -((-t0 + a.n0 - 1) / a.n0);
+      const int s1 = t1 >= 0 ? t1 / a.n1 : -((-t1 + a.n1 - 1) / a.n1);
+      const int s2 = t2 >= 0 ? t2 / a.n2 : -((-t2 + a.n2 - 1) / a.n2);
+      t0 -= s0 * a.n0;
+      t1 -= s1 * a.n1;
+      t2 -= s2 * a.n2;
+      const int cid = (t0 * a.n1 + t1) * a.n2 + t2;
+      from = a.cell_start[cid];
+      atoms = a.cell_start[cid + 1] - from;
+      packed = ((uint32_t)(s0 + 128) << 16) | ((uint32_t)(s1 + 128) << 8) | (uint32_t)(s2 + 128);
+    }
+    int incl = atoms;
+#pragma unroll
+    for (int off = 1; off < FMD_WAVE; off <<= 1) {
+      const int o = __shfl_up(incl, off, FMD_WAVE);
+      if (lane >= off) incl += o;
+    }
+    first[lane] = incl - atoms;
+    start[lane] = from;
+    shift[lane] = packed;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int total = __shfl(incl, FMD_WAVE - 1, FMD_WAVE);
+    for (int f0 = 0; f0 < total; f0 += FMD_WAVE) {
+      const int f = f0 + lane;
+      bool hit = false;
+      uint64_t key = 0;
+      if (f < total) {
+        int c = 0;  // the last cell whose first atom is at or before f (empty cells before it share its first)
+#pragma unroll
+        for (int step = FMD_WAVE / 2; step > 0; step >>= 1)
+          if (first[c + step] <= f) c += step;
+        const int32_t j = a.cell_atoms[start[c] + (f - first[c])];
+        const uint32_t sh = shift[c];
+        const int sx = (int)(sh >> 16) - 128, sy = (int)((sh >> 8) & 0xff) - 128, sz = (int)(sh & 0xff) - 128;
+        const float d2 = pair_d2(xi, yi, zi, a.wrapped[3 * j], a.wrapped[3 * j + 1], a.wrapped[3 * j + 2], (float)sx,
+                                 (float)sy, (float)sz, cm);
+        hit = d2 < a.cutoff2 && !(j == i && sx == 0 && sy == 0 && sz == 0);
+        // replicas of one system side by side (atoms [k S, (k+1) S) each): no pair across them
+        if (a.system_size > 0) hit = hit && (int64_t)j / a.system_size == i / a.system_size;
+        key = cand_key(j, sx, sy, sz);
+      }
+      const uint64_t m = __ballot(hit);
+      const int slot = count + lane_prefix(m);
+      if (hit && slot < kWaveKeys) keys[slot] = key;
+      count += __popcll(m);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  const bool fits = count <= kWaveKeys;
+  if (fits) {
+    const int end = query_slots(a, i, count, a.pad_mode);
+    int32_t* nrow = a.neighbor_matrix + i * a.bmax;
+    int32_t* srow = a.neighbor_shifts + i * a.bmax * 3;
+    uint64_t mine[kWaveKeys / FMD_WAVE];
+    int rank[kWaveKeys / FMD_WAVE];
+#pragma unroll
+    for (int u = 0; u < kWaveKeys / FMD_WAVE; ++u) {
+      const int s = u * FMD_WAVE + lane;
+      mine[u] = s < count ? keys[s] : ~0ull;
+      rank[u] = 0;
+    }
+    if (count <= FMD_WAVE) {
+      for (int s = 0; s < count; ++s) rank[0] += keys[s] < mine[0];
+    } else {
+      for (int s = 0; s < count; ++s) {
+        const uint64_t k = keys[s];
+#pragma unroll
+        for (int u = 0; u < kWaveKeys / FMD_WAVE; ++u) rank[u] += k < mine[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kWaveKeys / FMD_WAVE; ++u) {
+      if (u * FMD_WAVE + lane >= count || rank[u] >= a.bmax) continue;
+      const uint64_t key = mine[u];
+      nrow[rank[u]] = (int32_t)((int64_t)(key >> 24) + a.index_offset);
+      srow[3 * rank[u]] = (int)((key >> 16) & 0xff) - 128;
+      srow[3 * rank[u] + 1] = (int)((key >> 8) & 0xff) - 128;
+      srow[3 * rank[u] + 2] = (int)(key & 0xff) - 128;
+    }
+    for (int s = count + lane; s < end; s += FMD_WAVE) {
+      nrow[s] = (int32_t)(a.n + a.index_offset);
+      srow[3 * s] = srow[3 * s + 1] = srow[3 * s + 2] = 0;
+    }
+  }
+  if (lane == 0) {
+    a.num_neighbors[i] = count;
+    if (count > a.bmax) a.capacity_valid[0] = 0;
   }
 }
 
@@ -1160,12 +1323,13 @@ int fmd_nl_wrap(const void* positions, int32_t pos_is_f64, const float* inv_cell
   return FMD_OK;
 }
 
-int fmd_nl_candidates(const float* wrapped, const float* frac, const float* cell, int64_t n_atoms, float cutoff2,
-                      const int32_t* ncells, const int32_t* reach, int32_t bmax, int32_t* cell_count,
+int fmd_nl_candidates_pad(const float* wrapped, const float* frac, const float* cell, int64_t n_atoms, float cutoff2,
+                          const int32_t* ncells, const int32_t* reach, int32_t bmax, int32_t* cell_count,
                       int32_t* cell_start, int32_t* cell_atoms, int32_t* neighbor_matrix, int32_t* neighbor_shifts,
                       int32_t* num_neighbors, uint8_t* capacity_valid, int64_t system_size, int64_t index_offset,
-                      hipStream_t stream) {
+                          int32_t pad_mode, hipStream_t stream) {
   FMD_REQUIRE(n_atoms > 0 && bmax > 0 && ncells && reach);
+  FMD_REQUIRE(pad_mode >= FMD_NL_PAD_ALL && pad_mode <= FMD_NL_PAD_NONE);
   FMD_REQUIRE(index_offset >= 0 && n_atoms + index_offset < (int64_t(1) << 31));
   FMD_REQUIRE(system_size >= 0 && (system_size == 0 || n_atoms % system_size == 0));
   const int n0 = ncells[0], n1 = ncells[1], n2 = ncells[2];
@@ -1190,11 +1354,35 @@ int fmd_nl_candidates(const float* wrapped, const float* frac, const float* cell
   hipLaunchKernelGGL(cells_place_kernel, dim3((unsigned)fmd_cdiv(n_atoms, threads)), dim3(threads), 0, stream, frac,
                      n_atoms, n0, n1, n2, cell_count, cell_start, cell_atoms);
   FMD_CHECK_LAUNCH();
-  hipLaunchKernelGGL(cells_query_kernel, dim3((unsigned)n_atoms), dim3(256), (size_t)lcap * sizeof(uint64_t), stream,
-                     wrapped, frac, cell, n_atoms, cutoff2, n0, n1, n2, r0, r1, r2, bmax, lcap, cell_start, cell_atoms,
-                     neighbor_matrix, neighbor_shifts, num_neighbors, capacity_valid, system_size, index_offset);
+  QueryArgs a{wrapped, frac, cell, n_atoms, cutoff2, n0, n1, n2, r0, r1, r2, bmax, lcap, pad_mode, cell_start, cell_atoms,
+              neighbor_matrix, neighbor_shifts, num_neighbors, capacity_valid, system_size, index_offset};
+  const size_t lds = (size_t)lcap * sizeof(uint64_t);
+  // A cell is at least the cutoff thick along each axis, so an atom has at most about 4.2 (the sphere in
+  // cutoffs cubed) times the mean atoms per cell as candidates. The wave form where three quarters of
+  // its keys hold that; rows past its keys (an inhomogeneous system) go to the workgroup form after it.
+  // The workgroup form alone where the mean row would: it searches such rows once.
+  if (4.19 * (double)n_atoms / (double)ncell <= 0.75 * kWaveKeys) {
+    hipLaunchKernelGGL(cells_query_wave_kernel, dim3((unsigned)fmd_cdiv(n_atoms, 256 / FMD_WAVE)), dim3(256), 0, stream,
+                       a);
+    FMD_CHECK_LAUNCH();
+    a.pad_mode = pad_mode == FMD_NL_PAD_NONE ? FMD_NL_PAD_NONE : FMD_NL_PAD_ALL;  // the old counts are gone
+    hipLaunchKernelGGL(cells_query_kernel<true>, dim3((unsigned)fmd_cdiv(n_atoms, kSparseAtoms)), dim3(256), lds, stream,
+                       a);
+  } else {
+    hipLaunchKernelGGL(cells_query_kernel<false>, dim3((unsigned)n_atoms), dim3(256), lds, stream, a);
+  }
   FMD_CHECK_LAUNCH();
   return FMD_OK;
+}
+
+int fmd_nl_candidates(const float* wrapped, const float* frac, const float* cell, int64_t n_atoms, float cutoff2,
+                      const int32_t* ncells, const int32_t* reach, int32_t bmax, int32_t* cell_count,
+                      int32_t* cell_start, int32_t* cell_atoms, int32_t* neighbor_matrix, int32_t* neighbor_shifts,
+                      int32_t* num_neighbors, uint8_t* capacity_valid, int64_t system_size, int64_t index_offset,
+                      hipStream_t stream) {
+  return fmd_nl_candidates_pad(wrapped, frac, cell, n_atoms, cutoff2, ncells, reach, bmax, cell_count, cell_start,
+                               cell_atoms, neighbor_matrix, neighbor_shifts, num_neighbors, capacity_valid, system_size,
+                               index_offset, FMD_NL_PAD_ALL, stream);
 }
 
 int64_t fmd_nl_build_work_size(int64_t n_atoms) {

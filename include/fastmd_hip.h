@@ -63,6 +63,25 @@ int fmd_nl_candidates(const float* wrapped, const float* frac, const float* cell
                       uint8_t* capacity_valid, int64_t system_size, int64_t index_offset,
                       hipStream_t stream);
 
+/* fmd_nl_candidates writes every slot of every row. With FMD_NL_PAD_STALE (num_neighbors holds the
+ * counts of the rows' last search and the slots past them the pad value) only the slots up to the
+ * old and the new count are written: the same rows; with FMD_NL_PAD_NONE the unused slots are left
+ * as they are. */
+#define FMD_NL_PAD_ALL 0
+#define FMD_NL_PAD_STALE 1
+#define FMD_NL_PAD_NONE 2
+int fmd_nl_candidates_pad(const float* wrapped, const float* frac, const float* cell, int64_t n_atoms,
+                      float cutoff2, const int32_t* ncells, const int32_t* reach, int32_t bmax,
+                      int32_t* cell_count, int32_t* cell_start, int32_t* cell_atoms,
+                      int32_t* neighbor_matrix, int32_t* neighbor_shifts, int32_t* num_neighbors,
+                      uint8_t* capacity_valid, int64_t system_size, int64_t index_offset,
+                      int32_t pad_mode, hipStream_t stream);
+
+/* order [n_atoms] = the atoms in stable order of the Morton code (10 bits per axis) of their
+ * fractional coordinates [n, 3], for kernels that take one atom per wave in this order. work:
+ * fmd_csr_work_size(n_atoms) uint32 of scratch. No counterpart in the reference. */
+int fmd_nl_atom_order(const float* frac, int64_t n_atoms, uint32_t* work, int32_t* order, hipStream_t stream);
+
 /* Wrap (refresh flavour): float32 positions -> fractional coordinates in [0,1), integer
  * wraps and wrapped Cartesian coordinates; optionally resets the reference positions/wraps
  * and the wrap delta (refresh). `positions` are float32 (pos_is_f64 = 0) or float64 (1, cast
