@@ -24,7 +24,11 @@
 namespace {
 
 constexpr int kSmallThreads = 1024;   // fused single-workgroup build
-constexpr int kSmallMaxAtoms = 1024;  // LDS-resident wrapped coordinates up to this many atoms
+// The fused build up to this many atoms. Its one workgroup walks its atoms in turn, while the three
+// launches of the multi-block build cost the same 13 us at any size here (graph-captured builds with
+// reverse rows and window fold, us fused / three launches: 40 atoms 11.1 / 12.1, 60 12.8 / 12.7,
+// 90 16.5 / 12.9, 135 21.4 / 13.3, 400 51 / 13.5, 900 138 / 13.9).
+constexpr int kSmallMaxAtoms = 60;
 constexpr int kSmallBatch = 4;        // atoms per wave whose candidate loads are issued together
 constexpr int kSmallMaxEdges = 8192;  // rows whose reverse search runs on LDS copies of their keys
 constexpr int kImageBias = 512;       // packed image fields: component + 512 in 10 bits
@@ -1247,7 +1251,7 @@ int launch_build(const BuildArgs& a, hipStream_t stream) {
   FMD_REQUIRE(a.max_disp && a.cand_valid && a.overflow && a.isolated);
   FMD_REQUIRE(!a.system_of || a.pad_images);
   FMD_REQUIRE(a.n_dummy >= 0 && (a.n_dummy == 0 || !a.system_of) && a.n + a.n_dummy < (int64_t(1) << 31));
-  if (a.n <= kSmallMaxAtoms && a.n <= 1024) {
+  if (a.n <= kSmallMaxAtoms) {
     hipLaunchKernelGGL(nl_build_small_kernel, dim3(1), dim3(kSmallThreads), 0, stream, a);
     FMD_CHECK_LAUNCH();
     return FMD_OK;

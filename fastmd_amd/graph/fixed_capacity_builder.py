@@ -9,7 +9,7 @@ a fixed sequence of kernels with device-side status flags (no host sync, captura
 MI355X design: the candidate rows are written sorted by (neighbour, shift) at refresh, so the
 per-step rows come out in the canonical (centre, neighbour, image) order directly (the
 reference's per-build ``torch.sort`` of e_cap keys, :1968-1999, is gone); a build is one
-fused single-workgroup kernel up to 1024 atoms, three kernels beyond (count, scan,
+fused single-workgroup kernel up to 60 atoms, three kernels beyond (count, scan,
 materialize+pad), plus the reverse-edge index that the deterministic VJPs use.
 """
 from __future__ import annotations

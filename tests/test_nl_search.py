@@ -93,3 +93,30 @@ def test_morton_order_equals_the_host(n):
     frac[::7] = frac[0].clone()  # equal codes keep their order
     frac[n // 2] = torch.tensor([0.0, 1.0 - 2.0 ** -24, 0.5])
     assert torch.equal(morton_order(frac.cuda()).cpu(), morton_order(frac))
+
+
+@pytest.mark.parametrize("repeats", [(1, 1, 1), (2, 2, 2), (2, 2, 3), (1, 1, 13)])
+@pytest.mark.parametrize("short", [0, 40])
+def test_build_on_either_side_of_the_fused_form(device, repeats, short):
+    """5, 40, 60 atoms in one workgroup (the most of that form), 65 in three launches: every published
+    buffer bit-exact against the oracle, with rows to spare and with too few."""
+    from test_nl import _assert_build_equal, _oracle_build
+
+    from fastmd_amd import systems
+    from fastmd_amd.graph.fixed_capacity_builder import FixedCapacityGraphBuilder
+
+    s = systems.perovskite(repeats)
+    pairs = 9 * s.n_atoms - short // 2 * (s.n_atoms // 10)
+    builder = FixedCapacityGraphBuilder(cell=torch.tensor(s.cell, dtype=torch.float32), t_capacity=0,
+                                        atomic_numbers=torch.ones(s.n_atoms), u_capacity=pairs,
+                                        line_graph_cutoff=None, atom_graph_cutoff=6.0, candidate_cutoff=8.0,
+                                        padding=PaddingRule("far_self_loops"), device=device)
+    rng = np.random.default_rng(0)
+    cand, _, _ = _oracle_build(s.cell, s.positions, 6.0, 2.0, builder.e_capacity, inv=builder.inv_cell.cpu().numpy())
+    builder.refresh_candidates(torch.tensor(s.positions, device=device))
+    moved = s.positions + rng.normal(0, 0.1, s.positions.shape)
+    builder.build(torch.tensor(moved, device=device), rebuild_candidates=False)
+    _, ob, _ = _oracle_build(s.cell, moved, 6.0, 2.0, builder.e_capacity, ref_positions=s.positions,
+                             inv=builder.inv_cell.cpu().numpy())
+    _assert_build_equal(builder, ob, cand)
+    assert short == 0 or s.n_atoms < 10 or bool(builder._overflow.item())
