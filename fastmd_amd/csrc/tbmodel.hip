@@ -347,10 +347,21 @@ constexpr int bond_pass() {
 }
 constexpr int kRunBatch = 4;
 
-// eps[b] += scale * sum over b's triplets (first bond), in order, of silu(z3[k]) s_b s_b2
-template <int NC>
-__global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, const float* z3, int64_t ldz, int C,
-                                                           const float* geo, float scale, float* eps, int64_t lde) {
+// The pre-activation of a triplet from its bonds' and its atom's rows: z3[k] = u[b1] + v[b2] + h[atom] + aw[k].
+struct TripletTerms {
+  const float* u;  // [e_cap] rows (bond rows only), row stride ldu; null: z3 is given
+  const float* v;
+  const float* h;   // [n] rows, row stride ldh
+  const float* aw;  // [t_cap] rows, row stride lda
+  int64_t ldu, ldh, lda;
+};
+
+// eps[b] += scale * sum over b's triplets (first bond), in order, of silu(z3[k]) s_b s_b2. FORM: z3 is
+// formed here from its four rows and stored for the VJP, else read.
+template <int NC, bool FORM>
+__global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, float* z3, int64_t ldz, int C,
+                                                           const TripletTerms tt, const float* geo, float scale,
+                                                           float* eps, int64_t lde) {
   constexpr int U = bond_pass<NC>(), TQ = kRunBatch;
   const int lane = threadIdx.x & 63;
   const LaneCols<NC> cols(C);
@@ -367,17 +378,32 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, const floa
     bool empty;
     const int64_t ks = bs.slot_row(qs, lane % TQ, empty);
     const int b2raw = lc.line[5 * ks + 4];
+    const int bq = __shfl(bs.b, qs, 64);
+    const int b2 = empty ? bq : b2raw;  // an empty run's slots read the bond's own rows and add nothing
+    float ub[U][NC];
+    if constexpr (FORM) {
+      const int atom_l = empty ? 0 : lc.line[5 * ks];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        const int64_t at = lane_int(atom_l, q * TQ);
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc)
+          ub[q][cc] = tt.u[bs.bond(q) * tt.ldu + cols.col[cc]] + tt.h[at * tt.ldh + cols.col[cc]];
+      }
+    }
 #pragma unroll
     for (int q = 0; q < U; ++q)
 #pragma unroll
       for (int t = 0; t < TQ; ++t) {
         const int64_t k = lane_int((int)ks, q * TQ + t);
+        const int64_t r2 = FORM ? lane_int(b2, q * TQ + t) : 0;
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) x[q][t][cc] = z3[k * ldz + cols.col[cc]];
+        for (int cc = 0; cc < NC; ++cc)
+          x[q][t][cc] = FORM ? tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]]
+                             : z3[k * ldz + cols.col[cc]];
       }
-    const int bq = __shfl(bs.b, qs, 64);
     const float w1 = geo[8 * (int64_t)bq + 6];
-    const float ws = w1 * geo[8 * (int64_t)(empty ? bq : b2raw) + 6];
+    const float ws = w1 * geo[8 * (int64_t)b2 + 6];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       float acc[NC];
@@ -389,7 +415,10 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, const floa
         const float w = lane_value(ws, q * TQ + t);
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) {
-          const float v = x[q][t][cc] * tb_sigmoid(x[q][t][cc]) * w;
+          const float z = FORM ? x[q][t][cc] + ub[q][cc] : x[q][t][cc];
+          if (FORM && t < cnt && bs.stored(q) && cols.live[cc])
+            z3[(int64_t)lane_int((int)ks, q * TQ + t) * ldz + cols.col[cc]] = z;
+          const float v = z * tb_sigmoid(z) * w;
           acc[cc] = t < cnt ? acc[cc] + v : acc[cc];
         }
       }
@@ -402,15 +431,20 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, const floa
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int64_t k = k0 + (t < m ? t : m - 1);
-          wy[t] = w1q * geo[8 * (int64_t)lc.line[5 * k + 4] + 6];
+          const int64_t r2 = lc.line[5 * k + 4];
+          wy[t] = w1q * geo[8 * r2 + 6];
 #pragma unroll
-          for (int cc = 0; cc < NC; ++cc) y[t][cc] = z3[k * ldz + cols.col[cc]];
+          for (int cc = 0; cc < NC; ++cc)
+            y[t][cc] = FORM ? tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]]
+                            : z3[k * ldz + cols.col[cc]];
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
           for (int cc = 0; cc < NC; ++cc) {
-            const float v = y[t][cc] * tb_sigmoid(y[t][cc]) * wy[t];
+            const float z = FORM ? y[t][cc] + ub[q][cc] : y[t][cc];
+            if (FORM && t < m && bs.stored(q) && cols.live[cc]) z3[(k0 + t) * ldz + cols.col[cc]] = z;
+            const float v = z * tb_sigmoid(z) * wy[t];
             acc[cc] = t < m ? acc[cc] + v : acc[cc];
           }
       }
@@ -498,12 +532,14 @@ __global__ void __launch_bounds__(256) tb_triplet_bwd_kernel(LineCsr lc, const f
 
 // Per bond b: geps[b] += sum over b's triplets as first bond of ga3[k, 0:C], then as second bond
 // of ga3[k, C:2C]; gs[b] (+)= the same sums of gsw[k, 0] and gsw[k, 1] (stored, or added with
-// acc_gs). A second-bond slot of -1 (no triplet) adds zeros.
-template <int NC>
+// acc_gs). A second-bond slot of -1 (no triplet) adds zeros. SPLIT: ga3 is [t_cap, C] (the gradient of
+// z3), and its two sums are stored side by side, geps[b, 0:C] (first bond) and geps[b, C:2C] (second).
+template <int NC, bool SPLIT>
 __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const float* ga3, int64_t lda, int C,
                                                               const float* gsw, float* geps, int64_t ldg, float* gs,
                                                               int acc_gs) {
   constexpr int U = bond_pass<NC>(), TQ = kRunBatch;
+  const int64_t second = SPLIT ? 0 : C;  // column of the second bond's block
   const int lane = threadIdx.x & 63;
   const LaneCols<NC> cols(C);
   const int64_t nb = lc.short_offsets[lc.n], nw = (int64_t)gridDim.x * 4;
@@ -514,7 +550,7 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
 #pragma unroll
     for (int q = 0; q < U; ++q)
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) old[q][cc] = geps[bs.bond(q) * ldg + cols.col[cc]];
+      for (int cc = 0; cc < NC; ++cc) old[q][cc] = SPLIT ? 0.f : geps[bs.bond(q) * ldg + cols.col[cc]];
     // lane l < 2 U TQ: role l / (U TQ), slot ((l % U TQ) / TQ, l % TQ); role 1 through second_perm
     const int sl = lane % (U * TQ), role_l = lane < U * TQ ? 0 : 1;
     bool empty;
@@ -536,7 +572,7 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
       for (int t = 0; t < TQ; ++t) {
         const int k = lane_int(kk, U * TQ + q * TQ + t);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) x[q][1][t][cc] = ga3[(int64_t)(k >= 0 ? k : 0) * lda + C + cols.col[cc]];
+        for (int cc = 0; cc < NC; ++cc) x[q][1][t][cc] = ga3[(int64_t)(k >= 0 ? k : 0) * lda + second + cols.col[cc]];
       }
 #pragma unroll
     for (int q = 0; q < U; ++q) {
@@ -573,7 +609,7 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
             const int64_t k = ky[t] >= 0 ? ky[t] : 0;
             sy[t] = gsw[2 * k + role];
 #pragma unroll
-            for (int cc = 0; cc < NC; ++cc) y[t][cc] = ga3[k * lda + role * C + cols.col[cc]];
+            for (int cc = 0; cc < NC; ++cc) y[t][cc] = ga3[k * lda + role * second + cols.col[cc]];
           }
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
@@ -587,16 +623,344 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
             gsum = use ? gsum + v : gsum;
           }
         }
+        if constexpr (SPLIT) {
+          if (bs.stored(q)) {
+            float* out = geps + bs.bond(q) * ldg + role * C;
+#pragma unroll
+            for (int cc = 0; cc < NC; ++cc)
+              if (cols.live[cc]) out[cols.col[cc]] = acc[cc];
+          }
+#pragma unroll
+          for (int cc = 0; cc < NC; ++cc) acc[cc] = 0.f;
+        }
       }
       if (bs.stored(q)) {
         const int64_t b = bs.bond(q);
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc)
-          if (cols.live[cc]) geps[b * ldg + cols.col[cc]] = old[q][cc] + acc[cc];
+          if (!SPLIT && cols.live[cc]) geps[b * ldg + cols.col[cc]] = old[q][cc] + acc[cc];
         if (lane == 0) gs[b] = lane_value(gs_l, q) + gsum;
       }
     }
   }
+}
+
+// ---- the bond rows' products and the edge sums of the node-factored model. An edge row's pre-activation
+// z2 = h_j W2a + h_i W2b + eps_e W2c takes its first two terms from per-atom rows, and eps_e differs from
+// its initial ef_e We on the bond rows alone (a tenth of the edges): the other rows' last term is
+// ef_e (We W2c), an nb-term sum formed here per row, and the products with C x C blocks run on the
+// bond rows only. No edge-sized product and no triplet-sized one is left (5 000 atoms, 3.5 A: 84 000
+// edges, 10 300 bonds, 26 000 triplets).
+// Against gathering [h_j | eps_e] and [eps_b1 | eps_b2 | h_i] into products over the edge and triplet rows: an MD step
+// of 5 000 atoms at 64 channels 773 -> 698 us, of 375 atoms at 128 channels 767 -> 470, and an evaluation of
+// 500 atoms 988 -> 574.
+
+// C[e, 0:N] (+)= [a0[e] | a1[e]] B^T over the real bonds e = bond_rows[k]: a workgroup takes 16 bonds x 64 columns,
+// each wave one 16 x 16 block of v_mfma_f32_16x16x4_f32 with its operands straight into registers (lane group
+// g = l / 16 holds k = 8 g .. 8 g + 8 of a 32-k slice), the loads of up to four slices in flight: the operands are
+// one round trip per 128 of K behind the row look-up. The count is read on the device, the grid strides. Bound by that
+// chain of round trips: 7.9 us at 400 atoms and 128 channels (12.4 with one wave per 16 x 64 tile and one
+// slice in flight), 11.5 at 10 300 bonds and 64 channels (the same).
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+struct BondProduct {
+  const float *a0, *a1, *b;
+  float* c;
+  int64_t ld0, ld1, ldb, ldc;
+  int k0, k, n, accumulate;  // columns [0, k0) of K from a0, the rest from a1
+};
+
+__device__ __forceinline__ int64_t bond_count(const LineCsr& lc, int64_t e_cap) {
+  const int64_t nb = lc.short_offsets[lc.n];
+  return nb < e_cap ? nb : e_cap;
+}
+
+__global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_t e_cap, const BondProduct p) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
+  const int64_t ct = p.n / 16, tiles = fmd_cdiv(nb, 16) * ct;  // a multiple of four: a workgroup's waves share bonds
+  for (int64_t w = wave_id(); w < tiles; w += nw) {
+    const int64_t tm = w / ct, col = (w - tm * ct) * 16 + i, slot = tm * 16 + i;
+    const int e = lc.bond_rows[slot < nb ? slot : nb - 1];
+    const float *r0 = p.a0 + e * p.ld0, *r1 = p.a1 ? p.a1 + e * p.ld1 : r0, *bp = p.b + col * p.ldb + 8 * g;
+    f32x4_t acc{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < p.k; k0 += 128) {
+      float4 a[4][2], b[4][2];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 32 * q;
+        if (k >= p.k) break;
+        b[q][0] = *reinterpret_cast<const float4*>(bp + k);
+        b[q][1] = *reinterpret_cast<const float4*>(bp + k + 4);
+        const float* ap = (k < p.k0 ? r0 + k : r1 + (k - p.k0)) + 8 * g;
+        a[q][0] = *reinterpret_cast<const float4*>(ap);
+        a[q][1] = *reinterpret_cast<const float4*>(ap + 4);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (k0 + 32 * q >= p.k) break;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][h].x, b[q][h].x, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][h].y, b[q][h].y, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][h].z, b[q][h].z, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][h].w, b[q][h].w, acc, 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int64_t row = __shfl(e, 4 * g + v, 64);
+      if (tm * 16 + 4 * g + v >= nb) continue;
+      float* c = p.c + row * p.ldc + col;
+      *c = p.accumulate ? *c + acc[v] : acc[v];
+    }
+  }
+}
+
+// The bond rows' first values: out[e, block b] = ef[e] m[:, b C : (b + 1) C] for the three blocks of m [nb, 3 C],
+// stored at columns 0, 2 C and 3 C of the row (eps | . | u | v). A wave takes four bonds and 64 columns, eight rows
+// of m in flight together with the bond rows they do not depend on.
+__global__ void __launch_bounds__(256) tb_bond_init_kernel(LineCsr lc, int64_t e_cap, const float* ef, int nbasis,
+                                                           const float* m, int C, float* out, int64_t ldo) {
+  const int lane = threadIdx.x & 63, blocks = fmd_cdiv(3 * C, 64);
+  const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
+  for (int64_t w = wave_id(); w < fmd_cdiv(nb, 4) * blocks; w += nw) {
+    const int64_t j0 = w / blocks * 4;
+    const int c = (int)(w % blocks) * 64 + lane, col = c < 3 * C ? c : 3 * C - 1;
+    // lane l: bond l / 16, its basis values n0 + l % 16
+    const int64_t j = j0 + (lane >> 4);
+    const int mine = lc.bond_rows[j < nb ? j : nb - 1];
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int n0 = 0; n0 < nbasis; n0 += 8) {
+      float wm[8];
+#pragma unroll
+      for (int n = 0; n < 8; ++n) wm[n] = n0 + n < nbasis ? m[(int64_t)(n0 + n) * 3 * C + col] : 0.f;
+      const int nl = n0 + (lane & 7);
+      const float f = nl < nbasis ? ef[(int64_t)mine * nbasis + nl] : 0.f;
+#pragma unroll
+      for (int n = 0; n < 8; ++n)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] += lane_value(f, 16 * q + n) * wm[n];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (j0 + q < nb && c < 3 * C) out[(int64_t)lane_int(mine, 16 * q) * ldo + (c < C ? c : c + C)] = acc[q];
+  }
+}
+
+// gef[e, n] = sum_c geps[e, c] We[n, c] on the bond rows (over what the edge kernel left there).
+template <int NC>
+__global__ void __launch_bounds__(256) tb_bond_basis_kernel(LineCsr lc, int64_t e_cap, const float* geps, int64_t ldg,
+                                                            int C, const float* we, int nbasis, float* gef) {
+  const int lane = threadIdx.x & 63, idx = wave_sum8_index(lane);
+  const LaneCols<NC> lcol(C);
+  const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
+  for (int64_t j = wave_id(); j < nb; j += nw) {
+    const int64_t e = lc.bond_rows[j];
+    float g[NC];
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) g[cc] = lcol.live[cc] ? geps[e * ldg + lcol.col[cc]] : 0.f;
+    for (int n0 = 0; n0 < nbasis; n0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        v[n] = 0.f;
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc)
+          v[n] += n0 + n < nbasis ? g[cc] * we[(int64_t)(n0 + n) * C + lcol.col[cc]] : 0.f;
+      }
+      const float t = wave_sum8(v);
+      if ((lane & 7) == 0 && n0 + idx < nbasis) gef[e * nbasis + n0 + idx] = t;
+    }
+  }
+}
+
+// The edge rows of the sums below.
+struct EdgeRows {
+  const int64_t* off;  // [n + 1]: the rows of each centre
+  int64_t rows, n;
+  int C, nb;
+  const float* geo;  // column 4: the cutoff, the row's weight
+  const float* ef;   // [rows, nb]
+  const float* rt;   // [nb, C] = We W2c
+};
+
+// 8 basis values of 8 rows across the lanes: lane l holds value n0 + l % 8 of row r0 + l / 8 (clamped to m rows)
+__device__ __forceinline__ float basis_lanes(const EdgeRows& er, int64_t r0, int m, int n0) {
+  const int lane = threadIdx.x & 63, n = n0 + (lane & 7);
+  const int64_t r = r0 + ((lane >> 3) < m ? (lane >> 3) : m - 1);
+  return n < er.nb ? er.ef[r * er.nb + n] : 0.f;
+}
+
+template <int NC>
+__device__ __forceinline__ void basis_weights(const EdgeRows& er, int n0, const LaneCols<NC>& lc, float (&w)[8][NC]) {
+#pragma unroll
+  for (int n = 0; n < 8; ++n)
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) w[n][cc] = n0 + n < er.nb ? er.rt[(int64_t)(n0 + n) * er.C + lc.col[cc]] : 0.f;
+}
+
+// h[i] += scale * sum over i's rows of silu(z2) fc, z2 = p[j] + q[i] + (bond row: xb[e], else ef_e rt), stored for
+// the VJP. One wave per centre, batches of 8 rows with their loads issued together (as the gated sums). ONE: nb
+// <= 8, the basis weights stay in registers. Bound by the gathered rows' round trips and the z2 stream (21 MB at
+// 84 000 rows).
+template <int NC, bool ONE>
+__global__ void __launch_bounds__(256) tb_edge_sum_kernel(const EdgeRows er, const float* pq, int64_t ldp,
+                                                          const int32_t* ei, const uint8_t* flags, const float* xb,
+                                                          int64_t ldx, float scale, float* z2, float* h, int64_t ldh) {
+  constexpr int R = 8;
+  const int lane = threadIdx.x & 63;
+  const int64_t s = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (s >= er.n) return;
+  int64_t lo, hi;
+  run_of(er.off, s, er.rows, lo, hi);
+  const LaneCols<NC> lc(er.C);
+  float old[NC], acc[NC], q[NC], w[8][NC];
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc) {
+    old[cc] = h[s * ldh + lc.col[cc]];
+    q[cc] = pq[s * ldp + er.C + lc.col[cc]];
+    acc[cc] = 0.f;
+  }
+  if constexpr (ONE) basis_weights<NC>(er, 0, lc, w);
+  for (int64_t r0 = lo; r0 < hi; r0 += R) {
+    const int m = hi - r0 >= R ? R : (int)(hi - r0);
+    const int64_t rl = r0 + (lane < m ? lane : m - 1);
+    const int nbr = ei[2 * rl + 1];
+    const float fc = er.geo[8 * rl + 4];
+    const int bond = flags[rl];
+    float efl = basis_lanes(er, r0, m, 0);
+    float z[R][NC], xr[R][NC];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const float* pr = pq + (int64_t)lane_int(nbr, j) * ldp;
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) z[j][cc] = pr[lc.col[cc]];
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) xr[j][cc] = 0.f;
+      if (lane_int(bond, j)) {
+        const float* x = xb + (r0 + (j < m ? j : m - 1)) * ldx;
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc) xr[j][cc] = x[lc.col[cc]];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) z[j][cc] = (z[j][cc] + q[cc]) + xr[j][cc];
+    for (int n0 = 0; n0 < er.nb; n0 += 8) {
+      if constexpr (!ONE) {
+        basis_weights<NC>(er, n0, lc, w);
+        if (n0 > 0) efl = basis_lanes(er, r0, m, n0);
+      }
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        if (lane_int(bond, j)) continue;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+          const float f = lane_value(efl, 8 * j + n);
+#pragma unroll
+          for (int cc = 0; cc < NC; ++cc) z[j][cc] += f * w[n][cc];
+        }
+      }
+      if constexpr (ONE) break;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const float f = lane_value(fc, j);
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) {
+        if (j < m && lc.live[cc]) z2[(r0 + j) * er.C + lc.col[cc]] = z[j][cc];
+        const float v = z[j][cc] * tb_sigmoid(z[j][cc]) * f;
+        acc[cc] = j < m ? acc[cc] + v : acc[cc];
+      }
+    }
+  }
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc)
+    if (lc.live[cc]) h[s * ldh + lc.col[cc]] = old[cc] + scale * acc[cc];
+}
+
+// Its VJP: with g = scale gh[i] per row gz2 = g fc silu'(z2), gfc (+)= sum_c g silu(z2), gef[r, n] (+)= sum_c gz2 rt[n]
+// (the basis gradient of the rows that are no bonds; the bond rows' is overwritten at the end), per centre
+// gsum = sum of gz2. The rows' sums are kept on their lanes and stored once per batch.
+template <int NC, bool ONE>
+__global__ void __launch_bounds__(256) tb_edge_sum_bwd_kernel(const EdgeRows er, const float* gh, int64_t ldg,
+                                                              const float* z2, float scale, float* gz, float* gsum,
+                                                              int64_t ldgs, float* gfc, float* gef, int add) {
+  constexpr int R = 8;
+  const int lane = threadIdx.x & 63, idx = wave_sum8_index(lane), row = lane & 7;
+  const int64_t s = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (s >= er.n) return;
+  int64_t lo, hi;
+  run_of(er.off, s, er.rows, lo, hi);
+  const LaneCols<NC> lc(er.C);
+  float g[NC], acc[NC], w[8][NC];
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc) {
+    g[cc] = lc.live[cc] ? scale * gh[s * ldg + lc.col[cc]] : 0.f;
+    acc[cc] = 0.f;
+  }
+  if constexpr (ONE) basis_weights<NC>(er, 0, lc, w);
+  for (int64_t r0 = lo; r0 < hi; r0 += R) {
+    const int m = hi - r0 >= R ? R : (int)(hi - r0);
+    const int64_t rl = r0 + (lane < m ? lane : m - 1);
+    const float fc = er.geo[8 * rl + 4];
+    const float old_fc = add ? gfc[rl] : 0.f;
+    const bool mine = row < m;
+    float v[R][NC];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int64_t r = r0 + (j < m ? j : m - 1);
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) v[j][cc] = z2[r * er.C + lc.col[cc]];
+    }
+    float sums = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const float f = lane_value(fc, j);
+      float p = 0.f;
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) {
+        const float x = v[j][cc], sg = tb_sigmoid(x), si = x * sg;
+        p += g[cc] * si;
+        v[j][cc] = g[cc] * f * (sg + si * (1.0f - sg));
+        acc[cc] = j < m ? acc[cc] + v[j][cc] : acc[cc];
+        if (j < m && lc.live[cc]) gz[(r0 + j) * er.C + lc.col[cc]] = v[j][cc];
+      }
+      const float t = wave_sum(p);
+      sums = lane == j ? t : sums;
+    }
+    if (lane < m) gfc[rl] = old_fc + sums;
+    for (int n0 = 0; n0 < er.nb; n0 += 8) {
+      if constexpr (!ONE) basis_weights<NC>(er, n0, lc, w);
+      const bool use = mine && n0 + idx < er.nb;
+      float* ge = gef + (r0 + (mine ? row : m - 1)) * er.nb + (n0 + idx < er.nb ? n0 + idx : 0);
+      const float old = add && use ? *ge : 0.f;
+      float got = 0.f;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        float d[8];
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+          d[n] = 0.f;
+#pragma unroll
+          for (int cc = 0; cc < NC; ++cc) d[n] += v[j][cc] * w[n][cc];
+        }
+        const float t = wave_sum8(d);
+        got = row == j ? t : got;
+      }
+      if (use) *ge = old + got;
+      if constexpr (ONE) break;
+    }
+  }
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc)
+    if (lc.live[cc]) gsum[s * ldgs + lc.col[cc]] = acc[cc];
 }
 
 RowWeight make_weight(const float* w, int64_t ldw, const int32_t* i1, const int32_t* i2, int64_t ld_idx) {
@@ -612,6 +976,16 @@ RowWeight make_weight(const float* w, int64_t ldw, const int32_t* i1, const int3
       case 3: hipLaunchKernelGGL(KERNEL<3>, GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
       default: hipLaunchKernelGGL(KERNEL<4>, GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
     }                                                                                         \
+  } while (0)
+
+#define TB_LAUNCH_NC2(KERNEL, FLAG, CHANNELS, GRID, ...)                                              \
+  do {                                                                                                \
+    switch (fmd_cdiv((CHANNELS), 64)) {                                                               \
+      case 1: hipLaunchKernelGGL((KERNEL<1, FLAG>), GRID, dim3(256), 0, stream, __VA_ARGS__); break;  \
+      case 2: hipLaunchKernelGGL((KERNEL<2, FLAG>), GRID, dim3(256), 0, stream, __VA_ARGS__); break;  \
+      case 3: hipLaunchKernelGGL((KERNEL<3, FLAG>), GRID, dim3(256), 0, stream, __VA_ARGS__); break;  \
+      default: hipLaunchKernelGGL((KERNEL<4, FLAG>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
+    }                                                                                                 \
   } while (0)
 
 }  // namespace
@@ -671,7 +1045,106 @@ int fmd_tb_bond_sum_f32(const float* z3, int64_t ldz, int32_t channels, const fl
   if (n_atoms == 0 || t_cap == 0) return FMD_OK;
   FMD_REQUIRE(z3 && geo && short_offsets && bond_rows && edge_triplet_offsets && line_graph && eps);
   LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, nullptr, line_graph, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC(tb_bond_sum_kernel, channels, dim3(kStrideBlocks), lc, z3, ldz, channels, geo, scale, eps, lde);
+  TB_LAUNCH_NC2(tb_bond_sum_kernel, false, channels, dim3(kStrideBlocks), lc, const_cast<float*>(z3), ldz, channels,
+                TripletTerms{}, geo, scale, eps, lde);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const float* h, int64_t ldh, const float* aw,
+                           int64_t lda, int32_t channels, const float* geo, const int64_t* short_offsets,
+                           const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
+                           int64_t n_atoms, int64_t t_cap, float scale, float* z3, int64_t ldz, float* eps, int64_t lde,
+                           hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && t_cap >= 0 && channels > 0 && channels <= 256 && ldz >= channels && lde >= channels);
+  FMD_REQUIRE(ldu >= channels && ldh >= channels && lda >= channels);
+  if (n_atoms == 0 || t_cap == 0) return FMD_OK;
+  FMD_REQUIRE(u && v && h && aw && z3 && geo && short_offsets && bond_rows && edge_triplet_offsets && line_graph && eps);
+  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, nullptr, line_graph, nullptr, n_atoms, t_cap};
+  TB_LAUNCH_NC2(tb_bond_sum_kernel, true, channels, dim3(kStrideBlocks), lc, z3, ldz, channels,
+                (TripletTerms{u, v, h, aw, ldu, ldh, lda}), geo, scale, eps, lde);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_bond_init_f32(const float* ef, int32_t n_basis, const float* m, int32_t channels,
+                         const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
+                         float* out, int64_t ldo, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && channels > 0 && n_basis > 0 && ldo >= 4 * (int64_t)channels);
+  if (n_atoms == 0 || e_cap == 0) return FMD_OK;
+  FMD_REQUIRE(ef && m && short_offsets && bond_rows && out);
+  LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
+  hipLaunchKernelGGL(tb_bond_init_kernel, dim3(kStrideBlocks), dim3(256), 0, stream, lc, e_cap, ef, n_basis, m, channels,
+                     out, ldo);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const float* a1, int64_t ld1, int32_t k,
+                            const float* b, int64_t ldb, int32_t n, const int64_t* short_offsets,
+                            const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap, float* c, int64_t ldc,
+                            int32_t accumulate, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && k0 > 0 && k0 % 32 == 0 && k >= k0 && k % 32 == 0 && n > 0 && n % 64 == 0);
+  if (n_atoms == 0 || e_cap == 0) return FMD_OK;
+  FMD_REQUIRE(a0 && ld0 >= k0 && b && ldb >= k && c && ldc >= n && short_offsets && bond_rows);
+  FMD_REQUIRE(k == k0 || (a1 && ld1 >= k - k0));
+  const auto aligned = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  FMD_REQUIRE(aligned(a0) && ld0 % 4 == 0 && aligned(b) && ldb % 4 == 0 && (k == k0 || (aligned(a1) && ld1 % 4 == 0)));
+  LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
+  const BondProduct p{a0, k == k0 ? nullptr : a1, b, c, ld0, ld1, ldb, ldc, k0, k, n, accumulate};
+  hipLaunchKernelGGL(tb_bond_product_kernel, dim3(2 * kStrideBlocks), dim3(256), 0, stream, lc, e_cap, p);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_bond_basis_f32(const float* geps, int64_t ldg, int32_t channels, const float* we, int32_t n_basis,
+                          const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
+                          float* gef, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && channels > 0 && channels <= 256 && n_basis > 0 && ldg >= channels);
+  if (n_atoms == 0 || e_cap == 0) return FMD_OK;
+  FMD_REQUIRE(geps && we && short_offsets && bond_rows && gef);
+  LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
+  TB_LAUNCH_NC(tb_bond_basis_kernel, channels, dim3(kStrideBlocks), lc, e_cap, geps, ldg, channels, we, n_basis, gef);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_edge_sum_f32(const float* pq, int64_t ldp, const int32_t* edge_index, const float* ef, int32_t n_basis,
+                        const float* rt, int32_t channels, const float* geo, const uint8_t* short_flags,
+                        const float* bond_part, int64_t ldx, const int64_t* offsets, int64_t n_atoms, int64_t e_cap,
+                        float scale, float* z2, float* h, int64_t ldh, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && channels > 0 && channels <= 256 && n_basis > 0 && ldx >= channels);
+  FMD_REQUIRE(ldp >= 2 * (int64_t)channels && ldh >= channels);
+  if (n_atoms == 0) return FMD_OK;
+  FMD_REQUIRE(pq && edge_index && ef && rt && geo && short_flags && bond_part && offsets && z2 && h);
+  const EdgeRows er{offsets, e_cap, n_atoms, channels, n_basis, geo, ef, rt};
+  const dim3 grid((unsigned)fmd_cdiv(n_atoms, 4));
+  if (n_basis <= 8)
+    TB_LAUNCH_NC2(tb_edge_sum_kernel, true, channels, grid, er, pq, ldp, edge_index, short_flags, bond_part, ldx, scale,
+                  z2, h, ldh);
+  else
+    TB_LAUNCH_NC2(tb_edge_sum_kernel, false, channels, grid, er, pq, ldp, edge_index, short_flags, bond_part, ldx, scale,
+                  z2, h, ldh);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_edge_sum_bwd_f32(const float* gh, int64_t ldg, const float* z2, int32_t n_basis, const float* rt,
+                            int32_t channels, const float* geo, const int64_t* offsets, int64_t n_atoms, int64_t e_cap,
+                            float scale, float* gz2, float* gsum, int64_t ldgs, float* gfc, float* gef,
+                            int32_t accumulate, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && channels > 0 && channels <= 256 && n_basis > 0);
+  FMD_REQUIRE(ldg >= channels && ldgs >= channels);
+  if (n_atoms == 0) return FMD_OK;
+  FMD_REQUIRE(gh && z2 && rt && geo && offsets && gz2 && gsum && gfc && gef);
+  const EdgeRows er{offsets, e_cap, n_atoms, channels, n_basis, geo, nullptr, rt};
+  const dim3 grid((unsigned)fmd_cdiv(n_atoms, 4));
+  if (n_basis <= 8)
+    TB_LAUNCH_NC2(tb_edge_sum_bwd_kernel, true, channels, grid, er, gh, ldg, z2, scale, gz2, gsum, ldgs, gfc, gef,
+                  accumulate);
+  else
+    TB_LAUNCH_NC2(tb_edge_sum_bwd_kernel, false, channels, grid, er, gh, ldg, z2, scale, gz2, gsum, ldgs, gfc, gef,
+                  accumulate);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }
@@ -699,8 +1172,24 @@ int fmd_tb_bond_reduce_f32(const float* ga3, int64_t lda, int32_t channels, cons
   if (n_atoms == 0 || t_cap == 0) return FMD_OK;
   FMD_REQUIRE(ga3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && geps && gs);
   LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC(tb_bond_reduce_kernel, channels, dim3(kStrideBlocks), lc, ga3, lda, channels, gsw, geps, ldg, gs,
-               accumulate_gs);
+  TB_LAUNCH_NC2(tb_bond_reduce_kernel, false, channels, dim3(kStrideBlocks), lc, ga3, lda, channels, gsw, geps, ldg, gs,
+                accumulate_gs);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_bond_gradient_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
+                             const int64_t* short_offsets, const int32_t* bond_rows,
+                             const int64_t* edge_triplet_offsets, const int32_t* second_perm, int64_t n_atoms,
+                             int64_t t_cap, float* guv, int64_t ldg, float* gs, int32_t accumulate_gs,
+                             hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && t_cap >= 0 && channels > 0 && channels <= 256 && ldz >= channels);
+  FMD_REQUIRE(ldg >= 2 * (int64_t)channels);
+  if (n_atoms == 0 || t_cap == 0) return FMD_OK;
+  FMD_REQUIRE(gz3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && guv && gs);
+  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, nullptr, n_atoms, t_cap};
+  TB_LAUNCH_NC2(tb_bond_reduce_kernel, true, channels, dim3(kStrideBlocks), lc, gz3, ldz, channels, gsw, guv, ldg, gs,
+                accumulate_gs);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

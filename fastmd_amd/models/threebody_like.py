@@ -23,13 +23,20 @@ Model (per layer t; atom features h [N, C], bond features eps [E, C] on every di
   readout:     E_i = e0[Z_i] + h_i . wr
 Random init from ``torch.Generator().manual_seed(seed)``.
 
-dE/dpos is formed by explicit VJP kernels (one autograd node). Atom update: the gated-sum VJP
-gives the pre-activation gradients gz2, their per-centre sums and the cutoff gradient; by
-linearity the node gradient is the product of the per-centre and per-sender sums with the weight
-blocks, so only gz2 W2c^T is formed on the edge rows. Three-body update: per triplet gz3 and the
-envelope terms, ga3 = gz3 W3^T on the triplet rows (far fewer than the edges), then per bond the
-sums over its triplets as first and as second bond, per atom over its triplets. The Fourier VJP
-runs once over all layers' angle gradients.
+Evaluation. Both pre-activations are sums of products of one feature row with one weight block, so
+the products are formed where the feature lives and gathered, never on the edge or triplet rows:
+z3_k = U[b1] + V[b2] + H[i] + aw_k with U = eps W3a, V = eps W3b on the bond rows and H = h W3c per
+atom; z2_e = P[j] + Q[i] + (eps_e W2c) with P = h W2a, Q = h W2b per atom. eps_e differs from ef_e We
+on the bond rows only (about a tenth of the edges): on the others the last term is ef_e (We W2c), an
+n_basis-term sum in the edge kernel, and eps exists on the bond rows alone.
+
+dE/dpos is formed by explicit VJP kernels (one autograd node). Atom update: gz2 per edge, its
+per-centre and per-sender sums, the cutoff's gradient and, on the rows that are no bonds, the basis
+gradient gz2 (We W2c)^T. Three-body update: per triplet gz3 and the envelope terms, per bond its sums
+over the triplets as first and as second bond (gU, gV), per atom its sum. Then one product per layer
+on the bond rows, geps += [gz2 | gU' | gV'] [W2c; W3a'; W3b']^T (' = the next layer's), and one on the
+atoms, gh += [S_src | S_dst | S_tri] [W2a; W2b; W3c]^T. The Fourier VJP runs once over all layers'
+angle gradients.
 """
 from __future__ import annotations
 
@@ -45,7 +52,7 @@ from fastmd_amd.adapters.protocol import (CapacityStep, CaptureContract, GraphBa
                                          require_atom_rows, system_rows)
 from fastmd_amd.ops.csr_segment_sum import Csr, segment_sum_csr
 from fastmd_amd.ops.threebody import LineGraph, fourier_line_vjp
-from fastmd_amd.ops.wide_gemm import gemm, gemm_gather, gemm_group, split_planes
+from fastmd_amd.ops.wide_gemm import gemm, gemm_group, split_planes
 
 _ELEMENTS = 118
 # pairs and triplets in tiers of 128 with at least 128 of padding, held at 1.01x the pair and 1.06x
@@ -121,20 +128,30 @@ class ThreeBodyLike(nn.Module):
         C = self.config.channels
 
         def build():
-            out = {"w3t": [], "w2_je_t": [], "w2_i": [], "w3_vjp": [], "w2_nodes": [], "w2_eps": []}
-            for layer in self.layers:
-                W3, W2 = layer.W3.detach(), layer.W2.detach()
-                out["w3t"].append(W3[:3 * C].t().contiguous())  # [C, 3C] (N, K): the triplet GEMM
-                # the edge GEMM on [h_j | eps_e] ([C, 2C] (N, K)); the centre block h_i W2b per atom
-                out["w2_je_t"].append(torch.cat([W2[:C], W2[2 * C:]], 0).t().contiguous())
-                out["w2_i"].append(W2[C:2 * C].contiguous())  # [C, C] ([K, N])
-                out["w3_vjp"].append(W3[:3 * C].contiguous())  # [3C, C] (N, K): gz3 [W3a; W3b; W3c]^T
-                out["w2_nodes"].append(torch.cat([W2[:C], W2[C:2 * C]], 1).contiguous())  # [C, 2C] VJP
-                out["w2_eps"].append(W2[2 * C:].contiguous())  # [C, C] VJP
-            out["w3d"] = torch.cat([layer.W3.detach()[3 * C:] for layer in self.layers], 1).contiguous()  # [A, L C]
-            # the VJP group's weights as bf16 planes (its split-plane form; K = 2C and C)
-            out["w2_nodes_planes"] = [split_planes(w) for w in out["w2_nodes"]]
-            out["w2_eps_planes"] = [split_planes(w) for w in out["w2_eps"]]
+            W3 = [layer.W3.detach() for layer in self.layers]
+            W2 = [layer.W2.detach() for layer in self.layers]
+            We = self.We.detach().double()
+            last = len(W3) - 1
+            out = {"node": [], "bond": [], "node_vjp": [], "bond_vjp": [], "rt": []}
+            for t in range(last + 1):
+                w3a, w3b, w3c = W3[t][:C], W3[t][C:2 * C], W3[t][2 * C:3 * C]
+                w2a, w2b, w2c = W2[t][:C], W2[t][C:2 * C], W2[t][2 * C:]
+                following = [] if t == last else [W3[t + 1][:C], W3[t + 1][C:2 * C]]
+                # (N, K) layouts. Forward: h [W3c | W2a | W2b], eps [W2c | W3a' | W3b']
+                out["node"].append(torch.cat([w3c, w2a, w2b], 1).t().contiguous())
+                out["bond"].append(torch.cat([w2c, *following], 1).t().contiguous())
+                # VJP: [S_src | S_dst | S_tri] [W2a; W2b; W3c]^T, [gz2 | gU' | gV'] [W2c; W3a'; W3b']^T
+                out["node_vjp"].append(torch.cat([w2a, w2b, w3c], 1).contiguous())
+                out["bond_vjp"].append(torch.cat([w2c, *following], 1).contiguous())
+                out["rt"].append((We @ w2c.double()).float().contiguous())  # [nb, C]
+            first = W3[0][:2 * C].double()
+            # ef [We | We W3a | We W3b]: the bond rows' first eps, U and V; [gU | gV] [W3a; W3b]^T at the end
+            out["init"] = torch.cat([We, We @ first[:C], We @ first[C:]], 1).float().contiguous()  # [nb, 3C]
+            out["init_vjp"] = torch.cat([W3[0][:C], W3[0][C:2 * C]], 1).contiguous()  # [C, 2C]
+            out["w3d"] = torch.cat([w[3 * C:] for w in W3], 1).contiguous()  # [A, L C]
+            # the node products' weights as bf16 planes (their split-plane form)
+            out["node_planes"] = [split_planes(w) for w in out["node"]]
+            out["node_vjp_planes"] = [split_planes(w) for w in out["node_vjp"]]
             return out
 
         return self._cached("layouts", build)
@@ -193,24 +210,27 @@ def _forward(ctx, positions: Tensor, cell: Tensor, model: ThreeBodyLike, inputs:
     aw = gemm(alpha, lay["w3d"], b_layout=1)  # [T, L C]
     h = _empty(n, C, device=dev)
     _call("fmd_embed_f32", inputs.elem.data_ptr(), model.embedding.data_ptr(), n, C, h.data_ptr())
-    eps = gemm(ef, model.We, b_layout=1)  # [E, C]
-    line = lg.line_graph
-    row1, row2, atom = line[:, 2], line[:, 4], line[:, 0]
     inv_ang, inv_avg = 1.0 / cfg.avg_num_angles, 1.0 / cfg.avg_num_neighbors
+    lines = lg.short_offsets.data_ptr(), lg.bond_rows.data_ptr()
+    # per bond row [eps | eps W2c | U | V] (the other rows are never touched), per atom [H | P | Q]
+    x = _empty(e_cap, 4 * C, device=dev)
+    x_eps, x_c, x_u, x_v = (x[:, k * C:].data_ptr() for k in range(4))
+    hpq = _empty(n, 3 * C, device=dev)
+    _call("fmd_tb_bond_init_f32", ef.data_ptr(), nb, lay["init"].data_ptr(), C, *lines, lg.n_atoms, e_cap, x_eps, 4 * C)
     saved = []
     for t in range(L):
-        # three-body update of the bonds: gather-cat [eps_b1 | eps_b2 | h_i] fused into the GEMM's
-        # load, the angle block added per row
-        z3 = gemm_gather([(eps, row1), (eps, row2), (h, atom)], lay["w3t"][t], row_add=(aw[:, t * C:(t + 1) * C], None))
-        _call("fmd_tb_bond_sum_f32", z3.data_ptr(), C, C, geo.data_ptr(), lg.short_offsets.data_ptr(),
-              lg.bond_rows.data_ptr(), lg.edge_triplet_offsets.data_ptr(), lg.line_graph.data_ptr(), lg.n_atoms,
-              t_cap, inv_ang, eps.data_ptr(), C)
-        # atom update: [h_j | eps_e] gathered into the GEMM's load, the centre block h_i W2b formed
-        # once per atom and added per row
-        q2 = gemm(h, lay["w2_i"][t], b_layout=1)
-        z2 = gemm_gather([(h, ei[:, 1]), (eps, None)], lay["w2_je_t"][t], row_add=(q2, ei[:, 0]))
-        _call("fmd_tb_gated_sum_f32", z2.data_ptr(), C, e_cap, C, geo[:, 4:].data_ptr(), 8, None, None, 0,
-              off.data_ptr(), n, inv_avg, h.data_ptr(), C, 1)
+        gemm_group([{"a": h, "b": lay["node"][t], "b_planes": lay["node_planes"][t], "out": hpq}], b_layout=0)
+        z3 = _empty(t_cap, C, device=dev)
+        _call("fmd_tb_bond_update_f32", x_u, x_v, 4 * C, hpq.data_ptr(), 3 * C, aw[:, t * C:].data_ptr(), L * C, C,
+              geo.data_ptr(), *lines, lg.edge_triplet_offsets.data_ptr(), lg.line_graph.data_ptr(), lg.n_atoms, t_cap,
+              inv_ang, z3.data_ptr(), C, x_eps, 4 * C)
+        bond = lay["bond"][t]
+        _call("fmd_tb_bond_product_f32", x_eps, 4 * C, C, None, 0, C, bond.data_ptr(), C, bond.shape[0], *lines,
+              lg.n_atoms, e_cap, x_c, 4 * C, 0)
+        z2 = _empty(e_cap, C, device=dev)
+        _call("fmd_tb_edge_sum_f32", hpq[:, C:].data_ptr(), 3 * C, ei.data_ptr(), ef.data_ptr(), nb,
+              lay["rt"][t].data_ptr(), C, geo.data_ptr(), lg.short_flags.data_ptr(), x_c, 4 * C, off.data_ptr(), n,
+              e_cap, inv_avg, z2.data_ptr(), h.data_ptr(), C)
         saved.append((z3, z2))
     energy = _empty(n, device=dev)
     _call("fmd_tb_readout_f32", h.data_ptr(), C, C, model.wr.data_ptr(), inputs.elem.data_ptr(), model.e0.data_ptr(),
@@ -237,47 +257,48 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
 
     gh = _empty(n, C, device=dev)
     _call("fmd_tb_readout_bwd_f32", _abi.ptr(gE), 1.0, model.wr.data_ptr(), C, n, gh.data_ptr(), C)
-    # stored by the first layer the loop takes (the last), added to by the others: no zero fills
+    # bond rows only; stored by the first layer the loop takes (the last), added to by the others
     geps = _empty(e_cap, C, device=dev)
+    guv = _empty(e_cap, 2 * C, device=dev)  # [gU | gV], bond rows only
+    gef = _empty(e_cap, nb, device=dev)
     gfc = _empty(e_cap, device=dev)
     gs = _empty(e_cap, device=dev)  # written on the bond rows only (read there only)
     gz3_all = _empty(t_cap, L * C, device=dev)
     gz2 = _empty(e_cap, C, device=dev)
-    s_dst = _empty(n, C, device=dev)
+    sums = _empty(n, 3 * C, device=dev)  # [S_src | S_dst | S_tri]
     gsw = _empty(t_cap, 2, device=dev)
     per_atom = Csr(lg.pair_offsets, None, t_cap)
+    lines = lg.short_offsets.data_ptr(), lg.bond_rows.data_ptr()
+
+    def bond_product(a0, k0, a1, weight, accumulate):
+        _call("fmd_tb_bond_product_f32", a0.data_ptr(), k0, k0, _abi.ptr(a1), 2 * C, weight.shape[1],
+              weight.data_ptr(), weight.shape[1], C, *lines, n, e_cap, geps.data_ptr(), C, accumulate)
+
     for t in reversed(range(L)):
         z3, z2 = ctx.saved[t]
-        first = t == L - 1
-        # atom update: gz2 and its per-centre sums; the cutoff's gradient accumulates over layers
-        _call("fmd_tb_gated_sum_bwd_f32", gh.data_ptr(), C, z2.data_ptr(), C, e_cap, C, geo[:, 4:].data_ptr(), 8, None,
-              None, 0, off.data_ptr(), n, inv_avg, gz2.data_ptr(), C, s_dst.data_ptr(), C, gfc.data_ptr(), 1,
-              0 if first else 1)
-        s_src = segment_sum_csr([(gz2, inputs.csr_src, 0, 1.0, None)], n, C)
-        # gh += [S_src | S_dst] [W2a; W2b]^T and geps += gz2 W2c^T in one launch
-        # (the split-plane form of the group, weights split once: 0.91 -> 0.86 ms/step at 5 000
-        # atoms against the fp32 MFMA tiles)
-        gemm_group([{"a": s_src, "a2": s_dst, "b": lay["w2_nodes"][t], "b_planes": lay["w2_nodes_planes"][t],
-                     "out": gh, "accumulate": True},
-                    {"a": gz2, "b": lay["w2_eps"][t], "b_planes": lay["w2_eps_planes"][t], "out": geps,
-                     "accumulate": not first}], b_layout=0)
-        # three-body update: gz3 per triplet (this layer's column block) and its envelope terms,
-        # ga3 = gz3 [W3a; W3b; W3c]^T on the triplet rows, then per bond the sums of its triplets as
-        # first and second bond into geps (and gs), per atom those of its triplets into gh
+        later = 0 if t == L - 1 else 1
+        _call("fmd_tb_edge_sum_bwd_f32", gh.data_ptr(), C, z2.data_ptr(), nb, lay["rt"][t].data_ptr(), C,
+              geo.data_ptr(), off.data_ptr(), n, e_cap, inv_avg, gz2.data_ptr(), sums[:, C:].data_ptr(), 3 * C,
+              gfc.data_ptr(), gef.data_ptr(), later)
+        segment_sum_csr([(gz2, inputs.csr_src, 0, 1.0, None)], n, C, out=sums[:, :C])
+        bond_product(gz2, C, guv if later else None, lay["bond_vjp"][t], later)
+        # gz3 per triplet (this layer's column block) and its envelope terms
         gz3 = gz3_all[:, t * C:(t + 1) * C]
         _call("fmd_tb_triplet_bwd_f32", geps.data_ptr(), C, z3.data_ptr(), C, C, geo.data_ptr(),
               lg.line_graph.data_ptr(), lg.pair_offsets.data_ptr(), n, t_cap, inv_ang, gz3.data_ptr(), L * C,
               gsw.data_ptr())
-        ga3 = gemm(gz3, lay["w3_vjp"][t], b_layout=0)  # [T, 3C]
-        _call("fmd_tb_bond_reduce_f32", ga3.data_ptr(), 3 * C, C, gsw.data_ptr(), lg.short_offsets.data_ptr(),
-              lg.bond_rows.data_ptr(), lg.edge_triplet_offsets.data_ptr(), lg.second_perm.data_ptr(), n, t_cap,
-              geps.data_ptr(), C, gs.data_ptr(), 0 if first else 1)
-        segment_sum_csr([(ga3, per_atom, 2 * C, 1.0, None)], n, C, out=gh, accumulate=True)
+        _call("fmd_tb_bond_gradient_f32", gz3.data_ptr(), L * C, C, gsw.data_ptr(), *lines,
+              lg.edge_triplet_offsets.data_ptr(), lg.second_perm.data_ptr(), n, t_cap, guv.data_ptr(), 2 * C,
+              gs.data_ptr(), later)
+        segment_sum_csr([(gz3, per_atom, 0, 1.0, None)], n, C, out=sums[:, 2 * C:])
+        gemm_group([{"a": sums, "b": lay["node_vjp"][t], "b_planes": lay["node_vjp_planes"][t], "out": gh,
+                     "accumulate": True}], b_layout=0)
+    bond_product(guv, 2 * C, None, lay["init_vjp"], 1)
+    _call("fmd_tb_bond_basis_f32", geps.data_ptr(), C, C, model.We.data_ptr(), nb, *lines, n, e_cap, gef.data_ptr())
     # the angle basis: all layers' angle gradients at once, then the Fourier VJP (short rows)
     galpha = gemm(gz3_all, lay["w3d"], b_layout=0)  # [T, A]
     gu = _empty(e_cap, 3, device=dev)  # written on the bond rows only (read there only)
     fourier_line_vjp(galpha, geo[:, :3], lg, model.freqs, model.fourier_scale, out=gu, accumulate=False)
-    gef = gemm(geps, model.We, b_layout=0)  # [E, nb]
     gvec = _empty(e_cap, 3, device=dev)
     _call("fmd_tb_geometry_bwd_f32", geo.data_ptr(), ctx.de.data_ptr(), nb, gef.data_ptr(), nb, gu.data_ptr(), 3,
           gfc.data_ptr(), gs.data_ptr(), lg.short_flags.data_ptr(), batch.n_edges.data_ptr(), e_cap, gvec.data_ptr())

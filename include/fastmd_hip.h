@@ -296,6 +296,47 @@ int fmd_tb_bond_reduce_f32(const float* ga3, int64_t lda, int32_t channels, cons
                            const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
                            const int32_t* second_perm, int64_t n_atoms, int64_t t_cap, float* geps, int64_t ldg,
                            float* gs, int32_t accumulate_gs, hipStream_t stream);
+/* fmd_tb_bond_sum_f32 with the pre-activation formed and stored on the way: z3[k] = u[b1] + v[b2] +
+ * h[atom] + aw[k] over the real triplets (b1, b2, atom of line_graph; u, v rows of stride ldu). */
+int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const float* h, int64_t ldh, const float* aw,
+                           int64_t lda, int32_t channels, const float* geo, const int64_t* short_offsets,
+                           const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
+                           int64_t n_atoms, int64_t t_cap, float scale, float* z3, int64_t ldz, float* eps, int64_t lde,
+                           hipStream_t stream);
+/* The sums of fmd_tb_bond_reduce_f32 of gz3 [t_cap, C] itself, kept apart: guv[b] = (sum as first bond
+ * | sum as second bond) [., 2 C], stored on every bond row; gs as there. */
+int fmd_tb_bond_gradient_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
+                             const int64_t* short_offsets, const int32_t* bond_rows,
+                             const int64_t* edge_triplet_offsets, const int32_t* second_perm, int64_t n_atoms,
+                             int64_t t_cap, float* guv, int64_t ldg, float* gs, int32_t accumulate_gs,
+                             hipStream_t stream);
+/* Products on the bond rows e = bond_rows[0, short_offsets[n]) alone (the count read on the device): c[e,
+ * 0:n] (+)= [a0[e, 0:k0] | a1[e, 0:k-k0]] b^T, b [n, k] K-contiguous. k0, k multiples of 32, n of 64, operands 16-byte
+ * aligned with strides of 4. */
+int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const float* a1, int64_t ld1, int32_t k,
+                            const float* b, int64_t ldb, int32_t n, const int64_t* short_offsets,
+                            const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap, float* c, int64_t ldc,
+                            int32_t accumulate, hipStream_t stream);
+/* out[e] = ef[e] m per bond row, m [n_basis, 3 C] in blocks stored at columns 0, 2 C and 3 C. */
+int fmd_tb_bond_init_f32(const float* ef, int32_t n_basis, const float* m, int32_t channels,
+                         const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
+                         float* out, int64_t ldo, hipStream_t stream);
+/* gef[e, n] = sum_c geps[e, c] we[n, c] per bond row (the other rows are left). */
+int fmd_tb_bond_basis_f32(const float* geps, int64_t ldg, int32_t channels, const float* we, int32_t n_basis,
+                          const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
+                          float* gef, hipStream_t stream);
+/* The edge -> atom update: z2[e] = pq[j, 0:C] + pq[i, C:2C] + (short_flags[e] ? bond_part[e] : ef[e] rt) with
+ * (i, j) of edge_index and rt [n_basis, C], stored; h[i] += scale * sum over i's rows of silu(z2) fc (geo column 4). */
+int fmd_tb_edge_sum_f32(const float* pq, int64_t ldp, const int32_t* edge_index, const float* ef, int32_t n_basis,
+                        const float* rt, int32_t channels, const float* geo, const uint8_t* short_flags,
+                        const float* bond_part, int64_t ldx, const int64_t* offsets, int64_t n_atoms, int64_t e_cap,
+                        float scale, float* z2, float* h, int64_t ldh, hipStream_t stream);
+/* Its VJP: gz2[e] = scale gh[i] fc silu'(z2[e]), gsum[i] = sum over i's rows of gz2, gfc[e] (+)= sum_c scale gh[i]
+ * silu(z2[e]), gef[e, n] (+)= sum_c gz2[e, c] rt[n, c] (with accumulate added). Rows of no atom are left. */
+int fmd_tb_edge_sum_bwd_f32(const float* gh, int64_t ldg, const float* z2, int32_t n_basis, const float* rt,
+                            int32_t channels, const float* geo, const int64_t* offsets, int64_t n_atoms, int64_t e_cap,
+                            float scale, float* gz2, float* gsum, int64_t ldgs, float* gfc, float* gef,
+                            int32_t accumulate, hipStream_t stream);
 /* energy[i] = e0[elem[i]] + h[i] . wr, and its VJP gh[i] = (gE ? gE[i] : sign) * wr. */
 int fmd_tb_readout_f32(const float* h, int64_t ldh, int32_t channels, const float* wr, const int32_t* elem,
                        const float* e0, int64_t n, float* energy, hipStream_t stream);

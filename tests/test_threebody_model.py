@@ -265,3 +265,63 @@ def test_gated_segment_sum_and_vjp(device, two_index, C, max_run):
     if two_index:
         gw_total.index_add_(0, idx[:used, 2].long(), gw[:used, 1].cpu().double())
     assert torch.allclose(gw_total, w64.grad, atol=1e-3, rtol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels,n_basis,layers,n_cells", [(64, 5, 1, 2), (64, 16, 2, 3), (128, 20, 2, 2),
+                                                             (256, 9, 3, 2)])
+def test_threebody_gpu_basis_sizes_match_oracle(device, channels, n_basis, layers, n_cells):
+    """Basis sizes on both sides of the eight the edge kernels keep in registers, one layer (no later
+    layer's blocks in the bond products) to three: the bounds of the parity tests above."""
+    from fastmd_amd.engine.energy_derivative import EnergyDerivative
+    from fastmd_amd.models.threebody_like import ThreeBodyAdapter, ThreeBodyConfig, ThreeBodyLike
+
+    print(f"[threebody] channels={channels} basis={n_basis} layers={layers}", flush=True)
+    s = systems.perovskite(n_cells, sigma=0.2)
+    n = s.n_atoms
+    config = ThreeBodyConfig(channels=channels, n_basis=n_basis, num_interactions=layers, bond_cutoff=3.5)
+    m = ThreeBodyLike(config)
+    params, cfg = {k: v.detach().clone() for k, v in m.named_parameters()}, dataclasses.asdict(config)
+    adapter = ThreeBodyAdapter(m, device=device)
+    builder = _builder(s, 3.5, device)
+    builder.build(torch.tensor(s.positions, device=device))
+    out = EnergyDerivative(adapter)(builder.batch, adapter.prepare(builder.batch), n_real=n)
+    torch.cuda.synchronize()
+    edges = _edges(s)
+    bonds = torch.nonzero(builder.short_flags[:len(edges[0])].cpu().bool()).flatten()
+    e_ref, f_ref, _ = om.energy_and_forces(_fn(params, cfg, s, edges, bond_rows=bonds), edges[3])
+    assert abs(float(out["e"].item()) - float(e_ref)) / n < 1e-5
+    assert float((out["f"][0].cpu().double() - f_ref).abs().max()) < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,k0,k1,n,accumulate", [(0, 64, 0, 64, 0), (1, 64, 0, 192, 0), (16, 64, 128, 64, 1),
+                                                      (17, 128, 256, 128, 0), (333, 32, 0, 64, 1),
+                                                      (70000, 64, 0, 64, 1)])
+def test_bond_product_rows(device, count, k0, k1, n, accumulate):
+    """fmd_tb_bond_product_f32 on `count` listed rows of a strided array, in random order: the product against
+    float64 within k rounding errors of float32 times the sum of magnitudes, every other row and column
+    as it was. Counts around the 16-row tile and past one pass of the grid."""
+    from fastmd_amd import _abi
+
+    gen = torch.Generator().manual_seed(count + n)
+    rows, k = count + 40, k0 + k1
+    a0, a1 = torch.randn(rows, k0 + 4, generator=gen), torch.randn(rows, max(k1, 4), generator=gen)
+    b = torch.randn(n, k, generator=gen)
+    c = torch.randn(rows, n + 3, generator=gen)
+    listed = torch.randperm(rows, generator=gen)[:count]
+    offsets = torch.tensor([0, count // 2, count])
+    d = lambda t: t.to(device)  # noqa: E731
+    pad = torch.zeros(8, dtype=torch.int32)
+    a0d, a1d, bd, cd, rd, od = d(a0), d(a1), d(b), d(c), d(torch.cat([listed.int(), pad])), d(offsets)
+    _abi.call("fmd_tb_bond_product_f32", a0d.data_ptr(), k0 + 4, k0, a1d.data_ptr(), max(k1, 4), k, bd.data_ptr(), k, n,
+              od.data_ptr(), rd.data_ptr(), 2, rows, cd.data_ptr(), n + 3, accumulate, _abi.stream_handle())
+    torch.cuda.synchronize()
+    got = cd.cpu()
+    a = torch.cat([a0[:, :k0], a1[:, :k1]], 1).double()[listed]
+    want = a @ b.double().t() + (c[listed, :n].double() if accumulate else 0.0)
+    bound = 2 ** -23 * (k + 1) * (a.abs() @ b.abs().double().t() + c[listed, :n].abs())
+    assert bool(((got[listed, :n].double() - want).abs() <= bound).all())
+    left = torch.ones(rows, dtype=torch.bool)
+    left[listed] = False
+    assert torch.equal(got[left], c[left]) and torch.equal(got[:, n:], c[:, n:])
