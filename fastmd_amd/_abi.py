@@ -197,7 +197,13 @@ def ptr(tensor) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    """torch's current HIP stream (the stream every entry point launches on)."""
+    """torch's current HIP stream (the stream every entry point launches on). Without a device, and with
+    torch's GPU state up in this process, its raw handle: 0.15 us, where the stream object, made for every
+    launch, takes 2.7 in a loop and 20 between other work (with the pooled flags of the index checks:
+    gather-cat and its VJP at 160 000 rows 222 -> 150 us, the Fourier basis and its VJP 213 -> 115, a
+    135-atom block 419 -> 260)."""
+    if device is None and torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return torch.cuda.current_stream(device).cuda_stream
 
 

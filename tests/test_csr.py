@@ -65,3 +65,34 @@ def test_negative_segments_are_refused(rows):
         csr_segment_sum(value, index, 50)
     with pytest.raises(RuntimeError):
         weighted_segment_sum(value, value, index, 50)
+
+
+@pytest.mark.gpu
+def test_negative_flags_are_cleared_between_calls_and_threads():
+    """The pooled flags of a refused index do not reach a later check, also with checks of several threads
+    and streams open at a time: each reports its own index."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from fastmd_amd.ops.csr_segment_sum import _NegativeCheck, csr_from_segments, refuse_negative
+
+    def one(k):
+        bad = k % 3 == 0
+        with torch.cuda.stream(torch.cuda.Stream()):
+            seg = torch.full((500 + k,), 4, dtype=torch.int32, device="cuda")
+            seg[k % 500] = -1 if bad else 2
+            for _ in range(3):
+                open_checks = [csr_from_segments([(seg, 9)])[1] for _ in range(3)]
+                for check in open_checks:
+                    if bad:
+                        with pytest.raises(RuntimeError, match="non-negative"):
+                            refuse_negative(check)
+                    else:
+                        refuse_negative(check)
+        return bad
+
+    one(0)
+    one(1)
+    with ThreadPoolExecutor(8) as pool:
+        assert list(pool.map(one, range(24))) == [k % 3 == 0 for k in range(24)]
+    assert all(len(idle) <= _NegativeCheck._KEPT and not any(any(f.tolist()) for f, _ in idle)
+               for idle in _NegativeCheck._idle.values())
