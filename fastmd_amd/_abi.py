@@ -31,6 +31,8 @@ SIGNATURES: dict[str, tuple] = {
                                          _i64, _p]),
     "fmd_nl_candidates_pad": (ctypes.c_int, [_p, _p, _p, _i64, _f32, _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64,
                                              _i64, _i32, _p]),
+    "fmd_host_report": (ctypes.c_int, [_i32, _p, _p, _p, _p, _p, _p, _i64, _p, _p]),
+    "fmd_count_demand": (ctypes.c_int, [_p, _i64, _i32, _p, _p]),
     "fmd_nl_atom_order": (ctypes.c_int, [_p, _i64, _p, _p, _p]),
     "fmd_nl_wrap": (ctypes.c_int, [_p, _i32, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "fmd_nl_build_work_size": (_i64, [_i64]),
@@ -197,13 +199,16 @@ def ptr(tensor) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    """torch's current HIP stream (the stream every entry point launches on). Without a device, and with
-    torch's GPU state up in this process, its raw handle: 0.15 us, where the stream object, made for every
+    """torch's current HIP stream (the stream every entry point launches on). For the current or an
+    indexed device, and with torch's GPU state up in this process, its raw handle: 0.15 us, where the stream object, made for every
     launch, takes 2.7 in a loop and 20 between other work (with the pooled flags of the index checks:
     gather-cat and its VJP at 160 000 rows 222 -> 150 us, the Fourier basis and its VJP 213 -> 115, a
     135-atom block 419 -> 260)."""
-    if device is None and torch.cuda.is_initialized():
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if torch.cuda.is_initialized():
+        if device is None:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+            return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

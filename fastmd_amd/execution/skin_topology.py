@@ -28,12 +28,13 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from fastmd_amd import _abi
 from fastmd_amd._roctx import roctx_range
 from fastmd_amd.adapters.protocol import PaddingRule
 from fastmd_amd.engine.capacity_policy import held_demand, tier
 from fastmd_amd.engine.energy_derivative import engine_derivative
 from fastmd_amd.execution.graph_capture import capture_graph
-from fastmd_amd.graph.fixed_capacity_builder import FixedCapacityGraphBuilder, fixed_capacity_exceeded
+from fastmd_amd.graph.fixed_capacity_builder import FixedCapacityGraphBuilder, counts_exceed
 
 # The host refreshes the candidates before the launch once an atom moved this fraction of the skin
 # (0.9 of the device's limit of half the skin: the margin covers the host's float64 vs the
@@ -129,12 +130,16 @@ class SkinTopologyRunner:
     def _body(self, builder: FixedCapacityGraphBuilder):
         graph, status = builder.build(self.positions, rebuild_candidates=False)
         out = self._derivative(builder.batch, graph, task="ef", n_real=self.n_real)
-        flags = torch.cat([status.candidate_valid.reshape(1).long(),
-                           builder._candidate_capacity_valid.reshape(1).long(),
-                           fixed_capacity_exceeded(status, builder).reshape(1).long(),
-                           status.edge_count.reshape(1).long(), status.triplet_count.reshape(1).long(),
-                           status.isolated_atom_count.reshape(1).long()])
-        return out, flags
+        # the status, the float64 energy and the real rows' forces, into the pinned memory _read takes
+        energy = out["e"].reshape(-1)[:1].to(torch.float64)
+        forces = out["f"][0][: self.n_real].to(torch.float32).contiguous()
+        scalars = (status.candidate_valid, builder._candidate_capacity_valid, status.invalid_pairs,
+                   status.edge_count, status.triplet_count, status.isolated_atom_count)
+        _abi.call("fmd_host_report", len(scalars), _abi.ptr_array([s.data_ptr() for s in scalars]),
+                  _abi.array(_abi._i32, [s.element_size() for s in scalars]), self._pinned_flags.data_ptr(),
+                  energy.data_ptr(), self._pinned_energy.data_ptr(), forces.data_ptr(), forces.numel(),
+                  self._pinned_forces.data_ptr(), _abi.stream_handle())
+        return out
 
     def _make_bucket(self, key) -> dict:
         u_cap, t_cap = key
@@ -143,7 +148,7 @@ class SkinTopologyRunner:
             kwargs.update(line_graph_cutoff=self.triplet_cutoff, t_capacity=t_cap)
         builder = FixedCapacityGraphBuilder(u_capacity=u_cap, candidates_from=self.owner,
                                             prepare=self.adapter.prepare, **kwargs)
-        entry = {"builder": builder, "graph": None, "out": None, "flags": None}
+        entry = {"builder": builder, "graph": None, "out": None}
         if self.capture:
             side = torch.cuda.Stream(device=self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
@@ -154,8 +159,8 @@ class SkinTopologyRunner:
             torch.cuda.synchronize(self.device)
             graph = torch.cuda.CUDAGraph()
             with capture_graph(graph, pool=self.pool, name="skin_topology_capture"):
-                out, flags = self._body(builder)
-            entry.update(graph=graph, out=out, flags=flags)
+                out = self._body(builder)
+            entry.update(graph=graph, out=out)
             self.captures += 1
         self.buckets[key] = entry
         return entry
@@ -193,19 +198,17 @@ class SkinTopologyRunner:
         self._demand = ((edges + 1) // 2, t)
         self.refreshes += 1
 
-    def _launch(self, entry):
-        if entry["graph"] is not None:
-            entry["graph"].replay()
-            return entry["out"], entry["flags"]
-        return self._body(entry["builder"])
-
     @torch.no_grad()
-    def _read(self, out, flags):
-        """One readback: the status vector, the float64 energy and the real rows' forces."""
-        self._pinned_flags.copy_(flags, non_blocking=True)
-        self._pinned_energy.copy_(out["e"].reshape(-1)[:1].to(torch.float64), non_blocking=True)
-        self._pinned_forces.copy_(out["f"][0][: self.n_real], non_blocking=True)
-        torch.cuda.current_stream(self.device).synchronize()
+    def _read(self, entry):
+        """One evaluation and its readback: the status, the float64 energy and the real rows' forces, written
+        by the evaluation's last kernel (waited for in any case: nothing writes the pinned memory later)."""
+        try:
+            if entry["graph"] is not None:
+                entry["graph"].replay()
+            else:
+                self._body(entry["builder"])
+        finally:
+            torch.cuda.current_stream(self.device).synchronize()
         return self._pinned_flags.tolist(), {"e": float(self._pinned_energy[0]),
                                              "f": self._pinned_forces.numpy().copy()}
 
@@ -227,8 +230,9 @@ class SkinTopologyRunner:
                     self._refresh(positions)
             for _ in range(MAX_ATTEMPTS):
                 entry = self._bucket(*self._demand)
-                flags, result = self._read(*self._launch(entry))
-                candidates_valid, capacity_valid, exceeded, edges, triplets, isolated = flags
+                flags, result = self._read(entry)
+                candidates_valid, capacity_valid, invalid, edges, triplets, isolated = flags
+                exceeded = counts_exceed(entry["builder"], edges, triplets, bool(invalid))
                 if not capacity_valid:
                     raise SkinTopologyUnavailable(f"a candidate row exceeds {self.owner.buffer_max} slots")
                 if not candidates_valid:

@@ -55,10 +55,14 @@ def fixed_capacity_exceeded(status, builder) -> Tensor:
     """Device predicate: the real graph does not fit (fixed_capacity_builder.py:796-814). An
     edges-only builder fits up to ``e_capacity`` inclusive; with a line graph, equality is an
     overflow too."""
+    return counts_exceed(builder, status.edge_count[0], status.triplet_count[0], status.invalid_pairs[0])
+
+
+def counts_exceed(builder, edges, triplets, invalid):
+    """``fixed_capacity_exceeded`` of a build's counts, device scalars or host values."""
     if getattr(builder, "edges_only", False):
-        return (status.edge_count[0] > builder.e_capacity) | status.invalid_pairs[0]
-    return ((status.edge_count[0] >= builder.e_capacity) | (status.triplet_count[0] > builder.t_capacity)
-            | status.invalid_pairs[0])
+        return (edges > builder.e_capacity) | invalid
+    return (edges >= builder.e_capacity) | (triplets > builder.t_capacity) | invalid
 
 
 def self_loop_padding(padding: PaddingRule, cell: Tensor, cutoff: float):

@@ -90,6 +90,15 @@ class TensorGraphBuilder:
         self._cell_start = torch.zeros(ncell + 1, dtype=torch.int32, device=dev)
         self._cell_atoms = torch.zeros(n, dtype=torch.int32, device=dev)
 
+    def _read_back(self, launch) -> list[int]:
+        """The two numbers that ``launch(address)`` writes into pinned memory of this call."""
+        read = torch.empty(2, dtype=torch.int64, pin_memory=True)
+        try:
+            launch(read.data_ptr())
+        finally:  # nothing writes the memory once it is given back
+            torch.cuda.current_stream(self.device).synchronize()
+        return read.tolist()
+
     @torch.no_grad()
     @roctx_ranged("neighbor_list")
     def build(self, positions: Tensor) -> GraphBatch:
@@ -125,7 +134,8 @@ class TensorGraphBuilder:
                       _abi.array(_abi._i32, self._ncells), _abi.array(_abi._i32, self._reach), bmax,
                       self._cell_count.data_ptr(), self._cell_start.data_ptr(), self._cell_atoms.data_ptr(),
                       nm.data_ptr(), ns.data_ptr(), num.data_ptr(), valid.data_ptr(), 0, 0, _abi.NL_PAD_NONE, stream)
-            max_count, total = torch.stack([num.max().long(), num.clamp(max=bmax).long().sum()]).tolist()
+            max_count, total = self._read_back(
+                lambda read: _abi.call("fmd_count_demand", num.data_ptr(), n, bmax, read, stream))
             if max_count <= bmax:
                 break
             self.max_neighbors = grown_max_neighbors(bmax, max_count)
@@ -153,7 +163,10 @@ class TensorGraphBuilder:
                   edge_index.data_ptr(), edge_image.data_ptr(), max_disp.data_ptr(), cand_valid.data_ptr(),
                   overflow.data_ptr(), isolated.data_ptr(), 0.0, None, None, None, None, None, None, None, 0,
                   stream)
-        edges, iso = torch.stack([offsets[-1], isolated[0].long()]).tolist()
+        scalars = _abi.ptr_array([offsets.data_ptr() + 8 * n, isolated.data_ptr()])
+        edges, iso = self._read_back(
+            lambda read: _abi.call("fmd_host_report", 2, scalars, _abi.array(_abi._i32, [8, 4]), read, None, None, None,
+                                   0, None, stream))
         if self.check_isolated_atoms:
             raise_if_isolated_atoms(iso)
         reverse = torch.empty(max(edges, 1), **i32)

@@ -356,6 +356,14 @@ int fmd_tb_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, cons
 int fmd_nl_pad_rows(int32_t* edge_index, float* edge_image, int32_t* edge_reverse, int64_t e_real, int64_t e_cap,
                     int64_t n_atoms, int32_t pad_ix, int32_t pad_iy, int32_t pad_iz, hipStream_t stream);
 
+/* What the host reads after a launch sequence, in one launch: out[k] = the scalar at src[k] (bytes[k] 1 unsigned,
+ * 4 or 8 signed; count <= 8), energy_out = *energy (nullable), values_out[0:n] = values[0:n]. The outputs may be
+ * pinned host memory, complete once the stream has passed. */
+int fmd_host_report(int32_t count, const void* const* src, const int32_t* bytes, int64_t* out, const double* energy,
+                    double* energy_out, const float* values, int64_t n, float* values_out, hipStream_t stream);
+/* out [2] = (max of counts, sum of min(counts, limit)) over n > 0 counts; out as above. */
+int fmd_count_demand(const int32_t* counts, int64_t n, int32_t limit, int64_t* out, hipStream_t stream);
+
 /* Reverse edge of every real row e < min(E, e_cap): the row of (neighbour, centre, -image),
  * or -1 when it is not stored (overflowed build). Gives the sender-side CSR of the sorted
  * edge list (perm = reverse, off = edge_offsets), used by the deterministic VJPs. No
