@@ -535,15 +535,15 @@ __global__ void __launch_bounds__(256) tb_triplet_bwd_kernel(LineCsr lc, const f
 // acc_gs). A second-bond slot of -1 (no triplet) adds zeros. SPLIT: ga3 is [t_cap, C] (the gradient of
 // z3), and its two sums are stored side by side, geps[b, 0:C] (first bond) and geps[b, C:2C] (second).
 template <int NC, bool SPLIT>
-__global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const float* ga3, int64_t lda, int C,
-                                                              const float* gsw, float* geps, int64_t ldg, float* gs,
-                                                              int acc_gs) {
+__device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3, int64_t lda, int C, const float* gsw,
+                                            float* geps, int64_t ldg, float* gs, int acc_gs, int64_t first_wave,
+                                            int64_t nw) {
   constexpr int U = bond_pass<NC>(), TQ = kRunBatch;
   const int64_t second = SPLIT ? 0 : C;  // column of the second bond's block
   const int lane = threadIdx.x & 63;
   const LaneCols<NC> cols(C);
-  const int64_t nb = lc.short_offsets[lc.n], nw = (int64_t)gridDim.x * 4;
-  for (int64_t j0 = wave_id(); j0 < nb; j0 += U * nw) {
+  const int64_t nb = lc.short_offsets[lc.n];
+  for (int64_t j0 = first_wave; j0 < nb; j0 += U * nw) {
     const BondSlots<U> bs(lc, j0, nw, nb);
     const float gs_l = acc_gs ? gs[bs.b] : 0.f;
     float old[U][NC], x[U][2][TQ][NC];
@@ -645,6 +645,88 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
   }
 }
 
+template <int NC>
+__global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const float* ga3, int64_t lda, int C,
+                                                              const float* gsw, float* geps, int64_t ldg, float* gs,
+                                                              int acc_gs) {
+  bond_reduce<NC, false>(lc, ga3, lda, C, gsw, geps, ldg, gs, acc_gs, wave_id(), (int64_t)gridDim.x * 4);
+}
+
+// out[c] = sum over entries [lo, hi) of row perm[k] (null: row k; negative: none) of v, a wave: G groups of C / 4
+// lanes take the entries in turn, U of each group's rows in flight, the groups added in a fixed order.
+template <int NC>
+__device__ __forceinline__ void row_sums(const float* v, int64_t ld, const int32_t* perm, int64_t lo, int64_t hi,
+                                         float* out) {
+  constexpr int LPR = 16 * NC, G = NC == 1 ? 4 : NC == 2 ? 2 : 1, U = NC == 1 ? 5 : 8;
+  const int lane = threadIdx.x & 63, g = G == 1 ? 0 : lane / LPR, c = 4 * (lane - g * LPR);
+  const bool live = lane < G * LPR;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int64_t base = lo; base < hi; base += 64) {
+    const int cnt = hi - base < 64 ? (int)(hi - base) : 64;
+    const int64_t k = base + (lane < cnt ? lane : cnt - 1);
+    const int row = perm ? perm[k] : (int)k;
+    for (int k0 = 0; k0 < cnt; k0 += G * U) {
+      float4 x[U];
+      bool use[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int at = k0 + u * G + g, r = __shfl(row, at < cnt ? at : cnt - 1, 64);
+        use[u] = at < cnt && r >= 0;
+        x[u] = *reinterpret_cast<const float4*>(v + (int64_t)(r >= 0 ? r : 0) * ld + (live ? c : 0));
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        acc.x = use[u] ? acc.x + x[u].x : acc.x;
+        acc.y = use[u] ? acc.y + x[u].y : acc.y;
+        acc.z = use[u] ? acc.z + x[u].z : acc.z;
+        acc.w = use[u] ? acc.w + x[u].w : acc.w;
+      }
+    }
+  }
+#pragma unroll
+  for (int s = LPR; s < LPR * G; s *= 2) {
+    acc.x += __shfl_xor(acc.x, s, 64);
+    acc.y += __shfl_xor(acc.y, s, 64);
+    acc.z += __shfl_xor(acc.z, s, 64);
+    acc.w += __shfl_xor(acc.w, s, 64);
+  }
+  if (live && g == 0) *reinterpret_cast<float4*>(out + c) = acc;
+}
+
+struct NodeSums {
+  const float* gz2;        // [e_cap, C]
+  const int64_t* off;      // [n + 1]
+  const int32_t* reverse;  // [e_cap]: the rows sent by an atom
+  int64_t e_cap;
+  float *src, *tri;        // [n] rows of stride ld
+  int64_t ld;
+};
+
+// The sums that a layer's VJP forms once gz2 and gz3 are there, none of which reads another: per bond [gU | gV] and
+// the envelope terms (the first blocks: the longest chain), per atom the gz2 of the edges that it sends and the gz3
+// of its triplets. One launch instead of three:
+// 13.8 us against 12.5 + 8 + 4.7 at 5 000 atoms and 64 channels (MD step 698 -> 647 us; 375 atoms, 128 channels 470 ->
+// 422).
+template <int NC>
+__global__ void __launch_bounds__(256) tb_vjp_sums_kernel(LineCsr lc, const float* gz3, int64_t ldz, int C,
+                                                           const float* gsw, float* guv, int64_t ldg, float* gs,
+                                                           int acc_gs, const NodeSums ns, int64_t bond_blocks) {
+  if ((int64_t)blockIdx.x < bond_blocks) {
+    bond_reduce<NC, true>(lc, gz3, ldz, C, gsw, guv, ldg, gs, acc_gs, wave_id(), bond_blocks * 4);
+    return;
+  }
+  const int64_t w = wave_id() - bond_blocks * 4, i = w >> 1;
+  if (i >= lc.n) return;
+  int64_t lo, hi;
+  if (w & 1) {
+    run_of(lc.pair_offsets, i, lc.t_cap, lo, hi);
+    row_sums<NC>(gz3, ldz, nullptr, lo, hi, ns.tri + i * ns.ld);
+  } else {
+    run_of(ns.off, i, ns.e_cap, lo, hi);
+    row_sums<NC>(ns.gz2, C, ns.reverse, lo, hi, ns.src + i * ns.ld);
+  }
+}
+
 // ---- the bond rows' products and the edge sums of the node-factored model. An edge row's pre-activation
 // z2 = h_j W2a + h_i W2b + eps_e W2c takes its first two terms from per-atom rows, and eps_e differs from
 // its initial ef_e We on the bond rows alone (a tenth of the edges): the other rows' last term is
@@ -652,7 +734,7 @@ __global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const f
 // bond rows only. No edge-sized product and no triplet-sized one is left (5 000 atoms, 3.5 A: 84 000
 // edges, 10 300 bonds, 26 000 triplets).
 // Against gathering [h_j | eps_e] and [eps_b1 | eps_b2 | h_i] into products over the edge and triplet rows: an MD step
-// of 5 000 atoms at 64 channels 773 -> 698 us, of 375 atoms at 128 channels 767 -> 470, and an evaluation of
+// of 5 000 atoms at 64 channels 773 -> 698 us (647 with the sums below in one launch), of 375 atoms at 128 channels 767 -> 470 (422), and an evaluation of
 // 500 atoms 988 -> 574.
 
 // C[e, 0:N] (+)= [a0[e] | a1[e]] B^T over the real bonds e = bond_rows[k]: a workgroup takes 16 bonds x 64 columns,
@@ -1172,24 +1254,30 @@ int fmd_tb_bond_reduce_f32(const float* ga3, int64_t lda, int32_t channels, cons
   if (n_atoms == 0 || t_cap == 0) return FMD_OK;
   FMD_REQUIRE(ga3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && geps && gs);
   LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC2(tb_bond_reduce_kernel, false, channels, dim3(kStrideBlocks), lc, ga3, lda, channels, gsw, geps, ldg, gs,
-                accumulate_gs);
+  TB_LAUNCH_NC(tb_bond_reduce_kernel, channels, dim3(kStrideBlocks), lc, ga3, lda, channels, gsw, geps, ldg, gs,
+               accumulate_gs);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }
 
-int fmd_tb_bond_gradient_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
-                             const int64_t* short_offsets, const int32_t* bond_rows,
-                             const int64_t* edge_triplet_offsets, const int32_t* second_perm, int64_t n_atoms,
-                             int64_t t_cap, float* guv, int64_t ldg, float* gs, int32_t accumulate_gs,
-                             hipStream_t stream) {
-  FMD_REQUIRE(n_atoms >= 0 && t_cap >= 0 && channels > 0 && channels <= 256 && ldz >= channels);
-  FMD_REQUIRE(ldg >= 2 * (int64_t)channels);
-  if (n_atoms == 0 || t_cap == 0) return FMD_OK;
-  FMD_REQUIRE(gz3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && guv && gs);
-  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC2(tb_bond_reduce_kernel, true, channels, dim3(kStrideBlocks), lc, gz3, ldz, channels, gsw, guv, ldg, gs,
-                accumulate_gs);
+int fmd_tb_vjp_sums_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
+                        const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
+                        const int32_t* second_perm, const int64_t* pair_offsets, int64_t n_atoms, int64_t t_cap,
+                        float* guv, int64_t ldg, float* gs, int32_t accumulate_gs, const float* gz2,
+                        const int64_t* offsets, const int32_t* reverse, int64_t e_cap, float* s_src, float* s_tri,
+                        int64_t lds, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && t_cap > 0 && e_cap >= 0 && channels > 0 && channels <= 256 && channels % 64 == 0);
+  FMD_REQUIRE(ldz >= channels && ldz % 4 == 0 && ldg >= 2 * (int64_t)channels && lds >= channels && lds % 4 == 0);
+  if (n_atoms == 0) return FMD_OK;
+  FMD_REQUIRE(gz3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && pair_offsets && guv && gs);
+  FMD_REQUIRE(offsets && s_src && s_tri && (e_cap == 0 || (gz2 && reverse)));
+  const auto aligned = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  FMD_REQUIRE(aligned(gz3) && aligned(gz2) && aligned(s_src) && aligned(s_tri));
+  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, pair_offsets, n_atoms, t_cap};
+  const NodeSums ns{gz2, offsets, reverse, e_cap, s_src, s_tri, lds};
+  const int64_t bond_blocks = kStrideBlocks;
+  TB_LAUNCH_NC(tb_vjp_sums_kernel, channels, dim3((unsigned)(bond_blocks + fmd_cdiv(2 * n_atoms, 4))), lc, gz3, ldz,
+               channels, gsw, guv, ldg, gs, accumulate_gs, ns, bond_blocks);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

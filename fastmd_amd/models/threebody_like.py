@@ -50,7 +50,7 @@ from torch.autograd import Function
 from fastmd_amd import _abi
 from fastmd_amd.adapters.protocol import (CapacityStep, CaptureContract, GraphBatch, PaddingRule, TopologySpec,
                                          require_atom_rows, system_rows)
-from fastmd_amd.ops.csr_segment_sum import Csr, segment_sum_csr
+from fastmd_amd.ops.csr_segment_sum import Csr, _prep_off, _prep_perm, segment_sum_csr
 from fastmd_amd.ops.threebody import LineGraph, fourier_line_vjp
 from fastmd_amd.ops.wide_gemm import gemm, gemm_group, split_planes
 
@@ -267,8 +267,8 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
     gz2 = _empty(e_cap, C, device=dev)
     sums = _empty(n, 3 * C, device=dev)  # [S_src | S_dst | S_tri]
     gsw = _empty(t_cap, 2, device=dev)
-    per_atom = Csr(lg.pair_offsets, None, t_cap)
     lines = lg.short_offsets.data_ptr(), lg.bond_rows.data_ptr()
+    sent, sent_off = _prep_perm(inputs.csr_src.perm), _prep_off(inputs.csr_src.off)
 
     def bond_product(a0, k0, a1, weight, accumulate):
         _call("fmd_tb_bond_product_f32", a0.data_ptr(), k0, k0, _abi.ptr(a1), 2 * C, weight.shape[1],
@@ -280,17 +280,17 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
         _call("fmd_tb_edge_sum_bwd_f32", gh.data_ptr(), C, z2.data_ptr(), nb, lay["rt"][t].data_ptr(), C,
               geo.data_ptr(), off.data_ptr(), n, e_cap, inv_avg, gz2.data_ptr(), sums[:, C:].data_ptr(), 3 * C,
               gfc.data_ptr(), gef.data_ptr(), later)
-        segment_sum_csr([(gz2, inputs.csr_src, 0, 1.0, None)], n, C, out=sums[:, :C])
         bond_product(gz2, C, guv if later else None, lay["bond_vjp"][t], later)
         # gz3 per triplet (this layer's column block) and its envelope terms
         gz3 = gz3_all[:, t * C:(t + 1) * C]
         _call("fmd_tb_triplet_bwd_f32", geps.data_ptr(), C, z3.data_ptr(), C, C, geo.data_ptr(),
               lg.line_graph.data_ptr(), lg.pair_offsets.data_ptr(), n, t_cap, inv_ang, gz3.data_ptr(), L * C,
               gsw.data_ptr())
-        _call("fmd_tb_bond_gradient_f32", gz3.data_ptr(), L * C, C, gsw.data_ptr(), *lines,
-              lg.edge_triplet_offsets.data_ptr(), lg.second_perm.data_ptr(), n, t_cap, guv.data_ptr(), 2 * C,
-              gs.data_ptr(), later)
-        segment_sum_csr([(gz3, per_atom, 0, 1.0, None)], n, C, out=sums[:, 2 * C:])
+        # per bond gU, gV and the envelope terms, per atom the sent edges' gz2 and the triplets' gz3
+        _call("fmd_tb_vjp_sums_f32", gz3.data_ptr(), L * C, C, gsw.data_ptr(), *lines,
+              lg.edge_triplet_offsets.data_ptr(), lg.second_perm.data_ptr(), lg.pair_offsets.data_ptr(), n, t_cap,
+              guv.data_ptr(), 2 * C, gs.data_ptr(), later, gz2.data_ptr(), sent_off.data_ptr(),
+              sent.data_ptr(), e_cap, sums.data_ptr(), sums[:, 2 * C:].data_ptr(), 3 * C)
         gemm_group([{"a": sums, "b": lay["node_vjp"][t], "b_planes": lay["node_vjp_planes"][t], "out": gh,
                      "accumulate": True}], b_layout=0)
     bond_product(guv, 2 * C, None, lay["init_vjp"], 1)

@@ -303,13 +303,17 @@ int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const fl
                            const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
                            int64_t n_atoms, int64_t t_cap, float scale, float* z3, int64_t ldz, float* eps, int64_t lde,
                            hipStream_t stream);
-/* The sums of fmd_tb_bond_reduce_f32 of gz3 [t_cap, C] itself, kept apart: guv[b] = (sum as first bond
- * | sum as second bond) [., 2 C], stored on every bond row; gs as there. */
-int fmd_tb_bond_gradient_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
-                             const int64_t* short_offsets, const int32_t* bond_rows,
-                             const int64_t* edge_triplet_offsets, const int32_t* second_perm, int64_t n_atoms,
-                             int64_t t_cap, float* guv, int64_t ldg, float* gs, int32_t accumulate_gs,
-                             hipStream_t stream);
+/* The sums of a layer's VJP in one launch. Per bond those of fmd_tb_bond_reduce_f32 of gz3 [t_cap, C] itself,
+ * kept apart: guv[b] = (sum as first bond | sum as second bond) [., 2 C], stored on every bond row; gs as there. Per
+ * atom s_src[i] = sum of gz2 [e_cap, C] over the rows reverse[offsets[i] .. offsets[i + 1]) (negative entries
+ * skipped) and s_tri[i] = sum of gz3 over its triplets. channels a multiple of 64; t_cap > 0; gz3, gz2, s_src,
+ * s_tri 16-byte aligned, strides multiples of 4. */
+int fmd_tb_vjp_sums_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
+                        const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
+                        const int32_t* second_perm, const int64_t* pair_offsets, int64_t n_atoms, int64_t t_cap,
+                        float* guv, int64_t ldg, float* gs, int32_t accumulate_gs, const float* gz2,
+                        const int64_t* offsets, const int32_t* reverse, int64_t e_cap, float* s_src, float* s_tri,
+                        int64_t lds, hipStream_t stream);
 /* Products on the bond rows e = bond_rows[0, short_offsets[n]) alone (the count read on the device): c[e,
  * 0:n] (+)= [a0[e, 0:k0] | a1[e, 0:k-k0]] b^T, b [n, k] K-contiguous. k0, k multiples of 32, n of 64, operands 16-byte
  * aligned with strides of 4. */

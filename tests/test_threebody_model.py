@@ -325,3 +325,67 @@ def test_bond_product_rows(device, count, k0, k1, n, accumulate):
     left = torch.ones(rows, dtype=torch.bool)
     left[listed] = False
     assert torch.equal(got[left], c[left]) and torch.equal(got[:, n:], c[:, n:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels,longest", [(64, 21), (64, 300), (128, 17), (192, 9), (256, 70)])
+def test_vjp_sums(device, channels, longest):
+    """fmd_tb_vjp_sums_f32 on a made-up line graph, with empty runs, runs past one pass and past the 64 entries
+    looked up at a time, missing reverse rows and a run that ends past the capacity: every sum within its
+    number of terms rounding errors of float32 times the sum of magnitudes."""
+    from fastmd_amd import _abi
+
+    gen = torch.Generator().manual_seed(channels + longest)
+    C, n = channels, 37
+    sent = torch.randint(0, longest + 1, (n,), generator=gen)
+    off = torch.cat([torch.zeros(1, dtype=torch.int64), sent.cumsum(0)])
+    e_cap = int(off[-1]) - 2  # the last run is cut
+    reverse = torch.randint(-1, e_cap, (e_cap,), generator=gen, dtype=torch.int32)
+    bonds = torch.randint(0, 5, (n,), generator=gen)  # per atom; every ordered pair of them a triplet
+    short_off = torch.cat([torch.zeros(1, dtype=torch.int64), bonds.cumsum(0)])
+    rows = torch.randperm(e_cap, generator=gen)[:int(short_off[-1])]
+    pair_off = torch.cat([torch.zeros(1, dtype=torch.int64), (bonds * (bonds - 1)).cumsum(0)])
+    t_cap = int(pair_off[-1]) + 9
+    eto, second = torch.zeros(e_cap + 1, dtype=torch.int64), torch.full((t_cap,), -1, dtype=torch.int32)
+    pairs = [(int(short_off[i]) + a, int(short_off[i]) + b) for i in range(n) for a in range(int(bonds[i]))
+             for b in range(int(bonds[i])) if a != b]
+    first_of, second_of = {}, {}
+    for k, (a, b) in enumerate(pairs):
+        first_of.setdefault(a, []).append(k)
+        second_of.setdefault(b, []).append(k)
+    # a bond's run lies at its row of eto: the entry behind it has to be its end, so rows are taken in steps of two
+    rows = 2 * torch.randperm((e_cap - 1) // 2, generator=gen)[:len(rows)]
+    for b in range(len(rows)):
+        run = first_of.get(b, [])
+        eto[rows[b]], eto[rows[b] + 1] = (run[0], run[-1] + 1) if run else (0, 0)
+        for q, k in enumerate(second_of.get(b, [])):
+            second[run[0] + q] = k
+    gz3, gz2 = torch.randn(t_cap, C + 8, generator=gen), torch.randn(e_cap, C, generator=gen)
+    gsw = torch.randn(t_cap, 2, generator=gen)
+    d = lambda t: t.to(device)  # noqa: E731
+    dev = [d(t) for t in (gz3, gsw, short_off, torch.cat([rows.int(), torch.zeros(8, dtype=torch.int32)]), eto, second,
+                          pair_off, gz2, off, reverse)]
+    guv, gs = torch.zeros(e_cap, 2 * C, device=device), torch.zeros(e_cap, device=device)
+    sums = torch.full((n, 2 * C + 4), 3.0, device=device)
+    z3, sw, so, br, et, se, po, z2, of, rv = (t.data_ptr() for t in dev)
+    _abi.call("fmd_tb_vjp_sums_f32", z3, C + 8, C, sw, so, br, et, se, po, n, t_cap, guv.data_ptr(), 2 * C,
+              gs.data_ptr(), 0, z2, of, rv, e_cap, sums.data_ptr(), sums[:, C:].data_ptr(), 2 * C + 4,
+              _abi.stream_handle())
+    torch.cuda.synchronize()
+    eps = 2.0 ** -23
+
+    def close(got, terms):
+        if len(terms) == 0:
+            return not bool(got.any())
+        terms = terms.double().reshape(len(terms), -1)
+        return bool(((got.cpu().double().reshape(-1) - terms.sum(0)).abs() <= eps * len(terms) * terms.abs().sum(0)).all())
+
+    for i in range(n):
+        run = reverse[int(off[i]):min(int(off[i + 1]), e_cap)]
+        assert close(sums[i, :C], gz2[run[run >= 0].long()])
+        assert close(sums[i, C:2 * C], gz3[int(pair_off[i]):int(pair_off[i + 1]), :C])
+    for b, row in enumerate(rows.tolist()):
+        f, s2 = first_of.get(b, []), second_of.get(b, [])
+        assert close(guv[row, :C], gz3[f, :C]) and close(guv[row, C:], gz3[s2, :C])
+        assert close(gs[row], torch.cat([gsw[f, 0], gsw[s2, 1]]))
+    assert bool((sums[:, 2 * C:] == 3.0).all())
