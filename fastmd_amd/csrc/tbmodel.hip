@@ -734,8 +734,8 @@ __global__ void __launch_bounds__(256) tb_vjp_sums_kernel(LineCsr lc, const floa
 // bond rows only. No edge-sized product and no triplet-sized one is left (5 000 atoms, 3.5 A: 84 000
 // edges, 10 300 bonds, 26 000 triplets).
 // Against gathering [h_j | eps_e] and [eps_b1 | eps_b2 | h_i] into products over the edge and triplet rows: an MD step
-// of 5 000 atoms at 64 channels 773 -> 698 us (647 with the sums below in one launch), of 375 atoms at 128 channels 767 -> 470 (422), and an evaluation of
-// 500 atoms 988 -> 574.
+// of 5 000 atoms at 64 channels 773 -> 698 us, of 375 atoms at 128 channels 767 -> 470, an evaluation of 500
+// atoms 988 -> 574 (then 647, 422 and 550 with the sums above in one launch).
 
 // C[e, 0:N] (+)= [a0[e] | a1[e]] B^T over the real bonds e = bond_rows[k]: a workgroup takes 16 bonds x 64 columns,
 // each wave one 16 x 16 block of v_mfma_f32_16x16x4_f32 with its operands straight into registers (lane group
