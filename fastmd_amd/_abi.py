@@ -114,6 +114,10 @@ SIGNATURES: dict[str, tuple] = {
     "fmd_nhc_work_size": (_i64, [_i64]),
     "fmd_sum_f64": (ctypes.c_int, [_p, _i32, _i64, _p, _p]),
     "fmd_edge_geometry_f32": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _f32, _i32, _p, _p, _p, _p]),
+    "fmd_edge_forces_f32": (ctypes.c_int, [_p, _p, _i32, _p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _i64, _f32, _p, _p,
+                                           _p]),
+    "fmd_tb_edge_forces_f32": (ctypes.c_int, [_p, _p, _i32, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _i64,
+                                              _f32, _p, _p, _p]),
     "fmd_edge_geometry_bwd_f32": (ctypes.c_int, [_p, _p, _i32, _p, _i64, _p, _i64, _p, _p, _i64, _p, _p]),
     "fmd_mace_message_f32": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _p, _p, _f32, _p, _p, _i32,
                                             _p, _p, _i32, _i32, _p]),

@@ -291,3 +291,61 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* s_wave, T* total) {
   *total = s_wave[FMD_WAVE / 4];
   return s_wave[wave] + incl - v;
 }
+
+// Forces of one atom by one wave, from the gradient of the energy with respect to the edge vectors: the rows
+// [off[i], off[i + 1]) that it receives and their reverse rows, which it sends (reverse[e] < 0: none).
+// forces[i] = sign * (sum of the sent rows' gradients - sum of the received rows'). 32 rows a pass, lane l the
+// received row (l < 32) or its reverse: `grad(row, v)` forms each row's gradient where it is summed, twice per row
+// in all, instead of writing it and gathering it back. Stored to gvec, too, when given (the virial reads it).
+template <typename Grad>
+__device__ __forceinline__ void edge_forces_of(int64_t i, const int64_t* off, const int32_t* reverse, int64_t rows,
+                                               float sign, float* forces, float* gvec, const Grad& grad) {
+  const int lane = threadIdx.x & 63;
+  const bool sent = lane >= 32;
+  int64_t lo = off[i], hi = off[i + 1];
+  hi = hi < rows ? hi : rows;
+  float acc[3] = {0.f, 0.f, 0.f};
+  for (int64_t base = lo; base < hi; base += 32) {
+    const int64_t e = base + (lane & 31);
+    int64_t r = e < hi ? (sent ? (int64_t)reverse[e] : e) : -1;
+    const bool use = r >= 0 && r < rows;
+    r = use ? r : base;  // a real row, read and not added
+    float v[3];
+    grad(r, v);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (gvec && use && !sent) gvec[3 * r + k] = v[k];
+      acc[k] += use ? (sent ? v[k] : -v[k]) : 0.f;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) acc[k] = wave_sum(acc[k]);
+  if (lane < 3) forces[3 * i + lane] = sign * (lane == 0 ? acc[0] : lane == 1 ? acc[1] : acc[2]);
+}
+
+// sum_n (a[n] (+ b[n])) d[n] in order over n, a and b nullable; with eight 16-byte aligned values per row (`wide`)
+// every load is issued before the first product
+__device__ __forceinline__ float basis_dot(const float* d, const float* a, const float* b, int nb, bool wide) {
+  float s = 0.f;
+  if (wide) {
+    float4 x[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      x[h][0] = reinterpret_cast<const float4*>(d)[h];
+      x[h][1] = a ? reinterpret_cast<const float4*>(a)[h] : make_float4(0.f, 0.f, 0.f, 0.f);
+      x[h][2] = b ? reinterpret_cast<const float4*>(b)[h] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s += (x[h][1].x + x[h][2].x) * x[h][0].x;
+      s += (x[h][1].y + x[h][2].y) * x[h][0].y;
+      s += (x[h][1].z + x[h][2].z) * x[h][0].z;
+      s += (x[h][1].w + x[h][2].w) * x[h][0].w;
+    }
+    return s;
+  }
+  for (int n = 0; n < nb; ++n) s += ((a ? a[n] : 0.f) + (b ? b[n] : 0.f)) * d[n];
+  return s;
+}
+
+inline bool fmd_wide_rows(const void* p, int64_t ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

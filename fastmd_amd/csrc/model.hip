@@ -122,15 +122,9 @@ __global__ void edge_geometry_kernel(const GeoArgs a) {
 // up to two layers (gef0, gef1, times d ef / dr), the unit-vector and cutoff gradients (ggeo).
 __device__ __forceinline__ void edge_vec_grad(const float* geo, const float* def, int nb, const float* gef0,
                                               int64_t ld0, const float* gef1, int64_t ld1, const float* ggeo,
-                                              int64_t e, float (&out)[3]) {
+                                              int64_t e, bool wide, float (&out)[3]) {
   const float* g = geo + 8 * e;
-  float gr = 0.f;
-  for (int n = 0; n < nb; ++n) {
-    float ge = 0.f;
-    if (gef0) ge += gef0[e * ld0 + n];
-    if (gef1) ge += gef1[e * ld1 + n];
-    gr += ge * def[e * nb + n];
-  }
+  float gr = basis_dot(def + e * nb, gef0 ? gef0 + e * ld0 : nullptr, gef1 ? gef1 + e * ld1 : nullptr, nb, wide);
   float gu[3] = {0.f, 0.f, 0.f};
   if (ggeo) {
     gu[0] = ggeo[4 * e];
@@ -155,9 +149,25 @@ __global__ void edge_geometry_bwd_kernel(const float* geo, const float* def, int
     return;
   }
   float v[3];
-  edge_vec_grad(geo, def, nb, gef0, ld0, gef1, ld1, ggeo, e, v);
+  edge_vec_grad(geo, def, nb, gef0, ld0, gef1, ld1, ggeo, e, false, v);
 #pragma unroll
   for (int k = 0; k < 3; ++k) gvec[3 * e + k] = v[k];
+}
+
+// Forces straight from the rows' geometry gradients, one launch instead of the row kernel and the two-term segment
+// sum over its output: 12.6 + 9.2 -> 13.2 us at 10 000 atoms, 5.7 + 4.6 -> 5.2 at 1 080; bound by the gathered reverse
+// rows (a 135-atom MD step 135 -> 131 us).
+__global__ void __launch_bounds__(kThreads) edge_forces_kernel(const float* geo, const float* def, int nb,
+                                                               const float* gef0, int64_t ld0, const float* gef1,
+                                                               int64_t ld1, const float* ggeo, const int64_t* off,
+                                                               const int32_t* reverse, const int64_t* n_edges,
+                                                               int64_t e_cap, int64_t n, float sign, bool wide,
+                                                               float* forces, float* gvec) {
+  const int64_t i = fmd_xcd_block(blockIdx.x, gridDim.x) * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (i >= n) return;
+  edge_forces_of(i, off, reverse, real_rows(n_edges, e_cap), sign, forces, gvec, [&](int64_t e, float (&v)[3]) {
+    edge_vec_grad(geo, def, nb, gef0, ld0, gef1, ld1, ggeo, e, wide, v);
+  });
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1461,6 +1471,22 @@ int fmd_edge_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, co
   if (e_cap == 0) return FMD_OK;
   hipLaunchKernelGGL(edge_geometry_bwd_kernel, dim3((unsigned)fmd_cdiv(e_cap, 256)), dim3(256), 0, stream, geo, def,
                      nb, gef0, ld0, gef1, ld1, ggeo, n_edges, e_cap, gvec);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_edge_forces_f32(const float* geo, const float* def, int32_t nb, const float* gef0, int64_t ld0,
+                        const float* gef1, int64_t ld1, const float* ggeo, const int64_t* offsets,
+                        const int32_t* reverse, const int64_t* n_edges, int64_t e_cap, int64_t n_atoms, float sign,
+                        float* forces, float* gvec, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && nb > 0);
+  if (n_atoms == 0) return FMD_OK;
+  FMD_REQUIRE(offsets && n_edges && forces && (e_cap == 0 || (geo && def && reverse)));
+  const bool wide = nb == 8 && fmd_wide_rows(def, 8) && (!gef0 || fmd_wide_rows(gef0, ld0)) &&
+                    (!gef1 || fmd_wide_rows(gef1, ld1));
+  hipLaunchKernelGGL(edge_forces_kernel, dim3((unsigned)fmd_cdiv(n_atoms, kWaves)), dim3(kThreads), 0, stream, geo, def,
+                     nb, gef0, ld0, gef1, ld1, ggeo, offsets, reverse, n_edges, e_cap, n_atoms, sign, wide, forces,
+                     gvec);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

@@ -250,34 +250,53 @@ __global__ void tb_readout_bwd_kernel(const float* ge, float sign, const float* 
 }
 
 // gvec = gr u + (gu - (gu . u) u) / r with gr = sum_n gef def + gfc dfc + gs ds
-__global__ void tb_geometry_bwd_kernel(const float* geo, const float* def, int nb, const float* gef, int64_t ldgef,
-                                       const float* gu, int64_t ldgu, const float* gfc, const float* gs,
-                                       const uint8_t* bond_flags, const int64_t* n_edges, int64_t e_cap,
-                                       float* gvec) {
+struct RowGrads {
+  const float *geo, *def, *gef, *gu, *gfc, *gs;
+  const uint8_t* bond_flags;
+  int64_t ldgef, ldgu;
+  int nb;
+  bool wide;
+  __device__ __forceinline__ void operator()(int64_t e, float (&out)[3]) const {
+    const float* g = geo + 8 * e;
+    float gr = gef ? basis_dot(def + e * nb, gef + e * ldgef, nullptr, nb, wide) : 0.f;
+    if (gfc) gr += gfc[e] * g[5];
+    // gs and gu hold values on the bond rows only (with bond_flags; else on every row)
+    const bool bond = bond_flags ? bond_flags[e] != 0 : true;
+    if (gs && bond) gr += gs[e] * g[7];
+    float v[3] = {0.f, 0.f, 0.f};
+    if (gu && bond) {
+      v[0] = gu[e * ldgu];
+      v[1] = gu[e * ldgu + 1];
+      v[2] = gu[e * ldgu + 2];
+    }
+    const float inv_r = 1.0f / g[3];
+    const float gdotu = v[0] * g[0] + v[1] * g[1] + v[2] * g[2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) out[k] = gr * g[k] + (v[k] - gdotu * g[k]) * inv_r;
+  }
+};
+
+__global__ void tb_geometry_bwd_kernel(const RowGrads rg, const int64_t* n_edges, int64_t e_cap, float* gvec) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= e_cap) return;
   if (e >= tb_real_rows(n_edges, e_cap)) {
     gvec[3 * e] = gvec[3 * e + 1] = gvec[3 * e + 2] = 0.f;
     return;
   }
-  const float* g = geo + 8 * e;
-  float gr = 0.f;
-  if (gef)
-    for (int n = 0; n < nb; ++n) gr += gef[e * ldgef + n] * def[e * nb + n];
-  if (gfc) gr += gfc[e] * g[5];
-  // gs and gu hold values on the bond rows only (with bond_flags; else on every row)
-  const bool bond = bond_flags ? bond_flags[e] != 0 : true;
-  if (gs && bond) gr += gs[e] * g[7];
-  float v[3] = {0.f, 0.f, 0.f};
-  if (gu && bond) {
-    v[0] = gu[e * ldgu];
-    v[1] = gu[e * ldgu + 1];
-    v[2] = gu[e * ldgu + 2];
-  }
-  const float inv_r = 1.0f / g[3];
-  const float gdotu = v[0] * g[0] + v[1] * g[1] + v[2] * g[2];
+  float v[3];
+  rg(e, v);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) gvec[3 * e + k] = gr * g[k] + (v[k] - gdotu * g[k]) * inv_r;
+  for (int k = 0; k < 3; ++k) gvec[3 * e + k] = v[k];
+}
+
+// the forces straight from them (edge_forces_of): 8.3 + 6.0 us of the row kernel and the segment sum -> 6.8 at
+// 5 000 atoms
+__global__ void __launch_bounds__(256) tb_edge_forces_kernel(const RowGrads rg, const int64_t* off,
+                                                             const int32_t* reverse, const int64_t* n_edges,
+                                                             int64_t e_cap, int64_t n, float sign, float* forces,
+                                                             float* gvec) {
+  const int64_t i = fmd_xcd_block(blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (i < n) edge_forces_of(i, off, reverse, tb_real_rows(n_edges, e_cap), sign, forces, gvec, rg);
 }
 
 // ---- angle -> bond sums over the line graph. The work is a few bonds and triplets per atom, far
@@ -1312,8 +1331,26 @@ int fmd_tb_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, cons
   FMD_REQUIRE(geo && def && n_edges && gvec);
   FMD_REQUIRE(!gef || ldgef >= nb);
   FMD_REQUIRE(!gu || ldgu >= 3);
-  hipLaunchKernelGGL(tb_geometry_bwd_kernel, dim3((unsigned)fmd_cdiv(e_cap, 256)), dim3(256), 0, stream, geo, def, nb,
-                     gef, ldgef, gu, ldgu, gfc, gs, bond_flags, n_edges, e_cap, gvec);
+  const RowGrads rg{geo, def, gef, gu, gfc, gs, bond_flags, ldgef, ldgu, nb, false};
+  hipLaunchKernelGGL(tb_geometry_bwd_kernel, dim3((unsigned)fmd_cdiv(e_cap, 256)), dim3(256), 0, stream, rg, n_edges,
+                     e_cap, gvec);
+  FMD_CHECK_LAUNCH();
+  return FMD_OK;
+}
+
+int fmd_tb_edge_forces_f32(const float* geo, const float* def, int32_t nb, const float* gef, int64_t ldgef,
+                           const float* gu, int64_t ldgu, const float* gfc, const float* gs, const uint8_t* bond_flags,
+                           const int64_t* offsets, const int32_t* reverse, const int64_t* n_edges, int64_t e_cap,
+                           int64_t n_atoms, float sign, float* forces, float* gvec, hipStream_t stream) {
+  FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && nb > 0);
+  if (n_atoms == 0) return FMD_OK;
+  FMD_REQUIRE(offsets && n_edges && forces && (e_cap == 0 || (geo && def && reverse)));
+  FMD_REQUIRE(!gef || ldgef >= nb);
+  FMD_REQUIRE(!gu || ldgu >= 3);
+  const bool wide = nb == 8 && fmd_wide_rows(def, 8) && (!gef || fmd_wide_rows(gef, ldgef));
+  const RowGrads rg{geo, def, gef, gu, gfc, gs, bond_flags, ldgef, ldgu, nb, wide};
+  hipLaunchKernelGGL(tb_edge_forces_kernel, dim3((unsigned)fmd_cdiv(n_atoms, 4)), dim3(256), 0, stream, rg, offsets,
+                     reverse, n_edges, e_cap, n_atoms, sign, forces, gvec);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

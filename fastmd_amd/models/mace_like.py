@@ -41,7 +41,7 @@ from torch.autograd import Function
 from fastmd_amd import _abi
 from fastmd_amd.adapters.protocol import (CapacityStep, CaptureContract, GraphBatch, PaddingRule, TopologySpec,
                                          require_atom_rows, system_rows)
-from fastmd_amd.ops.csr_segment_sum import Csr, segment_sum_csr
+from fastmd_amd.ops.csr_segment_sum import Csr
 from fastmd_amd.ops.wide_gemm import (Planes, gemm, gemm_gather, gemm_group, gemm_planes, gemm_splitk,
                                      split_planes)
 
@@ -794,12 +794,14 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
                     b_planes=model.w1_node_blocks_planes(t))
         gefs.append((gef, nb))
         g_out0, g_out1 = g_in0, g_in1
-    gvec = _empty(e_cap, 3, device=dev)
+    # the gradient of every edge vector, kept for the virial only, and the forces from it
+    gvec = None if stress_cell is None else _empty(e_cap, 3, device=dev)
+    forces = _empty(n, 3, device=dev)
     (g0, ld0) = gefs[0]
     (g1, ld1) = gefs[1] if len(gefs) > 1 else (None, 0)
-    _call("fmd_edge_geometry_bwd_f32", ctx.geo.data_ptr(), ctx.de.data_ptr(), nb, g0.data_ptr(), ld0,
-          _abi.ptr(g1), ld1, ggeo.data_ptr(), n_edges.data_ptr(), e_cap, gvec.data_ptr())
-    forces = segment_sum_csr([(gvec, inputs.csr_src, 0, sign, None), (gvec, inputs.csr_dst, 0, -sign, None)], n, 3)
+    _call("fmd_edge_forces_f32", ctx.geo.data_ptr(), ctx.de.data_ptr(), nb, g0.data_ptr(), ld0, _abi.ptr(g1), ld1,
+          ggeo.data_ptr(), off.data_ptr(), rev.data_ptr(), n_edges.data_ptr(), e_cap, n, sign, forces.data_ptr(),
+          _abi.ptr(gvec))
     if stress_cell is None:
         return forces
     from fastmd_amd.engine.energy_derivative import edge_stress

@@ -50,7 +50,7 @@ from torch.autograd import Function
 from fastmd_amd import _abi
 from fastmd_amd.adapters.protocol import (CapacityStep, CaptureContract, GraphBatch, PaddingRule, TopologySpec,
                                          require_atom_rows, system_rows)
-from fastmd_amd.ops.csr_segment_sum import Csr, _prep_off, _prep_perm, segment_sum_csr
+from fastmd_amd.ops.csr_segment_sum import Csr, _prep_off, _prep_perm
 from fastmd_amd.ops.threebody import LineGraph, fourier_line_vjp
 from fastmd_amd.ops.wide_gemm import gemm, gemm_group, split_planes
 
@@ -299,10 +299,11 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
     galpha = gemm(gz3_all, lay["w3d"], b_layout=0)  # [T, A]
     gu = _empty(e_cap, 3, device=dev)  # written on the bond rows only (read there only)
     fourier_line_vjp(galpha, geo[:, :3], lg, model.freqs, model.fourier_scale, out=gu, accumulate=False)
-    gvec = _empty(e_cap, 3, device=dev)
-    _call("fmd_tb_geometry_bwd_f32", geo.data_ptr(), ctx.de.data_ptr(), nb, gef.data_ptr(), nb, gu.data_ptr(), 3,
-          gfc.data_ptr(), gs.data_ptr(), lg.short_flags.data_ptr(), batch.n_edges.data_ptr(), e_cap, gvec.data_ptr())
-    forces = segment_sum_csr([(gvec, inputs.csr_src, 0, sign, None), (gvec, inputs.csr_dst, 0, -sign, None)], n, 3)
+    gvec = None if stress_cell is None else _empty(e_cap, 3, device=dev)  # the virial reads it
+    forces = _empty(n, 3, device=dev)
+    _call("fmd_tb_edge_forces_f32", geo.data_ptr(), ctx.de.data_ptr(), nb, gef.data_ptr(), nb, gu.data_ptr(), 3,
+          gfc.data_ptr(), gs.data_ptr(), lg.short_flags.data_ptr(), sent_off.data_ptr(), sent.data_ptr(),
+          batch.n_edges.data_ptr(), e_cap, n, sign, forces.data_ptr(), _abi.ptr(gvec))
     if stress_cell is None:
         return forces
     from fastmd_amd.engine.energy_derivative import edge_stress

@@ -353,6 +353,12 @@ int fmd_tb_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, cons
                             const float* gu, int64_t ldgu, const float* gfc, const float* gs, const uint8_t* bond_flags,
                             const int64_t* n_edges, int64_t e_cap, float* gvec, hipStream_t stream);
 
+/* The same with the forces formed and stored as fmd_edge_forces_f32 does (gvec nullable, real rows only). */
+int fmd_tb_edge_forces_f32(const float* geo, const float* def, int32_t nb, const float* gef, int64_t ldgef,
+                           const float* gu, int64_t ldgu, const float* gfc, const float* gs, const uint8_t* bond_flags,
+                           const int64_t* offsets, const int32_t* reverse, const int64_t* n_edges, int64_t e_cap,
+                           int64_t n_atoms, float sign, float* forces, float* gvec, hipStream_t stream);
+
 /* The padded rows of a model-graph bucket workspace (gpu_md.py model_graph, cuda_graph.py:209-293
  * _PaddedEdgesWorkspace.update): rows [e_real, e_cap) of a ragged build copied into a fixed
  * capacity become the builder's far self-loops of atom (row - e_real) mod n_atoms with the pad
@@ -658,6 +664,13 @@ int fmd_edge_geometry_f32(const float* positions, const float* cell, const int32
 int fmd_edge_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, const float* gef0, int64_t ld0,
                               const float* gef1, int64_t ld1, const float* ggeo, const int64_t* n_edges,
                               int64_t e_cap, float* gvec, hipStream_t stream);
+/* forces[i] = sign * (sum of gvec over the rows that atom i sends, reverse[offsets[i] .. offsets[i + 1]), negative
+ * entries skipped, - sum over the rows that it receives), gvec formed on the way (and stored on the real rows when
+ * given): fmd_edge_geometry_bwd_f32 and its two sums in one launch. */
+int fmd_edge_forces_f32(const float* geo, const float* def, int32_t nb, const float* gef0, int64_t ld0,
+                        const float* gef1, int64_t ld1, const float* ggeo, const int64_t* offsets,
+                        const int32_t* reverse, const int64_t* n_edges, int64_t e_cap, int64_t n_atoms, float sign,
+                        float* forces, float* gvec, hipStream_t stream);
 /* A0[i], A1[i] = inv_avg * sum over the rows of centre i of the messages. z [E, W] holds the
  * edge pre-activation blocks a | b | c | d (W = 4C) when h1 is given; with h1 null (zero vector
  * features, where c and d meet only zeros) z holds a | b only (W = 2C). The pre-activations are
