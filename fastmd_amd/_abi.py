@@ -65,9 +65,9 @@ SIGNATURES: dict[str, tuple] = {
                                               _f32, _p, _i64, _p, _i64, _p]),
     "fmd_tb_vjp_sums_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i64, _p, _i32, _p,
                                            _p, _p, _i64, _p, _p, _i64, _p]),
-    "fmd_tb_bond_product_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, _i32, _p, _i64, _i32, _p, _p, _i64, _i64, _p,
-                                               _i64, _i32, _p]),
-    "fmd_tb_bond_init_f32": (ctypes.c_int, [_p, _i32, _p, _i32, _p, _p, _i64, _i64, _p, _i64, _p]),
+    "fmd_tb_bond_product_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i64,
+                                               _p, _i64, _i32, _p]),
+    "fmd_tb_bond_init_f32": (ctypes.c_int, [_p, _i32, _p, _i32, _p, _p, _p, _i64, _i64, _p, _i64, _p]),
     "fmd_tb_bond_basis_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _i32, _p, _p, _i64, _i64, _p, _p]),
     "fmd_tb_edge_sum_f32": (ctypes.c_int, [_p, _i64, _p, _p, _i32, _p, _i32, _p, _p, _p, _i64, _p, _i64, _i64, _f32,
                                            _p, _p, _i64, _p]),

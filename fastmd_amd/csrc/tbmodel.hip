@@ -769,7 +769,17 @@ struct BondProduct {
   float* c;
   int64_t ld0, ld1, ldb, ldc;
   int k0, k, n, accumulate;  // columns [0, k0) of K from a0, the rest from a1
+  const uint8_t* overflow;   // nullable: the build's flag
 };
+
+// An overflowed build's bond rows and triplet rows do not belong together (its triplets are the padding topology's),
+// and rows that no kernel below writes may be read: what would be their products is zero on every row instead, so
+// that such an evaluation, whose results are discarded, is finite whatever the memory held.
+__device__ __forceinline__ void zero_rows(float* c, int64_t ldc, int64_t rows, int n) {
+  const int64_t step = (int64_t)gridDim.x * 4;
+  for (int64_t r = wave_id(); r < rows; r += step)
+    for (int k = threadIdx.x & 63; k < n; k += 64) c[r * ldc + k] = 0.f;
+}
 
 __device__ __forceinline__ int64_t bond_count(const LineCsr& lc, int64_t e_cap) {
   const int64_t nb = lc.short_offsets[lc.n];
@@ -779,6 +789,10 @@ __device__ __forceinline__ int64_t bond_count(const LineCsr& lc, int64_t e_cap) 
 __global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_t e_cap, const BondProduct p) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
+  if (p.overflow && p.overflow[0]) {
+    if (!p.accumulate) zero_rows(p.c, p.ldc, e_cap, p.n);
+    return;
+  }
   const int64_t ct = p.n / 16, tiles = fmd_cdiv(nb, 16) * ct;  // a multiple of four: a workgroup's waves share bonds
   for (int64_t w = wave_id(); w < tiles; w += nw) {
     const int64_t tm = w / ct, col = (w - tm * ct) * 16 + i, slot = tm * 16 + i;
@@ -823,7 +837,12 @@ __global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_
 // stored at columns 0, 2 C and 3 C of the row (eps | . | u | v). A wave takes four bonds and 64 columns, eight rows
 // of m in flight together with the bond rows they do not depend on.
 __global__ void __launch_bounds__(256) tb_bond_init_kernel(LineCsr lc, int64_t e_cap, const float* ef, int nbasis,
-                                                           const float* m, int C, float* out, int64_t ldo) {
+                                                           const float* m, int C, const uint8_t* overflow, float* out,
+                                                           int64_t ldo) {
+  if (overflow && overflow[0]) {
+    zero_rows(out, ldo, e_cap, 4 * C);
+    return;
+  }
   const int lane = threadIdx.x & 63, blocks = fmd_cdiv(3 * C, 64);
   const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
   for (int64_t w = wave_id(); w < fmd_cdiv(nb, 4) * blocks; w += nw) {
@@ -1169,22 +1188,22 @@ int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const fl
 }
 
 int fmd_tb_bond_init_f32(const float* ef, int32_t n_basis, const float* m, int32_t channels,
-                         const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
-                         float* out, int64_t ldo, hipStream_t stream) {
+                         const int64_t* short_offsets, const int32_t* bond_rows, const uint8_t* overflow,
+                         int64_t n_atoms, int64_t e_cap, float* out, int64_t ldo, hipStream_t stream) {
   FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && channels > 0 && n_basis > 0 && ldo >= 4 * (int64_t)channels);
   if (n_atoms == 0 || e_cap == 0) return FMD_OK;
   FMD_REQUIRE(ef && m && short_offsets && bond_rows && out);
   LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
   hipLaunchKernelGGL(tb_bond_init_kernel, dim3(kStrideBlocks), dim3(256), 0, stream, lc, e_cap, ef, n_basis, m, channels,
-                     out, ldo);
+                     overflow, out, ldo);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }
 
 int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const float* a1, int64_t ld1, int32_t k,
                             const float* b, int64_t ldb, int32_t n, const int64_t* short_offsets,
-                            const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap, float* c, int64_t ldc,
-                            int32_t accumulate, hipStream_t stream) {
+                            const int32_t* bond_rows, const uint8_t* overflow, int64_t n_atoms, int64_t e_cap,
+                            float* c, int64_t ldc, int32_t accumulate, hipStream_t stream) {
   FMD_REQUIRE(n_atoms >= 0 && e_cap >= 0 && k0 > 0 && k0 % 32 == 0 && k >= k0 && k % 32 == 0 && n > 0 && n % 64 == 0);
   if (n_atoms == 0 || e_cap == 0) return FMD_OK;
   FMD_REQUIRE(a0 && ld0 >= k0 && b && ldb >= k && c && ldc >= n && short_offsets && bond_rows);
@@ -1192,7 +1211,7 @@ int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const floa
   const auto aligned = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   FMD_REQUIRE(aligned(a0) && ld0 % 4 == 0 && aligned(b) && ldb % 4 == 0 && (k == k0 || (aligned(a1) && ld1 % 4 == 0)));
   LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
-  const BondProduct p{a0, k == k0 ? nullptr : a1, b, c, ld0, ld1, ldb, ldc, k0, k, n, accumulate};
+  const BondProduct p{a0, k == k0 ? nullptr : a1, b, c, ld0, ld1, ldb, ldc, k0, k, n, accumulate, overflow};
   hipLaunchKernelGGL(tb_bond_product_kernel, dim3(2 * kStrideBlocks), dim3(256), 0, stream, lc, e_cap, p);
   FMD_CHECK_LAUNCH();
   return FMD_OK;

@@ -216,7 +216,8 @@ def _forward(ctx, positions: Tensor, cell: Tensor, model: ThreeBodyLike, inputs:
     x = _empty(e_cap, 4 * C, device=dev)
     x_eps, x_c, x_u, x_v = (x[:, k * C:].data_ptr() for k in range(4))
     hpq = _empty(n, 3 * C, device=dev)
-    _call("fmd_tb_bond_init_f32", ef.data_ptr(), nb, lay["init"].data_ptr(), C, *lines, lg.n_atoms, e_cap, x_eps, 4 * C)
+    _call("fmd_tb_bond_init_f32", ef.data_ptr(), nb, lay["init"].data_ptr(), C, *lines,
+          _abi.ptr(lg.overflow), lg.n_atoms, e_cap, x_eps, 4 * C)
     saved = []
     for t in range(L):
         gemm_group([{"a": h, "b": lay["node"][t], "b_planes": lay["node_planes"][t], "out": hpq}], b_layout=0)
@@ -226,7 +227,7 @@ def _forward(ctx, positions: Tensor, cell: Tensor, model: ThreeBodyLike, inputs:
               inv_ang, z3.data_ptr(), C, x_eps, 4 * C)
         bond = lay["bond"][t]
         _call("fmd_tb_bond_product_f32", x_eps, 4 * C, C, None, 0, C, bond.data_ptr(), C, bond.shape[0], *lines,
-              lg.n_atoms, e_cap, x_c, 4 * C, 0)
+              _abi.ptr(lg.overflow), lg.n_atoms, e_cap, x_c, 4 * C, 0)
         z2 = _empty(e_cap, C, device=dev)
         _call("fmd_tb_edge_sum_f32", hpq[:, C:].data_ptr(), 3 * C, ei.data_ptr(), ef.data_ptr(), nb,
               lay["rt"][t].data_ptr(), C, geo.data_ptr(), lg.short_flags.data_ptr(), x_c, 4 * C, off.data_ptr(), n,
@@ -272,7 +273,8 @@ def _vjp(ctx, gE: Tensor | None, sign: float, stress_cell: Tensor | None = None)
 
     def bond_product(a0, k0, a1, weight, accumulate):
         _call("fmd_tb_bond_product_f32", a0.data_ptr(), k0, k0, _abi.ptr(a1), 2 * C, weight.shape[1],
-              weight.data_ptr(), weight.shape[1], C, *lines, n, e_cap, geps.data_ptr(), C, accumulate)
+              weight.data_ptr(), weight.shape[1], C, *lines, _abi.ptr(lg.overflow), n, e_cap, geps.data_ptr(), C,
+              accumulate)
 
     for t in reversed(range(L)):
         z3, z2 = ctx.saved[t]

@@ -316,15 +316,17 @@ int fmd_tb_vjp_sums_f32(const float* gz3, int64_t ldz, int32_t channels, const f
                         int64_t lds, hipStream_t stream);
 /* Products on the bond rows e = bond_rows[0, short_offsets[n]) alone (the count read on the device): c[e,
  * 0:n] (+)= [a0[e, 0:k0] | a1[e, 0:k-k0]] b^T, b [n, k] K-contiguous. k0, k multiples of 32, n of 64, operands 16-byte
- * aligned with strides of 4. */
+ * aligned with strides of 4. With the build's overflow flag given and set: every row of c is zero (left with
+ * accumulate). */
 int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const float* a1, int64_t ld1, int32_t k,
                             const float* b, int64_t ldb, int32_t n, const int64_t* short_offsets,
-                            const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap, float* c, int64_t ldc,
-                            int32_t accumulate, hipStream_t stream);
-/* out[e] = ef[e] m per bond row, m [n_basis, 3 C] in blocks stored at columns 0, 2 C and 3 C. */
+                            const int32_t* bond_rows, const uint8_t* overflow, int64_t n_atoms, int64_t e_cap,
+                            float* c, int64_t ldc, int32_t accumulate, hipStream_t stream);
+/* out[e] = ef[e] m per bond row, m [n_basis, 3 C] in blocks stored at columns 0, 2 C and 3 C (overflow as
+ * above: all 4 C columns of every row zero). */
 int fmd_tb_bond_init_f32(const float* ef, int32_t n_basis, const float* m, int32_t channels,
-                         const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,
-                         float* out, int64_t ldo, hipStream_t stream);
+                         const int64_t* short_offsets, const int32_t* bond_rows, const uint8_t* overflow,
+                         int64_t n_atoms, int64_t e_cap, float* out, int64_t ldo, hipStream_t stream);
 /* gef[e, n] = sum_c geps[e, c] we[n, c] per bond row (the other rows are left). */
 int fmd_tb_bond_basis_f32(const float* geps, int64_t ldg, int32_t channels, const float* we, int32_t n_basis,
                           const int64_t* short_offsets, const int32_t* bond_rows, int64_t n_atoms, int64_t e_cap,

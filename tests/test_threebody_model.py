@@ -315,7 +315,7 @@ def test_bond_product_rows(device, count, k0, k1, n, accumulate):
     pad = torch.zeros(8, dtype=torch.int32)
     a0d, a1d, bd, cd, rd, od = d(a0), d(a1), d(b), d(c), d(torch.cat([listed.int(), pad])), d(offsets)
     _abi.call("fmd_tb_bond_product_f32", a0d.data_ptr(), k0 + 4, k0, a1d.data_ptr(), max(k1, 4), k, bd.data_ptr(), k, n,
-              od.data_ptr(), rd.data_ptr(), 2, rows, cd.data_ptr(), n + 3, accumulate, _abi.stream_handle())
+              od.data_ptr(), rd.data_ptr(), None, 2, rows, cd.data_ptr(), n + 3, accumulate, _abi.stream_handle())
     torch.cuda.synchronize()
     got = cd.cpu()
     a = torch.cat([a0[:, :k0], a1[:, :k1]], 1).double()[listed]
@@ -389,3 +389,31 @@ def test_vjp_sums(device, channels, longest):
         assert close(guv[row, :C], gz3[f, :C]) and close(guv[row, C:], gz3[s2, :C])
         assert close(gs[row], torch.cat([gsw[f, 0], gsw[s2, 1]]))
     assert bool((sums[:, 2 * C:] == 3.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("u_cap,t_cap,overflow", [(None, None, False), (None, 300, True), (900, None, True)])
+def test_threebody_reads_no_unwritten_memory(device, u_cap, t_cap, overflow):
+    """With every allocation taken from memory full of NaN the results are the bits of a run without; an
+    overflowed build (triplets, then edges) gives finite ones, as its discarded step goes on from them."""
+    from fastmd_amd.engine.energy_derivative import EnergyDerivative
+    from fastmd_amd.models.threebody_like import ThreeBodyAdapter
+
+    s = systems.perovskite(3, sigma=0.2)
+    m, _, _, _ = _params(3.5)
+    adapter = ThreeBodyAdapter(m, device=device)
+    builder = _builder(s, 3.5, device, u_cap=u_cap, t_cap=t_cap)
+    _, status = builder.build(torch.tensor(s.positions, device=device))
+    assert bool(status.overflow.item()) == overflow
+    inputs = adapter.prepare(builder.batch)
+    deriv = EnergyDerivative(adapter)
+    first = deriv(builder.batch, inputs, n_real=s.n_atoms)
+    sizes = [2 ** k for k in range(9, 24)]  # floats: the blocks of the allocator's small and large pools
+    held = [torch.full((k,), float("nan"), device=device) for k in sizes for _ in range(8 if k < 2 ** 20 else 4)]
+    torch.cuda.synchronize()
+    del held
+    out = deriv(builder.batch, inputs, n_real=s.n_atoms)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(out["f"][0]).all()) and bool(torch.isfinite(out["e"]).all())
+    if not overflow:
+        assert torch.equal(out["e"], first["e"]) and torch.equal(out["f"][0], first["f"][0])
