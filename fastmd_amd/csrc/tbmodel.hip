@@ -761,7 +761,8 @@ __global__ void __launch_bounds__(256) tb_vjp_sums_kernel(LineCsr lc, const floa
 // g = l / 16 holds k = 8 g .. 8 g + 8 of a 32-k slice), the loads of up to four slices in flight: the operands are
 // one round trip per 128 of K behind the row look-up. The count is read on the device, the grid strides. Bound by that
 // chain of round trips: 7.9 us at 400 atoms and 128 channels (12.4 with one wave per 16 x 64 tile and one
-// slice in flight), 11.5 at 10 300 bonds and 64 channels (the same).
+// slice in flight), 11.4 at 10 300 bonds and 64 channels (the same). S: the slices in flight, two where K has no
+// more (fewer registers, seven waves per SIMD instead of four: K = 64 at 10 300 bonds 11.4 -> 10.5 us).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct BondProduct {
@@ -786,6 +787,7 @@ __device__ __forceinline__ int64_t bond_count(const LineCsr& lc, int64_t e_cap) 
   return nb < e_cap ? nb : e_cap;
 }
 
+template <int S>
 __global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_t e_cap, const BondProduct p) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int64_t nb = bond_count(lc, e_cap), nw = (int64_t)gridDim.x * 4;
@@ -799,10 +801,10 @@ __global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_
     const int e = lc.bond_rows[slot < nb ? slot : nb - 1];
     const float *r0 = p.a0 + e * p.ld0, *r1 = p.a1 ? p.a1 + e * p.ld1 : r0, *bp = p.b + col * p.ldb + 8 * g;
     f32x4_t acc{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < p.k; k0 += 128) {
-      float4 a[4][2], b[4][2];
+    for (int k0 = 0; k0 < p.k; k0 += 32 * S) {
+      float4 a[S][2], b[S][2];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < S; ++q) {
         const int k = k0 + 32 * q;
         if (k >= p.k) break;
         b[q][0] = *reinterpret_cast<const float4*>(bp + k);
@@ -812,7 +814,7 @@ __global__ void __launch_bounds__(256) tb_bond_product_kernel(LineCsr lc, int64_
         a[q][1] = *reinterpret_cast<const float4*>(ap + 4);
       }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < S; ++q) {
         if (k0 + 32 * q >= p.k) break;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -1212,7 +1214,10 @@ int fmd_tb_bond_product_f32(const float* a0, int64_t ld0, int32_t k0, const floa
   FMD_REQUIRE(aligned(a0) && ld0 % 4 == 0 && aligned(b) && ldb % 4 == 0 && (k == k0 || (aligned(a1) && ld1 % 4 == 0)));
   LineCsr lc{short_offsets, bond_rows, nullptr, nullptr, nullptr, nullptr, n_atoms, 0};
   const BondProduct p{a0, k == k0 ? nullptr : a1, b, c, ld0, ld1, ldb, ldc, k0, k, n, accumulate, overflow};
-  hipLaunchKernelGGL(tb_bond_product_kernel, dim3(2 * kStrideBlocks), dim3(256), 0, stream, lc, e_cap, p);
+  if (k <= 64)
+    hipLaunchKernelGGL((tb_bond_product_kernel<2>), dim3(2 * kStrideBlocks), dim3(256), 0, stream, lc, e_cap, p);
+  else
+    hipLaunchKernelGGL((tb_bond_product_kernel<4>), dim3(2 * kStrideBlocks), dim3(256), 0, stream, lc, e_cap, p);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }
