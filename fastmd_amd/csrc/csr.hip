@@ -21,6 +21,7 @@
 // event of its own: waiting for the whole sequence instead left the GPU idle between calls (279, 236
 // and 444 us). Host time bounded the three then: 150, 115 and 260 us with cheaper launches.
 #include "common.h"
+#include "search.h"
 
 namespace {
 
@@ -210,20 +211,7 @@ __global__ void __launch_bounds__(kThreads) csr_scatter_kernel(const Jobs jobs, 
   }
 }
 
-// off[s] = rows with a key below s (binary search over the sorted keys)
-template <typename Key>
-__device__ __forceinline__ int32_t lower_bound(const Key* key, int32_t rows, uint32_t s) {
-  int32_t lo = 0, hi = rows;
-  while (lo < hi) {
-    const int32_t mid = (lo + hi) >> 1;
-    if (key[mid] < s)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
+// off[s] = rows with a key below s
 __global__ void __launch_bounds__(kThreads) csr_offsets_kernel(const Jobs jobs) {
   const Job& j = jobs.j[blockIdx.y];
   const int64_t s = (int64_t)blockIdx.x * kThreads + threadIdx.x;
