@@ -24,11 +24,14 @@
 namespace {
 
 constexpr int kSmallThreads = 1024;   // fused single-workgroup build
-// The fused build up to this many atoms. Its one workgroup walks its atoms in turn, while the three
-// launches of the multi-block build cost the same 13 us at any size here (graph-captured builds with
+constexpr int kSmallMaxAtoms = 1024;  // LDS-resident wrapped coordinates up to this many atoms
+// fmd_nl_build takes the fused build up to this many atoms. Its one workgroup walks its atoms in turn, while
+// the three launches of the multi-block build cost the same 13 us at any size here (graph-captured builds with
 // reverse rows and window fold, us fused / three launches: 40 atoms 11.1 / 12.1, 60 12.8 / 12.7,
-// 90 16.5 / 12.9, 135 21.4 / 13.3, 400 51 / 13.5, 900 138 / 13.9).
-constexpr int kSmallMaxAtoms = 60;
+// 90 16.5 / 12.9, 135 21.4 / 13.3, 400 51 / 13.5, 900 138 / 13.9). The allocation-free entry takes it up to
+// kSmallMaxAtoms: it has no scratch of the call's own for the partials, and the fused build needs none, so
+// calls of such sizes may overlap.
+constexpr int kFusedAtoms = 60;
 constexpr int kSmallBatch = 4;        // atoms per wave whose candidate loads are issued together
 constexpr int kSmallMaxEdges = 8192;  // rows whose reverse search runs on LDS copies of their keys
 constexpr int kImageBias = 512;       // packed image fields: component + 512 in 10 bits
@@ -1240,10 +1243,10 @@ __global__ void nl_window_flags_kernel(const int64_t* edge_count, const uint8_t*
               w_edges, w_iso, max_disp ? max_disp[0] : 0.f, stats, triplet_count, t_cap, w_triplets);
 }
 
-// The build's launches (small systems: one fused workgroup; otherwise count -> offsets and
+// The build's launches (up to fused_atoms: one fused workgroup; otherwise count -> offsets and
 // materialize (one launch) -> reverse rows with the window flags, with the count kernel's
 // per-block partials in a.work).
-int launch_build(const BuildArgs& a, hipStream_t stream) {
+int launch_build(const BuildArgs& a, int64_t fused_atoms, hipStream_t stream) {
   FMD_REQUIRE(a.n > 0 && a.n < (int64_t(1) << 31) && a.e_cap > 0 && a.bmax > 0);
   FMD_REQUIRE(a.positions && a.inv_cell && a.cell && a.nbr && a.shifts && a.num);
   FMD_REQUIRE(a.ref_pos && a.ref_wraps && a.capacity_valid && a.work && a.frac && a.wrap_delta);
@@ -1251,7 +1254,7 @@ int launch_build(const BuildArgs& a, hipStream_t stream) {
   FMD_REQUIRE(a.max_disp && a.cand_valid && a.overflow && a.isolated);
   FMD_REQUIRE(!a.system_of || a.pad_images);
   FMD_REQUIRE(a.n_dummy >= 0 && (a.n_dummy == 0 || !a.system_of) && a.n + a.n_dummy < (int64_t(1) << 31));
-  if (a.n <= kSmallMaxAtoms) {
+  if (a.n <= fused_atoms) {
     hipLaunchKernelGGL(nl_build_small_kernel, dim3(1), dim3(kSmallThreads), 0, stream, a);
     FMD_CHECK_LAUNCH();
     return FMD_OK;
@@ -1414,7 +1417,7 @@ int fmd_nl_build(const void* positions, int32_t pos_is_f64, const float* inv_cel
               edge_index, edge_image, max_displacement, candidate_valid, overflow, isolated, line2, short_flags,
               edge_reverse, window_overflow, window_capacity, window_max_edges, window_max_isolated, window_stats,
               window_check_isolated};
-  return launch_build(a, stream);
+  return launch_build(a, kFusedAtoms, stream);
 }
 
 int fmd_nl_build_noalloc(const void* positions, int32_t pos_is_f64, const float* inv_cell, const float* cell,
@@ -1437,7 +1440,7 @@ int fmd_nl_build_noalloc(const void* positions, int32_t pos_is_f64, const float*
               n_dummy, system_of, pad_images, e_cap, work, frac, wrap_delta, wrapped_out, edge_counts, edge_offsets, center, neighbor, images, distances,
               edge_index, edge_image, max_displacement, candidate_valid, overflow, isolated, line2, short_flags,
               nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  return launch_build(a, stream);
+  return launch_build(a, kSmallMaxAtoms, stream);
 }
 
 // padded rows of a bucket workspace: rows [e_real, e_cap) become far self-loops of atom

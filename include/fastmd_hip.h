@@ -161,7 +161,8 @@ int fmd_nl_build(const void* positions, int32_t pos_is_f64, const float* inv_cel
  * It must not be called concurrently on one device: two calls whose kernels can overlap (on
  * streams the caller has not ordered, or from two host threads) overwrite each other's partials
  * and both return wrong edge offsets and flags, with no error reported. Calls on one stream, or
- * on streams ordered by events, are safe. */
+ * on streams ordered by events, are safe, and so are calls of at most 1 024 atoms, whose build (one
+ * workgroup) keeps its partials to itself. */
 #define FMD_NL_BUILD_NOALLOC_MAX_ATOMS (1 << 20)
 #define FMD_NL_BUILD_NOALLOC_SCRATCH 393218 /* fmd_nl_build_work_size(FMD_NL_BUILD_NOALLOC_MAX_ATOMS) */
 int fmd_nl_build_noalloc(const void* positions, int32_t pos_is_f64, const float* inv_cell, const float* cell,

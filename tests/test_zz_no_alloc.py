@@ -76,3 +76,40 @@ def test_noalloc_build_equals_the_build_with_a_work_buffer(device):
     status = _abi.load().fmd_nl_build_noalloc(*_noalloc_args(builder, moved, got, n_atoms=MAX_ATOMS + 1))
     assert status == ETOOLARGE
     assert "allocation-free" in _abi.load().fmd_error_string(status).decode()
+
+
+@pytest.mark.gpu
+def test_overlapping_calls_of_small_systems_keep_their_results(device):
+    """Up to 1 024 atoms the build shares nothing between calls: on streams that nothing orders, every call
+    gives what fmd_nl_build gives."""
+    import torch
+
+    from fastmd_amd import _abi
+    from fastmd_amd.graph.fixed_capacity_builder import FixedCapacityGraphBuilder
+
+    calls = []
+    for k, repeats in enumerate([(2, 2, 3), (1, 1, 13), (3, 3, 3), (4, 4, 4), (6, 6, 5), (6, 6, 5)]):
+        s = systems.perovskite(repeats)
+        n = s.n_atoms
+        builder = FixedCapacityGraphBuilder(cell=torch.tensor(s.cell, dtype=torch.float32),
+                                            atomic_numbers=torch.ones(n), u_capacity=9 * n + 64, t_capacity=0,
+                                            line_graph_cutoff=None, atom_graph_cutoff=6.0, candidate_cutoff=8.0,
+                                            padding=PaddingRule("far_self_loops"), device=device)
+        builder.build(torch.tensor(s.positions, device=device), rebuild_candidates=True)
+        moved = s.positions + np.random.default_rng(k).normal(0, 0.08, s.positions.shape)
+        moved = torch.tensor(moved, dtype=torch.float64, device=device)
+        before = {name: t.clone() for name, t in _outputs(builder).items()}
+        builder.build(moved, rebuild_candidates=False)
+        expected = {name: t.clone() for name, t in _outputs(builder).items()}
+        outs = [{name: t.clone() for name, t in before.items()} for _ in range(6)]
+        calls.append((builder, moved, expected, outs, torch.cuda.Stream()))
+    torch.cuda.synchronize()
+    for turn in range(6):
+        for builder, moved, _, outs, stream in calls:
+            with torch.cuda.stream(stream):
+                _abi.call("fmd_nl_build_noalloc", *_noalloc_args(builder, moved, outs[turn]))
+    torch.cuda.synchronize()
+    for builder, _, expected, outs, _ in calls:
+        for got in outs:
+            for name in expected:
+                assert torch.equal(got[name], expected[name]), (builder.n_real, name)
