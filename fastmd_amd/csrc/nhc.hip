@@ -14,6 +14,7 @@
 #pragma clang fp contract(off)
 
 #include "common.h"
+#include "nhc_math.h"
 
 namespace {
 
@@ -78,23 +79,10 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
-// a / b from r = 1 / b (rounded): the product, its remainder and one correction give the rounded quotient
-// (Markstein's theorem; away from overflow and underflow). A non-finite a keeps a * r.
-__device__ __forceinline__ double div_q(double a, double b, double r) {
-  const double q = a * r;
-  const double rem = fma(-q, b, a);
-  return rem == rem ? fma(rem, r, q) : q;
-}
-
-// exp(x). Below 2^-5 the Taylor polynomial of degree 9 (the next term is below 2^-71), summed in pairs and
-// added to 1 last: at most 0.51 units in the last place off.
+// exp(x), small arguments by exp_small
 __device__ __forceinline__ double exp_chain(double x) {
-  if (!__all(fabs(x) < 0.03125)) return exp(x);
-  const double x2 = x * x;
-  const double a = fma(x, 1.0 / 6, 0.5), b = fma(x, 1.0 / 120, 1.0 / 24);
-  const double c = fma(x, 1.0 / 5040, 1.0 / 720), d = fma(x, 1.0 / 362880, 1.0 / 40320);
-  const double lo = fma(x2, b, a), hi = fma(x2, d, c);
-  return 1.0 + fma(x2, fma(x2 * x2, hi, lo), x);
+  if (!__all(fabs(x) < kExpSmall)) return exp(x);
+  return exp_small(x);
 }
 
 // ASE _integrate_p_eta_j; j is a constant after unrolling, factor = exp(-delta/4 p_eta_{j+1} / Q_{j+1})

@@ -51,3 +51,33 @@ int main() {{
 }}
 """)
     assert out == "ok"
+
+
+def test_chain_exponential_and_quotient(tmp_path):
+    """exp_small over both signs against the 64-bit-mantissa exponential: within the bound its comment derives, 0.5 +
+    2^-6 + 2^-9 units in the last place; div_q: the rounded quotient."""
+    out = run_host(tmp_path, """
+#include <hip/hip_runtime.h>
+#include <cstdio>
+#include <random>
+#include "nhc_math.h"
+int main() {
+  std::mt19937_64 gen(1);
+  std::uniform_real_distribution<double> uniform(-kExpSmall, kExpSmall), power(-300, 300);
+  double worst[2] = {0, 0};  // below 0, above
+  for (int k = 0; k < 4000000; ++k) {
+    const double x = k == 0 ? -0x1.bd1823ee71d98p-6 : k % 4 == 0 ? uniform(gen) * 1e-3 : uniform(gen);
+    const long double off = fabsl((long double)exp_small(x) - expl((long double)x));
+    const double units = (double)(off * (x < 0 ? 0x1p53L : 0x1p52L));
+    if (units > worst[x >= 0]) worst[x >= 0] = units;
+  }
+  int wrong = 0;
+  for (int k = 0; k < 1000000; ++k) {
+    const double a = exp2(power(gen)) * uniform(gen), b = exp2(power(gen) / 2);
+    wrong += div_q(a, b, 1.0 / b) != a / b;
+  }
+  std::printf("%.6f %.6f %d", worst[0], worst[1], wrong);
+}
+""").split()
+    below, above, wrong = float(out[0]), float(out[1]), int(out[2])
+    assert 0.5 < max(below, above) <= 0.5 + 2.0 ** -6 + 2.0 ** -9 and wrong == 0
