@@ -270,10 +270,10 @@ def _assert_build_equal(builder, ob, cand=None):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_atoms", [135, 1080, 3430, 10000, 16875, 40000])
+@pytest.mark.parametrize("n_atoms", [40, 135, 1080, 3430, 10000, 16875, 40000])
 def test_builder_bit_exact(device, n_atoms):
     """Candidates, rows, flags and published buffers bit-exact vs the oracle, on the fused
-    single-workgroup path (<= 1024 atoms) and the multi-block path, fresh and with reused
+    single-workgroup path (40 atoms; up to 60) and the multi-block path, fresh and with reused
     candidates after seeded moves (wraps change, skin still valid)."""
     import torch
 
@@ -325,9 +325,9 @@ def test_builder_overflow_and_triclinic(device):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_atoms", [135, 3430])
+@pytest.mark.parametrize("n_atoms", [40, 135, 3430])
 def test_builder_minimum_image_bit_exact(device, n_atoms):
-    """minimum_image builds bit-exact vs the oracle on the single-workgroup and the multi-block
+    """minimum_image builds bit-exact vs the oracle on the single-workgroup (40 atoms) and the multi-block
     path, with atoms wrapped by lattice vectors since the refresh."""
     import torch
 
@@ -594,10 +594,11 @@ def _assert_line_equal(builder, b, lg):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_atoms,line_cutoff", [(135, 3.5), (1080, 3.0), (5000, 3.0), (5000, 3.5), (10000, 3.5)])
+@pytest.mark.parametrize("n_atoms,line_cutoff", [(40, 3.5), (135, 3.5), (1080, 3.0), (5000, 3.0), (5000, 3.5),
+                                                 (10000, 3.5)])
 def test_line_graph_builder_bit_exact(device, n_atoms, line_cutoff):
     """The HIP line graph (short-bond flags, undirected pairs, short lists, pair offsets, triplet
-    rows, flags) bit-exact vs the oracle on the fused (<= 1 024 atoms) and multi-block builds
+    rows, flags) bit-exact vs the oracle on the fused (40 atoms; up to 60) and multi-block builds
     (10 000 atoms: the pair scan's workgroup takes two passes of 8 192 atoms)."""
     import torch
 

@@ -168,12 +168,12 @@ def _gpu_builder(s, u_cap, kind, device, n_dummy=16, t_cap=0, line_cutoff=None):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_cells", [3, (6, 6, 6)])
+@pytest.mark.parametrize("n_cells", [2, 3, (6, 6, 6)])
 @pytest.mark.parametrize("kind", RULES)
 def test_edges_only_padding_rules_bit_exact(device, kind, n_cells):
     """Edges-only builds at the capacity boundary (edges above, equal to and 40 pairs below
     e_capacity; the last pads more rows than there are atoms, so the round robin wraps) on the
-    fused (135 atoms) and multi-block (1 080) paths: rows, published buffers, distances, sink
+    fused (40 atoms) and multi-block (135, 1 080) paths: rows, published buffers, distances, sink
     rows and override bit-exact vs the oracle; every index within the real and sink rows."""
     import torch
 
@@ -214,15 +214,17 @@ def test_edges_only_padding_rules_bit_exact(device, kind, n_cells):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_cells", [2, 3])
 @pytest.mark.parametrize("n_dummy", [0, 3])
-def test_line_graph_padding_and_overflow_topology_bit_exact(device, n_dummy):
+def test_line_graph_padding_and_overflow_topology_bit_exact(device, n_dummy, n_cells):
     """A line-graph builder with far self-loop or sink padding on the reference's boundary cases
     (one free pair, no free pair, triplets above t_capacity): pairs, triplets, flags and the
-    published rows (the all-padding topology on overflow) bit-exact vs the oracle."""
+    published rows (the all-padding topology on overflow) bit-exact vs the oracle, from the fused
+    (40 atoms) and the multi-block (135) build."""
     import torch
 
     print(f"[padding] line graph n_dummy={n_dummy}", flush=True)
-    s = systems.perovskite(3, sigma=0.1)
+    s = systems.perovskite(n_cells, sigma=0.1)
     n = s.n_atoms
     lc = 3.5
     b0, bmax = _oracle_build(s, 10 ** 6, line_cutoff=lc)

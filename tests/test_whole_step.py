@@ -70,14 +70,16 @@ def _state(md):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("model_name", ["morse", "mace_like", "threebody"])
-@pytest.mark.parametrize("steps_per_launch", [1, 5])
-def test_whole_step_equals_eager_bitwise(device, model_name, steps_per_launch):
+@pytest.mark.parametrize("steps_per_launch,n_cells", [(1, 3), (5, 3), (5, 2)])
+def test_whole_step_equals_eager_bitwise(device, model_name, steps_per_launch, n_cells):
+    """135 atoms (three-launch builds) and 40 (one workgroup, which folds the window's flags itself)."""
     import torch
 
-    print(f"[whole_step] {model_name} spl={steps_per_launch}", flush=True)
+    print(f"[whole_step] {model_name} spl={steps_per_launch} cells={n_cells}", flush=True)
     make = lambda: _adapter(model_name, device)  # noqa: E731
-    eager = _md(make(), "eager", device)
-    graph = _md(make(), "whole_step", device, steps_per_launch=steps_per_launch)
+    s = systems.perovskite(n_cells)
+    eager = _md(make(), "eager", device, system=s)
+    graph = _md(make(), "whole_step", device, steps_per_launch=steps_per_launch, system=s)
     assert torch.equal(_state(eager), _state(graph))
     eager.run(20)
     graph.run(20)
@@ -106,14 +108,15 @@ def test_whole_step_equals_eager_bitwise_configs3_sizes(device, k):
 
 
 @pytest.mark.gpu
-def test_whole_step_capacity_growth_and_refresh_paths(device):
-    """A tiny capacity step forces overflow -> growth -> recapture; a tiny skin forces candidate
+@pytest.mark.parametrize("n_cells", [3, 2])
+def test_whole_step_capacity_growth_and_refresh_paths(device, n_cells):
+    """On both forms of the build (135 and 40 atoms): a tiny capacity step forces overflow -> growth -> recapture; a tiny skin forces candidate
     refreshes and fallback windows. The trajectory stays the eager one, bitwise."""
     import torch
 
     from fastmd_amd.models.pair_potential import MorsePairAdapter
 
-    s = systems.perovskite(3)
+    s = systems.perovskite(n_cells)
     eager = _md(MorsePairAdapter(device=device), "eager", device, system=s)
     tight = CapacityConfig(u_step=1, min_pad_u=0, candidate_skin=0.05)
     graph = _md(MorsePairAdapter(device=device), "whole_step", device, steps_per_launch=2, capacity=tight, system=s)
