@@ -214,6 +214,7 @@ struct QueryArgs {
   uint8_t* capacity_valid;
   int64_t system_size;
   int64_t index_offset;
+  float full;  // (the sphere's volume / the share of the cell's cells within reach) / the wave form's keys
 };
 
 // The slots of atom i that a search writes, [0, end): its candidates and then the pad value, up to
@@ -318,23 +319,27 @@ __device__ __forceinline__ void query_atom(const QueryArgs& a, int64_t i, uint64
   }
 }
 
-// The workgroup form for every atom, or (SPARSE) for those whose candidates overflowed the wave form's
-// keys, 16 atoms per workgroup (all of them past it cost no more than a workgroup each).
+// The workgroup form for every atom, or (SPARSE) for those left over by the wave form, `per` atoms of a
+// workgroup in turn: at most 16, and few enough that kSparseGroups workgroups share them, since a slab or a cluster
+// in vacuum may hold nothing else. Slabs of 320 candidates per atom, refreshed: 4 000 atoms 1 190 us with 16 in
+// turn, 395 with one; 20 000 atoms 2 030 with 16, 1 640 with 9 (2 048 workgroups), 1 390 with 4. Workgroups with
+// nothing to do cost their launch (a crystal of 40 000 atoms 132 us with 16 in turn, 134 with 9).
 constexpr int kWaveKeys = 256;  // candidate keys of a wave
 constexpr int kSparseAtoms = 16;
+constexpr int64_t kSparseGroups = 4096;
 
 template <bool SPARSE>
-__global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a) {
+__global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a, int per) {
   extern __shared__ uint64_t keys[];
   if (!SPARSE) {
     query_atom(a, blockIdx.x, keys);
     return;
   }
-  const int64_t i0 = (int64_t)blockIdx.x * kSparseAtoms;
-  const int64_t mine = i0 + (threadIdx.x & (kSparseAtoms - 1));
-  const int count = mine < a.n ? a.num_neighbors[mine] : 0;
-  if (!__any(count > kWaveKeys)) return;  // every wave of the workgroup sees the same 16 counts
-  for (int k = 0; k < kSparseAtoms; ++k) {
+  const int64_t i0 = (int64_t)blockIdx.x * per;
+  const int mine = threadIdx.x & (kSparseAtoms - 1);
+  const int count = mine < per && i0 + mine < a.n ? a.num_neighbors[i0 + mine] : 0;
+  if (!__any(count > kWaveKeys)) return;  // every wave of the workgroup sees the same counts
+  for (int k = 0; k < per; ++k) {
     __syncthreads();  // keys and counter are free
     if (__shfl(count, k, FMD_WAVE) > kWaveKeys) query_atom(a, i0 + k, keys);
   }
@@ -344,9 +349,9 @@ __global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a) {
 // each lane finding its cell in the scanned counts, so that every lane tests an atom and the loads of
 // a pass go out together; candidate keys appended to the wave's LDS list by ballot. The list is put in
 // order by rank: a key's slot is the number of smaller keys (up to four keys per lane against the list,
-// read as LDS broadcasts), written straight to the row. More than kWaveKeys candidates: the count alone,
-// for the workgroup form. Bound by the latency of its loads (27 cells, 320 atoms per atom at 40 000):
-// 40 000 atoms 487 -> 65 us with the rows' unused slots no longer written.
+// read as LDS broadcasts), written straight to the row. More than kWaveKeys candidates, found or expected: the
+// search ends there, with a count above kWaveKeys for the workgroup form. Bound by the latency of its loads (27
+// cells, 320 atoms per atom at 40 000): 40 000 atoms 487 -> 65 us with the rows' unused slots no longer written.
 __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a) {
   __shared__ uint64_t s_keys[256 / FMD_WAVE][kWaveKeys];
   __shared__ int32_t s_first[256 / FMD_WAVE][FMD_WAVE];  // scanned atom counts of the wave's 64 cells
@@ -363,8 +368,11 @@ __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a
   const int c0 = cell_coord(a.frac[3 * i], a.n0), c1 = cell_coord(a.frac[3 * i + 1], a.n1),
             c2 = cell_coord(a.frac[3 * i + 2], a.n2);
   const int span1 = 2 * a.r1 + 1, span2 = 2 * a.r2 + 1, noff = (2 * a.r0 + 1) * span1 * span2;
+  const float volume = fabsf(cm.m[0] * (cm.m[4] * cm.m[8] - cm.m[5] * cm.m[7]) -
+                             cm.m[1] * (cm.m[3] * cm.m[8] - cm.m[5] * cm.m[6]) +
+                             cm.m[2] * (cm.m[3] * cm.m[7] - cm.m[4] * cm.m[6]));
   int count = 0;
-  for (int q0 = 0; q0 < noff; q0 += FMD_WAVE) {
+  for (int q0 = 0; q0 < noff && count <= kWaveKeys; q0 += FMD_WAVE) {
     const int q = q0 + lane;
     int from = 0, atoms = 0;
     uint32_t packed = 0;
@@ -394,7 +402,12 @@ __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const int total = __shfl(incl, FMD_WAVE - 1, FMD_WAVE);
-    for (int f0 = 0; f0 < total; f0 += FMD_WAVE) {
+    // cells so full that the sphere's share of them passes the keys: left to the workgroup form unsearched
+    if (noff <= FMD_WAVE && (float)total * a.full > volume) {
+      count = kWaveKeys + 1;
+      break;
+    }
+    for (int f0 = 0; f0 < total && count <= kWaveKeys; f0 += FMD_WAVE) {
       const int f = f0 + lane;
       bool hit = false;
       uint64_t key = 0;
@@ -459,7 +472,7 @@ __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a
   }
   if (lane == 0) {
     a.num_neighbors[i] = count;
-    if (count > a.bmax) a.capacity_valid[0] = 0;
+    if (fits && count > a.bmax) a.capacity_valid[0] = 0;  // else the workgroup form's to say
   }
 }
 
@@ -1363,20 +1376,27 @@ int fmd_nl_candidates_pad(const float* wrapped, const float* frac, const float* 
   FMD_CHECK_LAUNCH();
   QueryArgs a{wrapped, frac, cell, n_atoms, cutoff2, n0, n1, n2, r0, r1, r2, bmax, lcap, pad_mode, cell_start, cell_atoms,
               neighbor_matrix, neighbor_shifts, num_neighbors, capacity_valid, system_size, index_offset};
+  a.full = (float)(4.18879 * (double)cutoff2 * sqrt((double)cutoff2) * (double)ncell /
+                   ((2. * r0 + 1) * (2. * r1 + 1) * (2. * r2 + 1) * kWaveKeys));
   const size_t lds = (size_t)lcap * sizeof(uint64_t);
-  // A cell is at least the cutoff thick along each axis, so an atom has at most about 4.2 (the sphere in
-  // cutoffs cubed) times the mean atoms per cell as candidates. The wave form where three quarters of
-  // its keys hold that; rows past its keys (an inhomogeneous system) go to the workgroup form after it.
-  // The workgroup form alone where the mean row would: it searches such rows once.
-  if (4.19 * (double)n_atoms / (double)ncell <= 0.75 * kWaveKeys) {
+  // The wave form where three quarters of its keys hold a row at the mean density: the sphere has 4.19 cutoffs cubed,
+  // and a cell is at least 1 / reach of a cutoff thick along an axis of one cell, the cutoff along others. An upper
+  // bound at that density, since a cell is up to two cutoffs thick; the workgroup form above it, which searches
+  // a long row once (a bound without the reach sent 40 atoms in a 9 A cell, 404 candidates within 12 A, through
+  // both: 470 us, 46 now). Rows past the keys at a lower mean density go to the workgroup form after the wave form.
+  double row = 4.19 * (double)n_atoms / (double)ncell;
+  for (int k = 0; k < 3; ++k) row *= ncells[k] == 1 && reach[k] > 1 ? reach[k] : 1;
+  if (row <= 0.75 * kWaveKeys) {
     hipLaunchKernelGGL(cells_query_wave_kernel, dim3((unsigned)fmd_cdiv(n_atoms, 256 / FMD_WAVE)), dim3(256), 0, stream,
                        a);
     FMD_CHECK_LAUNCH();
     a.pad_mode = pad_mode == FMD_NL_PAD_NONE ? FMD_NL_PAD_NONE : FMD_NL_PAD_ALL;  // the old counts are gone
-    hipLaunchKernelGGL(cells_query_kernel<true>, dim3((unsigned)fmd_cdiv(n_atoms, kSparseAtoms)), dim3(256), lds, stream,
-                       a);
+    const int64_t per = n_atoms / kSparseGroups < 1 ? 1 : n_atoms / kSparseGroups < kSparseAtoms ? n_atoms / kSparseGroups
+                                                                                                : kSparseAtoms;
+    hipLaunchKernelGGL(cells_query_kernel<true>, dim3((unsigned)fmd_cdiv(n_atoms, per)), dim3(256), lds, stream, a,
+                       (int)per);
   } else {
-    hipLaunchKernelGGL(cells_query_kernel<false>, dim3((unsigned)n_atoms), dim3(256), lds, stream, a);
+    hipLaunchKernelGGL(cells_query_kernel<false>, dim3((unsigned)n_atoms), dim3(256), lds, stream, a, 1);
   }
   FMD_CHECK_LAUNCH();
   return FMD_OK;

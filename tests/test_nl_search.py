@@ -70,6 +70,52 @@ def test_dense_rows_take_the_workgroup_form(device):
         assert int(assert_rows(builder, positions, cell).min()) > 150
 
 
+@pytest.mark.parametrize("n,side,cutoff", [(5, 4.5, 11.0), (8, 4.0, 7.0), (40, 9.0, 11.0), (11, 9.0, 11.0)])
+def test_cells_thinner_than_the_cutoff(device, n, side, cutoff):
+    """One cell per axis searched over two images and more: rows above the wave form's keys from few atoms
+    (the first three), and below."""
+    cell = np.diag([side, side, side * 1.03])
+    builder = builder_of(cell, n, device, cutoff=cutoff, skin=1.0)
+    assert max(builder._reach) > 1
+    for seed in (0, 1):
+        positions = spread(n, cell, seed)
+        builder.refresh_candidates(torch.tensor(positions, device=device))
+        assert (int(assert_rows(builder, positions, cell).max()) > 256) == (n != 11)
+
+
+def test_slab_in_vacuum(device):
+    """A mean density of the wave form, rows of the workgroup form: left unsearched inside, ended early near the
+    surface; then over those rows a spread system and back."""
+    cell = np.diag([30.0, 30.0, 120.0])
+    n = 1700
+    builder = builder_of(cell, n, device, cutoff=8.0)
+    slab = np.diag([30.0, 30.0, 20.0])
+    for seed, box in ((0, slab), (1, cell), (2, slab)):
+        positions = spread(n, box, seed)
+        builder.refresh_candidates(torch.tensor(positions, device=device))
+        rows = assert_rows(builder, positions, cell)
+        assert rows.max() > 256 and rows.min() < 256 if box is slab else rows.max() <= 256
+
+
+def test_full_cells_with_short_rows_keep_the_capacity_flag(device):
+    """27 tight clusters within reach of each other's cells but not of the cutoff: more atoms in the cells than the
+    wave form expects to hold, rows that fit the slots."""
+    cell = np.eye(3) * 60.0
+    side = 60.0 / 7
+    centre = side * 3.5 + 12.0 * (np.stack(np.meshgrid(*[np.arange(3)] * 3, indexing="ij"), -1).reshape(-1, 3) - 1)
+    rng = np.random.default_rng(0)
+    positions = (centre[:, None] + rng.uniform(-0.2, 0.2, (27, 100, 3))).reshape(-1, 3)
+    n, slots = len(positions), 128
+    builder = builder_of(cell, n, device)
+    assert tuple(builder._ncells) == (7, 7, 7)
+    builder.buffer_max = slots
+    builder.neighbor_matrix = torch.full((n, slots), n, dtype=torch.int32, device=device)
+    builder.neighbor_shifts = torch.zeros((n, slots, 3), dtype=torch.int32, device=device)
+    builder.refresh_candidates(torch.tensor(positions, device=device))
+    assert int(assert_rows(builder, positions, cell).max()) == 99
+    assert bool(builder._candidate_capacity_valid.item())
+
+
 @pytest.mark.parametrize("skin,slots", [(0.5, 16), (2.0, 48)])
 def test_truncated_rows_of_the_wave_form(device, skin, slots):
     """More candidates than slots: the first in order, the flag cleared."""
