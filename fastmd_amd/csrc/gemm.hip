@@ -1615,6 +1615,22 @@ int fmd_gemm_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32
   return FMD_OK;
 }
 
+int fmd_gemm_f32_planes(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_layout, const float* bias,
+                        float* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int32_t accumulate,
+                        int32_t epilogue_kind, uint16_t* planes, hipStream_t stream) {
+  FMD_REQUIRE(m >= 0 && n >= 0 && k > 0 && k <= 65536 && c && ldc >= n && (b_layout == 0 || b_layout == 1));
+  FMD_REQUIRE(epilogue_kind == 0 || epilogue_kind == 1);
+  if (m == 0 || n == 0) return FMD_OK;
+  FMD_REQUIRE(a && b && planes && lda >= k && ldb >= (b_layout == 0 ? k : n));
+  const int32_t width = (int32_t)k;
+  const int status = b_layout == 0 ? fmd_split3_f32(b, ldb, n, width, planes, stream)
+                                   : fmd_split3_t_f32(b, ldb, k, n, planes, stream);
+  if (status != FMD_OK) return status;
+  const void* src = a;
+  return launch_gemm_x3p(0, 1, &src, nullptr, nullptr, &lda, &width, m, planes, 48 * fmd_cdiv(k, 16), k, nullptr,
+                         nullptr, 1, 0, bias, c, ldc, n, accumulate, epilogue_kind, stream);
+}
+
 int fmd_gemm_group_f32(int32_t count, const float* const* a, const int64_t* lda, const float* const* a2,
                        const int64_t* lda2, const int64_t* ksplit, const float* const* b, const int64_t* ldb,
                        int32_t b_layout, const float* const* bias, float* const* c, const int64_t* ldc,

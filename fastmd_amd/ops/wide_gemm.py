@@ -24,22 +24,44 @@ from fastmd_amd._device import require_cuda, rows_view, stream
 _EPILOGUES = {None: 0, "none": 0, "silu": 1}
 
 
-# A float32 gemm splits its B into the bf16 planes beforehand (one launch, about 11 us) and runs on the
-# split-plane kernel with fp32 A:
-# * b [K, N]: from 256 tiles of 128 x 128, as the b [N, K] kernel that splits both operands (the fp32
-#   MFMA form takes 2 217 us at [160 000, 1 024] x [1 024, 520], this one 1 060, 153 against 100 us with
+# A float32 gemm splits its B into the bf16 planes beforehand (one launch, about 4 us for a weight of some 1 000 x 1 000)
+# and runs on the split-plane kernel with fp32 A:
+# * b [K, N]: from 256 tiles of 128 x 128, as the b [N, K] kernel that splits both operands, where _planes_pay
+#   (the fp32 MFMA form takes 2 217 us at [160 000, 1 024] x [1 024, 520], this one 1 060, 153 against 100 us with
 #   10 000 rows; with 125 tiles, [16 000, 384] x [384, 128], 29 against 37);
-# * b [N, K]: from PLANES_MIN_WORK multiply-adds, where splitting B once instead of once per row tile
-#   saves more than the launch (1 110 against 985 us at [160 000, 520] x [520, 1 024], 265 against 260 with
-#   40 000 rows, 94 against 100 with 10 000).
+# * b [N, K]: from PLANES_MIN_WORK multiply-adds and PLANES_MIN_ROWS rows, where splitting B once instead of once per
+#   row tile saves more than the launch ([160 000, 520] x [520, 1 024] 1 110 against 985 us, [33 000, 1 024] x
+#   [1 024, 520] 261 against 232; with 2 200 rows of [., 4 096] x [4 096, 2 048] 314 against 342, with 9 600 899 against 906).
 PLANES_MIN_TILES = 256
 PLANES_MIN_WORK = 2 ** 34
+PLANES_MIN_ROWS = 16384
 
 
 def _takes_planes(m: int, n: int, k: int, b_layout: int) -> bool:
+    """Whether the split-plane form takes a float32 gemm of these sizes."""
     if k % 4 or k <= 16 or n <= 16 or k > 65536 or -(-m // 128) * -(-n // 128) < PLANES_MIN_TILES:
         return False
     return b_layout == 1 or m * n * k >= PLANES_MIN_WORK
+
+
+def _planes_pay(m: int, n: int, k: int, b_layout: int) -> bool:
+    """Whether it is the faster form there. b [K, N] (us, fp32 MFMA against planes): from 512 tiles, where the fp32 form
+    goes over to tiles of 128 x 128, always ([70 000, 20] x [20, 40] 30 / 14) but for the fewest rows, which the
+    split costs more than it saves ([100, 264] x [264, 70 000] 0.8 of the time, [300, 64] x [64, 32 768] 1.2 times it).
+    Between 256 and 511 tiles (64 x 64 there) the split's launch and a last column tile that is not whole blocks of
+    32 have to be earned: [32 836, K] x [K, 40] 8.4 / 12.5 at K = 20, 28.4 / 26.2 at 264; x [K, 136] 0.95 of the time at
+    K = 32, 1.11 at 48; x [K, 256] 1.16 at 20."""
+    if b_layout == 0:
+        return m >= PLANES_MIN_ROWS
+    tiles = -(-m // 128) * -(-n // 128)
+    if m < 256 or (m < 384 and tiles < 768):
+        return False
+    if tiles >= 512 or k >= 192:
+        return True
+    last = n % 128
+    if n % 32 and (32 < last < 64 or last > 96):  # a tile of its own width with idle columns in every row
+        return tiles >= 384 and n > 128
+    return k >= 48 or last == 0 or (tiles >= 384 and n > 32)
 
 
 def gemm(a: Tensor, b: Tensor, *, b_layout: int, bias: Tensor | None = None, out: Tensor | None = None,
@@ -71,11 +93,16 @@ def gemm(a: Tensor, b: Tensor, *, b_layout: int, bias: Tensor | None = None, out
     b, ldb = rows_view(b)
     if m == 0 or n == 0:
         return out
-    if name == "fmd_gemm_f32" and _takes_planes(m, n, k, b_layout) and lda % 4 == 0 and a.data_ptr() % 16 == 0:
-        return gemm_planes([(a, None)], split_planes(b, transpose=b_layout == 1), a_planes=False, out=out, bias=bias,
-                           accumulate=accumulate, epilogue=epilogue)
-    _abi.call(name, a.data_ptr(), lda, b.data_ptr(), ldb, b_layout, _abi.ptr(bias), out.data_ptr(),
-              out.stride(0) if m > 1 else n, m, n, k, 1 if accumulate else 0, _EPILOGUES[epilogue], stream())
+    args = (a.data_ptr(), lda, b.data_ptr(), ldb, b_layout, _abi.ptr(bias), out.data_ptr(),
+            out.stride(0) if m > 1 else n, m, n, k, 1 if accumulate else 0, _EPILOGUES[epilogue])
+    if (name == "fmd_gemm_f32" and _takes_planes(m, n, k, b_layout) and _planes_pay(m, n, k, b_layout)
+            and lda % 4 == 0 and a.data_ptr() % 16 == 0):
+        # one call for the split and the product: as two, a small product was bound by their host time (22 us of it;
+        # [32 768, 20] x [20, 128] 12 us in the fp32 form)
+        planes = torch.empty(n * -(-k // 16) * 48, dtype=torch.bfloat16, device=a.device)
+        _abi.call("fmd_gemm_f32_planes", *args, planes.data_ptr(), stream())
+    else:
+        _abi.call(name, *args, stream())
     return out
 
 

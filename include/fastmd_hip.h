@@ -472,6 +472,13 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
 int fmd_gemm_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_layout,
                  const float* bias, float* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
                  int32_t accumulate, int32_t epilogue, hipStream_t stream);
+/* The same product with B split into its bf16 planes first (either layout) and the split-plane kernel on fp32
+ * A: for many rows, and for b_layout 1, where the fp32 MFMA form is half as fast. planes: 48 N ceil(K / 16) uint16 of
+ * scratch, 16-byte aligned. A 16-byte aligned with lda and K multiples of 4, K at most 65 536 (FMD_EUNSUPPORTED
+ * otherwise, the split launched). */
+int fmd_gemm_f32_planes(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_layout,
+                        const float* bias, float* c, int64_t ldc, int64_t m, int64_t n, int64_t k,
+                        int32_t accumulate, int32_t epilogue, uint16_t* planes, hipStream_t stream);
 
 /* Up to four independent fmd_gemm_f32 problems of one b_layout in one launch (arrays of length
  * count, problem g: C_g = [A_g | A2_g] op(B_g) (+ bias_g) (+ C_g if accumulate_g)). A2_g (may be

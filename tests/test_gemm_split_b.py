@@ -38,6 +38,27 @@ def test_b_layout_1(m, n, k, form):
     assert float((got.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
 
 
+# either side of every line of the choice, by rows, tiles, K and the last column tile
+@pytest.mark.parametrize("m,n,k,b_layout,planes", [
+    (65600, 40, 20, 1, True), (65400, 40, 20, 1, False), (32700, 40, 188, 1, False), (32700, 40, 192, 1, True),
+    (16300, 136, 44, 1, False), (16300, 136, 48, 1, True), (16300, 256, 20, 1, True), (26000, 168, 20, 1, True),
+    (24300, 168, 64, 1, False), (24700, 160, 20, 1, True), (24000, 160, 20, 1, False), (49200, 24, 20, 1, False),
+    (255, 65536, 20, 1, False), (256, 49152, 20, 1, True), (383, 16384, 64, 1, False), (385, 16384, 64, 1, True),
+    (16384, 1024, 1028, 0, True), (16383, 1024, 1028, 0, False)])
+def test_choice_of_the_form(monkeypatch, m, n, k, b_layout, planes):
+    from fastmd_amd import _abi
+    from fastmd_amd.ops import wide_gemm
+
+    taken, call = [], _abi.call
+    monkeypatch.setattr(_abi, "call", lambda name, *args: (taken.append(name), call(name, *args))[1])
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=gen, device="cuda")
+    b = torch.randn(*((k, n) if b_layout else (n, k)), generator=gen, device="cuda")
+    got, want = wide_gemm.gemm(a, b, b_layout=b_layout), reference(a, b, b_layout)
+    assert taken == ["fmd_gemm_f32_planes" if planes else "fmd_gemm_f32"]
+    assert float((got.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
 def test_large_b_layout_0_equals_the_kernel_that_splits_both():
     """The same planes and K order: bitwise gemm_gather, which splits B in the kernel."""
     from fastmd_amd.ops import wide_gemm
