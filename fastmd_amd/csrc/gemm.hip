@@ -730,6 +730,85 @@ __device__ __forceinline__ void x3_finish(f32x16 (&acc)[MB][NB], const X3Part& r
   epilogue<MB, NB>(acc, row0, col0, m, n, bias, c, ldc, accumulate, act);
 }
 
+// The four values of a weight row (column of C) from k on: the sum of its planes.
+struct X3PlaneB {
+  const __bf16* b;
+  int64_t ld;
+  __device__ __forceinline__ float4 operator()(int64_t col, int64_t k) const {
+    const __bf16* e = b + col * ld + (k >> 4) * 48 + (k & 15);
+    const bf16x4 x = *reinterpret_cast<const bf16x4*>(e), y = *reinterpret_cast<const bf16x4*>(e + 16),
+                 z = *reinterpret_cast<const bf16x4*>(e + 32);
+    return make_float4((float)x[0] + ((float)y[0] + (float)z[0]), (float)x[1] + ((float)y[1] + (float)z[1]),
+                       (float)x[2] + ((float)y[2] + (float)z[2]), (float)x[3] + ((float)y[3] + (float)z[3]));
+  }
+};
+
+// One 32 x 32 block as fp32 products (v_mfma_f32_32x32x2_f32) straight from the operands: row and col are
+// this lane's operand rows; lane half h takes k = 8 u + 4 h .. + 4 of every group of 8.
+template <typename RowB>
+__device__ __forceinline__ f32x16 x3_block_f32(const X3Part& P0, const X3Part& P1, const X3Part& P2, int np,
+                                               const RowB& rowb, int64_t row, int64_t col, int h) {
+  f32x16 sum;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) sum[v] = 0.f;
+  int64_t base = 0;
+  for (int p = 0; p < np; ++p) {
+    const X3Part& P = p == 0 ? P0 : p == 1 ? P1 : P2;
+    const float* a = P.src + (P.idx ? (int64_t)P.idx[row * P.istride] : row) * P.ld;
+    for (int q0 = 0; q0 < P.width; q0 += 32) {
+      float4 x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = q0 + 8 * u + 4 * h;
+        const bool in = q < P.width;  // widths are multiples of 4
+        x[u] = in ? *reinterpret_cast<const float4*>(a + q) : make_float4(0.f, 0.f, 0.f, 0.f);
+        y[u] = in ? rowb(col, base + q) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u].x, y[u].x, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u].y, y[u].y, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u].z, y[u].z, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u].w, y[u].w, sum, 0, 0, 0);
+      }
+    }
+    base += P.width;
+  }
+  return sum;
+}
+
+// Elements of a finished tile that are NaN take the value of an fp32 product: a plane product cannot carry an
+// infinity (inf - inf in the split, inf * 0 between planes), so an operand that is infinite, or rounds to an
+// infinite bf16, shows as a NaN here. A block with a NaN is formed again whole, on the fp32 matrix cores;
+// outputs of finite operands never come here.
+template <int MB, int NB, typename RowB>
+__device__ __forceinline__ void x3_nonfinite(f32x16 (&acc)[MB][NB], const X3Part& P0, const X3Part& P1,
+                                             const X3Part& P2, int np, const RowB& rowb, int64_t m, int64_t n,
+                                             int64_t row0, int64_t col0, int h, int rr) {
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN if an element is NaN or infinite
+#pragma unroll
+  for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) zero[v & 3] = fmaf(acc[bi][bj][v], 0.f, zero[v & 3]);
+  const float all = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+  if (!__any(all != all)) return;
+#pragma unroll
+  for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj) {
+      bool nan = false;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) nan = nan || acc[bi][bj][v] != acc[bi][bj][v];
+      if (!__any(nan)) continue;
+      const f32x16 sum = x3_block_f32(P0, P1, P2, np, rowb, min(row0 + bi * 32 + rr, m - 1),
+                                      min(col0 + bj * 32 + rr, n - 1), h);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[bi][bj][v] = acc[bi][bj][v] != acc[bi][bj][v] ? sum[v] : acc[bi][bj][v];
+    }
+}
+
 // One 128 x BN tile of C at (row_blk, col_blk): A as up to three gathered column parts (K order
 // P0 | P1 | P2), B [N, K] K-contiguous, both split into their planes as they are staged. BN = 128:
 // waves 2 x 2, each 64 x 64 (MB = 2 blocks of 32 rows); BN = 64 (N <= 64, where a 128-wide tile
@@ -856,68 +935,12 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
         *reinterpret_cast<u32x4*>(sb_ + X3_OP + (t + j * kThreads) * 8) = pb##S[j];                  \
   } while (0)
 
-// Elements of a finished tile that are NaN, formed again as an fp32 FMA chain over the unsplit A and
-// B's planes added up: a plane product cannot carry an infinity (inf - inf in the split, inf * 0
-// between planes), so an operand that is infinite, or rounds to an infinite bf16, shows as a NaN
-// here and gets the value of an fp32 product; a sum that is NaN ends its chain. Outputs of finite
-// operands never come here.
-template <int MB, int NB>
-__device__ __forceinline__ void x3p_nonfinite(f32x16 (&acc)[MB][NB], const X3PPart& P0, const X3PPart& P1,
-                                              const X3PPart& P2, int np, const __bf16* __restrict__ bp, int64_t ldb,
-                                              int64_t m, int64_t n, int64_t k, int64_t row0, int64_t col0, int h,
-                                              int rr) {
-  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN if an element is NaN or infinite
-#pragma unroll
-  for (int bi = 0; bi < MB; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) zero[v & 3] = fmaf(acc[bi][bj][v], 0.f, zero[v & 3]);
-  const float all = (zero[0] + zero[1]) + (zero[2] + zero[3]);
-  if (!__any(all != all)) return;
-  uint64_t mask = 0;
-#pragma unroll
-  for (int bi = 0; bi < MB; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if (acc[bi][bj][v] != acc[bi][bj][v]) mask |= 1ull << ((bi * NB + bj) * 16 + v);
-  while (__any(mask != 0)) {
-    const int id = mask ? __ffsll((unsigned long long)mask) - 1 : -1;
-    float sum = 0.f;
-    if (id >= 0) {
-      const int v = id & 15, bj = (id >> 4) % NB, bi = (id >> 4) / NB;
-      const int64_t row = min(row0 + bi * 32 + (v / 4) * 8 + h * 4 + (v % 4), m - 1);
-      const int64_t col = min(col0 + bj * 32 + rr, n - 1);
-      const __bf16* b = bp + col * ldb;
-      int64_t kk = 0;
-      for (int p = 0; p < np && sum == sum; ++p) {
-        const X3PPart& P = p == 0 ? P0 : p == 1 ? P1 : P2;
-        const float* a = static_cast<const float*>(P.src) + (P.idx ? (int64_t)P.idx[row * P.istride] : row) * P.ld;
-        for (int q = 0; q < P.width && kk < k && sum == sum; ++q, ++kk) {
-          const __bf16* e = b + (kk >> 4) * 48 + (kk & 15);
-          sum = fmaf(a[q], (float)e[0] + ((float)e[16] + (float)e[32]), sum);
-        }
-      }
-    }
-#pragma unroll
-    for (int bi = 0; bi < MB; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          acc[bi][bj][v] = (bi * NB + bj) * 16 + v == id ? sum : acc[bi][bj][v];
-    mask &= mask - 1;
-  }
-}
-
 // One (32 MB WM) x BN tile with fp32 A and B's planes, in `lds` (2 X3_BUF elements). BN = 128: waves
 // 2 x 2 (WM = 2), each 32 MB x 64; BN = 64 or 32: waves 4 x 1 (WM = 4, MB = 1), each 32 x BN: the last
 // column tile of an N that is not a multiple of 128 (K = 2F + 8 as the output width of an input
 // gradient leaves 8 columns, of which a 128-wide tile would compute 120 for nothing: 160 000 rows, N = 136,
 // 264, 520 with K = 256, 512, 1 024: 125, 357, 1 132 -> 110, 315, 1 060 us; a narrow tile still stages all of
-// A). FIX: form NaN elements again (x3p_nonfinite). Two register stages
+// A). FIX: form NaN elements again (x3_nonfinite). Two register stages
 // (loads issued two slices ahead) measured no faster than one at two waves per SIMD instead of
 // three, so the tile keeps one stage: slice kt + 1 is stored into LDS and slice kt + 2 loaded into
 // the stage while the MFMAs of slice kt run.
@@ -980,7 +1003,12 @@ __device__ __forceinline__ void x3p_tile(__bf16* lds, const X3PPart& P0, const X
     __syncthreads();  // buffer cur is free, buffer cur ^ 1 is complete
   }
   const int64_t row0 = row_blk + wm * 32 * MB, col0 = col_blk + wn * 32 * NB;
-  if constexpr (FIX) x3p_nonfinite<MB, NB>(acc, P0, P1, P2, np, bp, ldb, m, n, k, row0, col0, h, rr);
+  if constexpr (FIX) {
+    const auto part = [](const X3PPart& P) {
+      return X3Part{static_cast<const float*>(P.src), P.idx, P.ld, P.istride, P.width};
+    };
+    x3_nonfinite<MB, NB>(acc, part(P0), part(P1), part(P2), np, X3PlaneB{bp, ldb}, m, n, row0, col0, h, rr);
+  }
   x3_finish<MB, NB>(acc, radd, bias, c, ldc, m, n, accumulate, act, row0, col0, h, rr);
 }
 

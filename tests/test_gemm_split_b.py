@@ -93,3 +93,34 @@ def test_non_finite_operands_follow_the_fp32_product(n):
     assert float((got - want)[fine].abs().max()) <= 1e-5 * float(want[fine].abs().max())
     big = torch.isfinite(want) & ~fine
     assert float(((got - want)[big] / want[big]).abs().max()) <= 1e-5
+
+
+def test_infinities_in_every_row():
+    """A blown-up input: every output element that is not finite is what float64 says, and the product is formed within
+    20 times the time of a finite one (blocks of it are formed twice; element by element it took several hundred)."""
+    from fastmd_amd.ops import wide_gemm
+
+    m, n, k = 65600, 128, 512
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    a, b = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(k, n, generator=gen, device="cuda")
+    bad = a.clone()
+    bad[torch.arange(m), torch.arange(m) % k] = float("inf")
+    bad[::5, 3] = float("-inf")
+    want, got = reference(bad, b, 1), wide_gemm.gemm(bad, b, b_layout=1).double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()]) and bool(want.isnan().any()) and bool(want.isinf().any())
+
+    def best(x):
+        out, times = torch.empty(m, n, device="cuda"), []
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            wide_gemm.gemm(x, b, b_layout=1, out=out)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    finite, blown = best(a), best(bad)
+    print(f"[infinities] finite {finite * 1e3:.0f} us, blown up {blown * 1e3:.0f} us", flush=True)
+    assert blown <= 20 * finite
