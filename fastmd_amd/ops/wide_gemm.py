@@ -66,7 +66,14 @@ def _planes_pay(m: int, n: int, k: int, b_layout: int) -> bool:
 
 def gemm(a: Tensor, b: Tensor, *, b_layout: int, bias: Tensor | None = None, out: Tensor | None = None,
          accumulate: bool = False, epilogue: str | None = None) -> Tensor:
-    """``a @ op(b) (+ bias) (+ out)``: op(b) = b^T for b_layout 0 (b [N, K]), b for 1 (b [K, N])."""
+    """``a @ op(b) (+ bias) (+ out)``: op(b) = b^T for b_layout 0 (b [N, K]), b for 1 (b [K, N]).
+
+    float32 has three forms, chosen by the sizes, so a row's last bits depend on how many rows the call has: fp32
+    matrix instructions; planes split beforehand (``_planes_pay``); and, for b [N, K] from 256 tiles of 128 x 128
+    otherwise, planes split in the kernel. A plane product keeps an operand's 24 bits down to magnitudes of about
+    2^-110 (its third plane is below bf16's range there: 16 bits at 2^-118). In the first two forms an infinity gives what
+    float64 gives; the third returns NaN for an operand that rounds to an infinite bf16 (its check cost
+    products of 256 tiles 3 to 6 %)."""
     require_cuda(a, b, bias, out)
     if a.dim() != 2 or b.dim() != 2:
         raise ValueError("gemm takes 2-D operands")
@@ -353,7 +360,8 @@ def gemm_planes(parts, b: Planes, *, a_planes: bool, out: Tensor | None = None, 
     """``gemm_gather`` with pre-split operands (fmd_gemm_x3_planes_f32): ``b`` the planes of the
     K-contiguous weight [N, K] (``split_planes(w)``), ``parts`` a list of up to three
     ``(src, index)`` with ``src`` Planes (``a_planes``) or float32 [rows, width]. Bitwise equal to
-    ``gemm_gather`` on the unsplit operands."""
+    ``gemm_gather`` on the unsplit operands where these round to finite bf16; with float32 parts an infinity
+    (or a value that rounds to one) gives what an fp32 product gives, in ``gemm_gather`` and with ``a_planes`` a NaN."""
     if not 1 <= len(parts) <= 3:
         raise ValueError("gemm_planes takes one to three parts")
     require_cuda(b.data, out, bias)
@@ -524,7 +532,7 @@ class _Linear(Function):
 def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, precision=None, parts=()) -> Tensor:
     """``F.linear(x, weight, bias)`` on the MFMA kernels (x 2-D float32). ``precision`` and
     ``parts`` are accepted for signature parity; there is one precision, fp32-accurate (fp32
-    MFMA, or three bf16 planes per operand for the large K-contiguous shapes)."""
+    MFMA, or three bf16 planes per operand for the large shapes of either layout, see ``gemm``)."""
     if x.dim() != 2:
         shape = x.shape
         return linear(x.reshape(-1, shape[-1]), weight, bias).reshape(*shape[:-1], weight.shape[0])
@@ -532,8 +540,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None = None, precision=None
 
 
 def linear_into(out: Tensor, x: Tensor, weight: Tensor, bias: Tensor | None = None, rows: int | None = None):
-    """``out[:] = x @ weight^T (+ bias)`` (no autograd); ``rows`` is accepted for parity (a row chunk
-    takes the same kernel as the whole GEMM, so the rows are equal either way)."""
+    """``out[:] = x @ weight^T (+ bias)`` (no autograd); ``rows`` is accepted for parity (the GEMM is never cut)."""
     with torch.no_grad():
         return gemm(x, weight, b_layout=0, bias=bias, out=out)
 

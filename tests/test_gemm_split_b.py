@@ -70,13 +70,14 @@ def test_large_b_layout_0_equals_the_kernel_that_splits_both():
     assert torch.equal(wide_gemm.gemm(a, b, b_layout=0), wide_gemm.gemm_gather([(a, None)], b))
 
 
-@pytest.mark.parametrize("n", [128, 136])
-def test_non_finite_operands_follow_the_fp32_product(n):
+# b [K, N] and, from 2^34 multiply-adds, b [N, K] through the planes; both in the fp32 form below 256 tiles
+@pytest.mark.parametrize("n,m,k,b_layout", [(128, 32700, 64, 1), (136, 32700, 64, 1), (520, 33000, 1024, 0),
+                                            (136, 2000, 64, 0), (136, 2000, 64, 1)])
+def test_non_finite_operands_follow_the_fp32_product(n, m, k, b_layout):
     """Infinities, NaN and values that round to an infinite bf16 give what float64 gives (an infinity
     kept, inf - inf and inf * 0 NaN), and leave the other rows and columns alone."""
     from fastmd_amd.ops import wide_gemm
 
-    m, k = 32700, 64
     gen = torch.Generator(device="cuda").manual_seed(2)
     a, b = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(k, n, generator=gen, device="cuda")
     b[:, 3] = b[:, 3].to(torch.bfloat16).float()  # its lower planes are zero
@@ -85,14 +86,57 @@ def test_non_finite_operands_follow_the_fp32_product(n):
     a[5, 7], a[6, 7], a[6, 9], a[7, 1], a[8, 2] = float("inf"), float("inf"), float("-inf"), float("nan"), 3.4e38
     b[4, n - 1], b[5, n - 2] = float("inf"), 3.4e38
     a[9, 4] = 0.0  # times that infinity
-    want = reference(a, b, 1)
-    got = wide_gemm.gemm(a, b, b_layout=1).double()
+    b = b if b_layout else b.t().contiguous()
+    assert wide_gemm._takes_planes(m, n, k, b_layout) == (m > 2000)
+    want = reference(a, b, b_layout)
+    got = wide_gemm.gemm(a, b, b_layout=b_layout).double()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
     assert torch.equal(got[got.isinf()], want[want.isinf()])
     fine = torch.isfinite(want) & (want.abs() < 1e30)
     assert float((got - want)[fine].abs().max()) <= 1e-5 * float(want[fine].abs().max())
     big = torch.isfinite(want) & ~fine
     assert float(((got - want)[big] / want[big]).abs().max()) <= 1e-5
+
+
+def test_non_finite_gathered_parts():
+    """Rows gathered from two sources and K in three parts: an infinity in each, the rows that gather them and no other."""
+    from fastmd_amd.ops import wide_gemm
+
+    m, n = 33000, 136
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, y, z = (torch.randn(r, w, generator=gen, device="cuda") for r, w in ((700, 48), (900, 16), (m, 20)))
+    w = torch.randn(n, 84, generator=gen, device="cuda")
+    x[5, 7], y[11, 3], z[17, 19] = float("inf"), float("-inf"), float("nan")
+    i, j = (torch.randint(0, r, (m,), generator=gen, device="cuda", dtype=torch.int32) for r in (700, 900))
+    want = reference(torch.cat([x[i.long()], y[j.long()], z], 1), w, 0)
+    parts = [(x, i), (y, j), (z, None)]
+    got = wide_gemm.gemm_planes(parts, wide_gemm.split_planes(w), a_planes=False).double()
+    fine = torch.isfinite(want)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()]) and bool(got.isinf().any())
+    # split in the kernel: not finite in the same places, the same values elsewhere
+    inside = wide_gemm.gemm_gather(parts, w).double()
+    assert torch.equal(torch.isfinite(inside), fine)
+    for x in (got, inside):
+        assert float((x - want)[fine].abs().max()) <= 1e-5 * float(want[fine].abs().max())
+
+
+# the third plane of an operand of 2^e has a step of 2^-133 (bf16's smallest): 24 bits down to e = -110, 24 - 8 from
+# there to -118; the fp32 form keeps 24 down to fp32's own range
+@pytest.mark.parametrize("exponent,bits", [(-100, 24), (-110, 24), (-118, 16)])
+def test_small_operands(exponent, bits):
+    from fastmd_amd.ops import wide_gemm
+
+    m, n, k = 33000, 256, 64
+    assert wide_gemm._takes_planes(m, n, k, 1) and wide_gemm._planes_pay(m, n, k, 1)
+    gen = torch.Generator(device="cuda").manual_seed(-exponent)
+    a = (1.0 + torch.rand(m, k, generator=gen, device="cuda")) * 2.0 ** exponent
+    b = 1.0 + torch.rand(k, n, generator=gen, device="cuda")
+    want = reference(a, b, 1)
+    worst = float(((wide_gemm.gemm(a, b, b_layout=1).double() - want) / want).abs().max())
+    print(f"[small operands] 2^{exponent}: {worst:.2e}", flush=True)
+    # positive terms: the operand's own error plus K roundings of the sum
+    assert worst <= 2.0 ** -(bits - 1) + k * 2.0 ** -24
 
 
 def test_infinities_in_every_row():
