@@ -7,7 +7,7 @@
 // Nothing here depends on the order in which waves run: the counters hold integer counts, and a
 // row's place is its digit's base plus its rank among the rows before it.
 //   * up to kSmallRows rows: one workgroup per index sorts (key, row) pairs in LDS and searches
-//     every segment's offset there: one launch;
+//     every segment's offset there: one launch (two above kSmallSegments segments: the search then has the chip);
 //   * above: per pass a histogram launch and a scatter launch over at most 256 contiguous chunks
 //     (each scatter workgroup sums the chunk histograms itself, so there is no scan launch), then
 //     one search per segment over the sorted keys. Up to two indices share the launches.
@@ -32,6 +32,9 @@ constexpr int kMaxChunks = 256;             // workgroups of a histogram / scatt
 constexpr int kChunkRows = 1024;            // rows from which another chunk is added
 constexpr int kGroups = 4;                  // rows per thread whose loads are issued together
 constexpr int kSmallRows = 8192;
+// The one workgroup searches 1 024 offsets in 0.7 us, another launch costs about 5: 1 000 rows in 3 000 000 segments
+// 2 240 us in it.
+constexpr int64_t kSmallSegments = 8192;
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / FMD_WAVE;
 
@@ -272,8 +275,11 @@ __global__ void __launch_bounds__(kSmallThreads) csr_small_kernel(const Jobs job
     __syncthreads();
   }
   const int fin = j.passes & 1;
-  for (int r = t; r < rows; r += kSmallThreads) j.perm[r] = s_row[fin][r];
-  if (j.off)
+  for (int r = t; r < rows; r += kSmallThreads) {
+    j.perm[r] = s_row[fin][r];
+    if (j.key[0]) j.key[0][r] = s_key[fin][r];  // csr_offsets_kernel follows
+  }
+  if (j.off && !j.key[0])
     for (int64_t s = t; s <= j.nseg; s += kSmallThreads) j.off[s] = lower_bound(s_key[fin], rows, (uint32_t)s);
 }
 
@@ -331,9 +337,20 @@ int fmd_csr_from_index(int32_t count, const void* const* index, const int32_t* i
     nseg = num_segment[q] > nseg ? num_segment[q] : nseg;
   }
   if (small) {
+    const bool search = nseg > kSmallSegments && work[0] && work[count - 1];
+    for (int q = 0; search && q < count; ++q) jobs.j[q].key[0] = jobs.j[q].key[1] = work[q];
     hipLaunchKernelGGL(csr_small_kernel, dim3(1, (unsigned)count), dim3(kSmallThreads), 0, stream, jobs);
     FMD_CHECK_LAUNCH();
-    return checked ? (int)hipEventRecord(checked, stream) : FMD_OK;
+    if (checked) {
+      const hipError_t err = hipEventRecord(checked, stream);
+      if (err != hipSuccess) return (int)err;
+    }
+    if (search) {
+      hipLaunchKernelGGL(csr_offsets_kernel, dim3((unsigned)fmd_cdiv(nseg + 1, kThreads), (unsigned)count),
+                         dim3(kThreads), 0, stream, jobs);
+      FMD_CHECK_LAUNCH();
+    }
+    return FMD_OK;
   }
   for (int q = 0; q < count; ++q) {
     FMD_REQUIRE(work[q]);

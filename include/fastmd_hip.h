@@ -448,8 +448,8 @@ int fmd_segsum_csr_t_f32(const float* gout, int64_t ld_gout, const float* value,
  * if some index is negative; `checked` (may be null) is recorded on the stream once every index
  * has been read, so the caller can refuse the call without waiting for the rest of it.
  * work[q]: fmd_csr_work_size(rows) uint32 of scratch (nothing in it has to be set). One launch
- * for at most 8192 rows per index, else two per 8 bits of num_segment and one for the offsets,
- * shared by both indices.
+ * for at most 8192 rows per index (two above 8192 segments), else two per 8 bits of num_segment
+ * and one for the offsets, shared by both indices.
  * Replaces the sort and counts behind the segment layouts of a plain index
  * (fastmd/engine/dispatch.py:604-630). */
 int64_t fmd_csr_work_size(int64_t rows);

@@ -17,7 +17,8 @@ def stable_csr(index, num_segment):
 # one workgroup up to 8192 rows; chunks of 1024 rows above, at most 256 of them (the largest case);
 # one pass of 8 bits up to 255 segments, then two and three
 @pytest.mark.parametrize("rows,num_segment", [(0, 5), (1, 1), (64, 255), (1023, 256), (2049, 3), (8192, 65536),
-                                              (8193, 1), (8193, 255), (30011, 256), (65537, 65536), (300007, 70001)])
+                                              (8193, 1), (8193, 255), (30011, 256), (65537, 65536), (300007, 70001),
+                                              (0, 20000), (1, 8192), (1, 8193), (1000, 300007)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("kind", ["random", "sorted", "few"])
 def test_csr_is_the_stable_order(rows, num_segment, dtype, kind):
@@ -36,7 +37,7 @@ def test_csr_is_the_stable_order(rows, num_segment, dtype, kind):
     assert sorted(csr.perm.cpu().numpy().tolist()) == list(range(rows))
 
 
-@pytest.mark.parametrize("rows", [(40, 9000), (9000, 40), (12000, 9000)])
+@pytest.mark.parametrize("rows", [(40, 9000), (9000, 40), (12000, 9000), (40, 8000)])
 def test_two_indices_share_the_launches(rows):
     from fastmd_amd.ops.csr_segment_sum import csr_from_segments, refuse_negative
 
