@@ -37,6 +37,16 @@ def test_csr_is_the_stable_order(rows, num_segment, dtype, kind):
     assert sorted(csr.perm.cpu().numpy().tolist()) == list(range(rows))
 
 
+def test_more_chunks_from_2_24_rows():
+    from fastmd_amd.ops.csr_segment_sum import csr_from_segment
+
+    rows, num_segment = 2 ** 24 + 7, 1_000_003
+    index = np.random.default_rng(0).integers(0, num_segment + 10, rows).astype(np.int32)
+    perm, off = stable_csr(index, num_segment)
+    csr = csr_from_segment(torch.tensor(index, device="cuda"), num_segment)
+    assert np.array_equal(csr.off.cpu().numpy(), off) and np.array_equal(csr.perm.cpu().numpy()[:off[-1]], perm)
+
+
 @pytest.mark.parametrize("rows", [(40, 9000), (9000, 40), (12000, 9000), (40, 8000)])
 def test_two_indices_share_the_launches(rows):
     from fastmd_amd.ops.csr_segment_sum import csr_from_segments, refuse_negative
