@@ -56,10 +56,7 @@ SIGNATURES: dict[str, tuple] = {
                                             _i32, _p]),
     "fmd_tb_gated_sum_bwd_f32": (ctypes.c_int, [_p, _i64, _p, _i64, _i64, _i32, _p, _i64, _p, _p, _i64, _p, _i64,
                                                 _f32, _p, _i64, _p, _i64, _p, _i64, _i32, _p]),
-    "fmd_tb_bond_sum_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _p, _p, _p, _p, _i64, _i64, _f32, _p, _i64, _p]),
     "fmd_tb_triplet_bwd_f32": (ctypes.c_int, [_p, _i64, _p, _i64, _i32, _p, _p, _p, _i64, _i64, _f32, _p, _i64, _p,
-                                              _p]),
-    "fmd_tb_bond_reduce_f32": (ctypes.c_int, [_p, _i64, _i32, _p, _p, _p, _p, _p, _i64, _i64, _p, _i64, _p, _i32,
                                               _p]),
     "fmd_tb_bond_update_f32": (ctypes.c_int, [_p, _p, _i64, _p, _i64, _p, _i64, _i32, _p, _p, _p, _p, _p, _i64, _i64,
                                               _f32, _p, _i64, _p, _i64, _p]),
@@ -205,11 +202,11 @@ def ptr(tensor) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    """torch's current HIP stream (the stream every entry point launches on). For the current or an
-    indexed device, and with torch's GPU state up in this process, its raw handle: 0.15 us, where the stream object, made for every
-    launch, takes 2.7 in a loop and 20 between other work (with the pooled flags of the index checks:
-    gather-cat and its VJP at 160 000 rows 222 -> 150 us, the Fourier basis and its VJP 213 -> 115, a
-    135-atom block 419 -> 260)."""
+    """torch's current HIP stream (the stream every entry point launches on). For the current or an indexed
+    device, and with torch's GPU state up in this process, its raw handle: 0.15 us, where the stream object, made for
+    every launch, takes 2.7 in a loop and up to 20 between other work (it and the pooled flags of the index checks
+    took 50 to 70 us off a gather-cat with its VJP, about 100 off the Fourier basis with its own and off a
+    135-atom block, by the box)."""
     if torch.cuda.is_initialized():
         if device is None:
             return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

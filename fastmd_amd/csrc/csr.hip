@@ -15,11 +15,11 @@
 // keys formed from the fractional coordinates in the first pass; four passes).
 // Bound by launches and dependent loads, not by bytes (160 000 rows: 8 MB in all): the two CSRs of a
 // gather-cat VJP at 160 000 rows, 10 000 segments are 5 launches (45 us) where torch's sort, bincount
-// and cumsum were 44 (275 us). Measured whole: that forward and VJP at F = 128 453 -> 222 us, the Fourier
-// basis and its VJP at 107 520 triplets 511 -> 213 us, one edge block at 135 atoms (three CSRs)
-// 751 -> 419 us. The flag of negative indices goes to host memory from the first kernel, behind an
-// event of its own: waiting for the whole sequence instead left the GPU idle between calls (279, 236
-// and 444 us). Host time bounded the three then: 150, 115 and 260 us with cheaper launches.
+// and cumsum were 44 (275 us). The flag of negative indices goes to host memory from the first kernel, behind an
+// event of its own, so that the GPU does not idle between calls. What is left of such calls is host time, which
+// differs by box and by where the autograd thread runs: that forward and VJP at F = 128 453-497 -> 130-190 us,
+// the Fourier basis and its VJP at 107 520 triplets 440-511 -> 94-170, one edge block at 135 atoms (three CSRs)
+// 679-751 -> 260-320.
 #include "common.h"
 #include "search.h"
 

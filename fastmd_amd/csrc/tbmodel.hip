@@ -368,16 +368,16 @@ constexpr int kRunBatch = 4;
 
 // The pre-activation of a triplet from its bonds' and its atom's rows: z3[k] = u[b1] + v[b2] + h[atom] + aw[k].
 struct TripletTerms {
-  const float* u;  // [e_cap] rows (bond rows only), row stride ldu; null: z3 is given
+  const float* u;  // [e_cap] rows (bond rows only), row stride ldu
   const float* v;
   const float* h;   // [n] rows, row stride ldh
   const float* aw;  // [t_cap] rows, row stride lda
   int64_t ldu, ldh, lda;
 };
 
-// eps[b] += scale * sum over b's triplets (first bond), in order, of silu(z3[k]) s_b s_b2. FORM: z3 is
-// formed here from its four rows and stored for the VJP, else read.
-template <int NC, bool FORM>
+// eps[b] += scale * sum over b's triplets (first bond), in order, of silu(z3[k]) s_b s_b2; z3 is formed here
+// from its four rows and stored for the VJP.
+template <int NC>
 __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, float* z3, int64_t ldz, int C,
                                                            const TripletTerms tt, const float* geo, float scale,
                                                            float* eps, int64_t lde) {
@@ -400,26 +400,23 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, float* z3,
     const int bq = __shfl(bs.b, qs, 64);
     const int b2 = empty ? bq : b2raw;  // an empty run's slots read the bond's own rows and add nothing
     float ub[U][NC];
-    if constexpr (FORM) {
-      const int atom_l = empty ? 0 : lc.line[5 * ks];
+    const int atom_l = empty ? 0 : lc.line[5 * ks];
 #pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int64_t at = lane_int(atom_l, q * TQ);
+    for (int q = 0; q < U; ++q) {
+      const int64_t at = lane_int(atom_l, q * TQ);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc)
-          ub[q][cc] = tt.u[bs.bond(q) * tt.ldu + cols.col[cc]] + tt.h[at * tt.ldh + cols.col[cc]];
-      }
+      for (int cc = 0; cc < NC; ++cc)
+        ub[q][cc] = tt.u[bs.bond(q) * tt.ldu + cols.col[cc]] + tt.h[at * tt.ldh + cols.col[cc]];
     }
 #pragma unroll
     for (int q = 0; q < U; ++q)
 #pragma unroll
       for (int t = 0; t < TQ; ++t) {
         const int64_t k = lane_int((int)ks, q * TQ + t);
-        const int64_t r2 = FORM ? lane_int(b2, q * TQ + t) : 0;
+        const int64_t r2 = lane_int(b2, q * TQ + t);
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc)
-          x[q][t][cc] = FORM ? tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]]
-                             : z3[k * ldz + cols.col[cc]];
+          x[q][t][cc] = tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]];
       }
     const float w1 = geo[8 * (int64_t)bq + 6];
     const float ws = w1 * geo[8 * (int64_t)b2 + 6];
@@ -434,8 +431,8 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, float* z3,
         const float w = lane_value(ws, q * TQ + t);
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) {
-          const float z = FORM ? x[q][t][cc] + ub[q][cc] : x[q][t][cc];
-          if (FORM && t < cnt && bs.stored(q) && cols.live[cc])
+          const float z = x[q][t][cc] + ub[q][cc];
+          if (t < cnt && bs.stored(q) && cols.live[cc])
             z3[(int64_t)lane_int((int)ks, q * TQ + t) * ldz + cols.col[cc]] = z;
           const float v = z * tb_sigmoid(z) * w;
           acc[cc] = t < cnt ? acc[cc] + v : acc[cc];
@@ -454,15 +451,14 @@ __global__ void __launch_bounds__(256) tb_bond_sum_kernel(LineCsr lc, float* z3,
           wy[t] = w1q * geo[8 * r2 + 6];
 #pragma unroll
           for (int cc = 0; cc < NC; ++cc)
-            y[t][cc] = FORM ? tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]]
-                            : z3[k * ldz + cols.col[cc]];
+            y[t][cc] = tt.aw[k * tt.lda + cols.col[cc]] + tt.v[r2 * tt.ldu + cols.col[cc]];
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
           for (int cc = 0; cc < NC; ++cc) {
-            const float z = FORM ? y[t][cc] + ub[q][cc] : y[t][cc];
-            if (FORM && t < m && bs.stored(q) && cols.live[cc]) z3[(k0 + t) * ldz + cols.col[cc]] = z;
+            const float z = y[t][cc] + ub[q][cc];
+            if (t < m && bs.stored(q) && cols.live[cc]) z3[(k0 + t) * ldz + cols.col[cc]] = z;
             const float v = z * tb_sigmoid(z) * wy[t];
             acc[cc] = t < m ? acc[cc] + v : acc[cc];
           }
@@ -549,27 +545,21 @@ __global__ void __launch_bounds__(256) tb_triplet_bwd_kernel(LineCsr lc, const f
   }
 }
 
-// Per bond b: geps[b] += sum over b's triplets as first bond of ga3[k, 0:C], then as second bond
-// of ga3[k, C:2C]; gs[b] (+)= the same sums of gsw[k, 0] and gsw[k, 1] (stored, or added with
-// acc_gs). A second-bond slot of -1 (no triplet) adds zeros. SPLIT: ga3 is [t_cap, C] (the gradient of
-// z3), and its two sums are stored side by side, geps[b, 0:C] (first bond) and geps[b, C:2C] (second).
-template <int NC, bool SPLIT>
-__device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3, int64_t lda, int C, const float* gsw,
-                                            float* geps, int64_t ldg, float* gs, int acc_gs, int64_t first_wave,
-                                            int64_t nw) {
+// Per bond b: guv[b, 0:C] = sum of gz3 [t_cap, C] (the gradient of z3) over b's triplets as first bond, guv[b, C:2C] as
+// second bond; gs[b] (+)= the same sums of gsw[k, 0] and gsw[k, 1] (stored, or added with acc_gs). A
+// second-bond slot of -1 (no triplet) adds zeros.
+template <int NC>
+__device__ __forceinline__ void bond_sums(const LineCsr& lc, const float* gz3, int64_t ldz, int C, const float* gsw,
+                                          float* guv, int64_t ldg, float* gs, int acc_gs, int64_t first_wave,
+                                          int64_t nw) {
   constexpr int U = bond_pass<NC>(), TQ = kRunBatch;
-  const int64_t second = SPLIT ? 0 : C;  // column of the second bond's block
   const int lane = threadIdx.x & 63;
   const LaneCols<NC> cols(C);
   const int64_t nb = lc.short_offsets[lc.n];
   for (int64_t j0 = first_wave; j0 < nb; j0 += U * nw) {
     const BondSlots<U> bs(lc, j0, nw, nb);
     const float gs_l = acc_gs ? gs[bs.b] : 0.f;
-    float old[U][NC], x[U][2][TQ][NC];
-#pragma unroll
-    for (int q = 0; q < U; ++q)
-#pragma unroll
-      for (int cc = 0; cc < NC; ++cc) old[q][cc] = SPLIT ? 0.f : geps[bs.bond(q) * ldg + cols.col[cc]];
+    float x[U][2][TQ][NC];
     // lane l < 2 U TQ: role l / (U TQ), slot ((l % U TQ) / TQ, l % TQ); role 1 through second_perm
     const int sl = lane % (U * TQ), role_l = lane < U * TQ ? 0 : 1;
     bool empty;
@@ -581,7 +571,7 @@ __device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3,
       for (int t = 0; t < TQ; ++t) {
         const int64_t k = lane_int((int)pl, q * TQ + t);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) x[q][0][t][cc] = ga3[k * lda + cols.col[cc]];
+        for (int cc = 0; cc < NC; ++cc) x[q][0][t][cc] = gz3[k * ldz + cols.col[cc]];
       }
     const int kk = role_l == 0 ? (int)pl : (empty ? -1 : sp);
     const float sw = gsw[2 * (int64_t)(kk >= 0 ? kk : 0) + role_l];
@@ -591,7 +581,7 @@ __device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3,
       for (int t = 0; t < TQ; ++t) {
         const int k = lane_int(kk, U * TQ + q * TQ + t);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) x[q][1][t][cc] = ga3[(int64_t)(k >= 0 ? k : 0) * lda + second + cols.col[cc]];
+        for (int cc = 0; cc < NC; ++cc) x[q][1][t][cc] = gz3[(int64_t)(k >= 0 ? k : 0) * ldz + cols.col[cc]];
       }
 #pragma unroll
     for (int q = 0; q < U; ++q) {
@@ -628,7 +618,7 @@ __device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3,
             const int64_t k = ky[t] >= 0 ? ky[t] : 0;
             sy[t] = gsw[2 * k + role];
 #pragma unroll
-            for (int cc = 0; cc < NC; ++cc) y[t][cc] = ga3[k * lda + role * second + cols.col[cc]];
+            for (int cc = 0; cc < NC; ++cc) y[t][cc] = gz3[k * ldz + cols.col[cc]];
           }
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
@@ -642,33 +632,18 @@ __device__ __forceinline__ void bond_reduce(const LineCsr& lc, const float* ga3,
             gsum = use ? gsum + v : gsum;
           }
         }
-        if constexpr (SPLIT) {
-          if (bs.stored(q)) {
-            float* out = geps + bs.bond(q) * ldg + role * C;
+        if (bs.stored(q)) {
+          float* out = guv + bs.bond(q) * ldg + role * C;
 #pragma unroll
-            for (int cc = 0; cc < NC; ++cc)
-              if (cols.live[cc]) out[cols.col[cc]] = acc[cc];
-          }
-#pragma unroll
-          for (int cc = 0; cc < NC; ++cc) acc[cc] = 0.f;
+          for (int cc = 0; cc < NC; ++cc)
+            if (cols.live[cc]) out[cols.col[cc]] = acc[cc];
         }
-      }
-      if (bs.stored(q)) {
-        const int64_t b = bs.bond(q);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc)
-          if (!SPLIT && cols.live[cc]) geps[b * ldg + cols.col[cc]] = old[q][cc] + acc[cc];
-        if (lane == 0) gs[b] = lane_value(gs_l, q) + gsum;
+        for (int cc = 0; cc < NC; ++cc) acc[cc] = 0.f;
       }
+      if (bs.stored(q) && lane == 0) gs[bs.bond(q)] = lane_value(gs_l, q) + gsum;
     }
   }
-}
-
-template <int NC>
-__global__ void __launch_bounds__(256) tb_bond_reduce_kernel(LineCsr lc, const float* ga3, int64_t lda, int C,
-                                                              const float* gsw, float* geps, int64_t ldg, float* gs,
-                                                              int acc_gs) {
-  bond_reduce<NC, false>(lc, ga3, lda, C, gsw, geps, ldg, gs, acc_gs, wave_id(), (int64_t)gridDim.x * 4);
 }
 
 // out[c] = sum over entries [lo, hi) of row perm[k] (null: row k; negative: none) of v, a wave: G groups of C / 4
@@ -731,7 +706,7 @@ __global__ void __launch_bounds__(256) tb_vjp_sums_kernel(LineCsr lc, const floa
                                                            const float* gsw, float* guv, int64_t ldg, float* gs,
                                                            int acc_gs, const NodeSums ns, int64_t bond_blocks) {
   if ((int64_t)blockIdx.x < bond_blocks) {
-    bond_reduce<NC, true>(lc, gz3, ldz, C, gsw, guv, ldg, gs, acc_gs, wave_id(), bond_blocks * 4);
+    bond_sums<NC>(lc, gz3, ldz, C, gsw, guv, ldg, gs, acc_gs, wave_id(), bond_blocks * 4);
     return;
   }
   const int64_t w = wave_id() - bond_blocks * 4, i = w >> 1;
@@ -1160,19 +1135,6 @@ int fmd_tb_gated_sum_bwd_f32(const float* gout, int64_t ldg, const float* z, int
   return FMD_OK;
 }
 
-int fmd_tb_bond_sum_f32(const float* z3, int64_t ldz, int32_t channels, const float* geo, const int64_t* short_offsets,
-                        const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
-                        int64_t n_atoms, int64_t t_cap, float scale, float* eps, int64_t lde, hipStream_t stream) {
-  FMD_REQUIRE(n_atoms >= 0 && t_cap >= 0 && channels > 0 && channels <= 256 && ldz >= channels && lde >= channels);
-  if (n_atoms == 0 || t_cap == 0) return FMD_OK;
-  FMD_REQUIRE(z3 && geo && short_offsets && bond_rows && edge_triplet_offsets && line_graph && eps);
-  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, nullptr, line_graph, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC2(tb_bond_sum_kernel, false, channels, dim3(kStrideBlocks), lc, const_cast<float*>(z3), ldz, channels,
-                TripletTerms{}, geo, scale, eps, lde);
-  FMD_CHECK_LAUNCH();
-  return FMD_OK;
-}
-
 int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const float* h, int64_t ldh, const float* aw,
                            int64_t lda, int32_t channels, const float* geo, const int64_t* short_offsets,
                            const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
@@ -1183,8 +1145,8 @@ int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const fl
   if (n_atoms == 0 || t_cap == 0) return FMD_OK;
   FMD_REQUIRE(u && v && h && aw && z3 && geo && short_offsets && bond_rows && edge_triplet_offsets && line_graph && eps);
   LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, nullptr, line_graph, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC2(tb_bond_sum_kernel, true, channels, dim3(kStrideBlocks), lc, z3, ldz, channels,
-                (TripletTerms{u, v, h, aw, ldu, ldh, lda}), geo, scale, eps, lde);
+  TB_LAUNCH_NC(tb_bond_sum_kernel, channels, dim3(kStrideBlocks), lc, z3, ldz, channels,
+               (TripletTerms{u, v, h, aw, ldu, ldh, lda}), geo, scale, eps, lde);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }
@@ -1284,21 +1246,6 @@ int fmd_tb_triplet_bwd_f32(const float* geps, int64_t ldg, const float* z3, int6
   LineCsr lc{nullptr, nullptr, nullptr, nullptr, line_graph, pair_offsets, n_atoms, t_cap};
   TB_LAUNCH_NC(tb_triplet_bwd_kernel, channels, dim3(kStrideBlocks), lc, geps, ldg, z3, ldz, channels, geo, scale, gz3,
                ldgz, gsw);
-  FMD_CHECK_LAUNCH();
-  return FMD_OK;
-}
-
-int fmd_tb_bond_reduce_f32(const float* ga3, int64_t lda, int32_t channels, const float* gsw,
-                           const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
-                           const int32_t* second_perm, int64_t n_atoms, int64_t t_cap, float* geps, int64_t ldg,
-                           float* gs, int32_t accumulate_gs, hipStream_t stream) {
-  FMD_REQUIRE(n_atoms >= 0 && t_cap >= 0 && channels > 0 && channels <= 256 && lda >= 2 * channels &&
-              ldg >= channels);
-  if (n_atoms == 0 || t_cap == 0) return FMD_OK;
-  FMD_REQUIRE(ga3 && gsw && short_offsets && bond_rows && edge_triplet_offsets && second_perm && geps && gs);
-  LineCsr lc{short_offsets, bond_rows, edge_triplet_offsets, second_perm, nullptr, nullptr, n_atoms, t_cap};
-  TB_LAUNCH_NC(tb_bond_reduce_kernel, channels, dim3(kStrideBlocks), lc, ga3, lda, channels, gsw, geps, ldg, gs,
-               accumulate_gs);
   FMD_CHECK_LAUNCH();
   return FMD_OK;
 }

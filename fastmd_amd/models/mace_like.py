@@ -41,7 +41,6 @@ from torch.autograd import Function
 from fastmd_amd import _abi
 from fastmd_amd.adapters.protocol import (CapacityStep, CaptureContract, GraphBatch, PaddingRule, TopologySpec,
                                          require_atom_rows, system_rows)
-from fastmd_amd.ops.csr_segment_sum import Csr
 from fastmd_amd.ops.wide_gemm import (Planes, gemm, gemm_gather, gemm_group, gemm_planes, gemm_splitk,
                                      split_planes)
 
@@ -353,8 +352,6 @@ class MaceLike(nn.Module):
 class MaceLikeInput:
     batch: GraphBatch
     elem: Tensor  # int32 [rows] element index of every atom row
-    csr_dst: Csr = field(default=None)
-    csr_src: Csr = field(default=None)
     # the energy launch's completion counter (uint32 [1], zero between launches): the explicit
     # force path forms the float64 total in that launch's last workgroup
     sum_counter: Tensor = field(default=None)
@@ -848,7 +845,7 @@ class MaceLikeAdapter:
 
     def prepare(self, batch: GraphBatch) -> MaceLikeInput:
         """Aliases of the batch plus the element index of every row (host check of the species,
-        outside any graph) and the two CSRs of the edge list."""
+        outside any graph)."""
         if batch.positions is None or batch.edge_offsets is None or batch.edge_reverse is None:
             raise ValueError("the MACE-like model needs an edges-only batch with its CSR (edge_offsets, edge_reverse)")
         require_atom_rows(batch, "MACE-like")
@@ -857,9 +854,7 @@ class MaceLikeAdapter:
         if bool(((species < 1) | (species > _ELEMENTS)).any()) or bool((table[species.clamp(1, _ELEMENTS)] < 0).any()):
             raise ValueError(f"the MACE-like model supports atomic numbers {list(self.module.config.elements)}")
         elem = table[species].to(torch.int32).contiguous()
-        rows = batch.edge_index.shape[0]
-        return MaceLikeInput(batch=batch, elem=elem, csr_dst=Csr(batch.edge_offsets, None, rows),
-                             csr_src=Csr(batch.edge_offsets, batch.edge_reverse, rows),
+        return MaceLikeInput(batch=batch, elem=elem,
                              sum_counter=torch.zeros(1, dtype=torch.int32, device=elem.device))
 
     def node_energy(self, inputs: MaceLikeInput, positions: Tensor, cell: Tensor) -> Tensor:

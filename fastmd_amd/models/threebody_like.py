@@ -162,8 +162,7 @@ class ThreeBodyInput:
     batch: GraphBatch
     line: LineGraph
     elem: Tensor  # int32 [rows]
-    csr_dst: Csr = field(default=None)
-    csr_src: Csr = field(default=None)
+    csr_src: Csr = field(default=None)  # the rows that an atom sends
 
 
 def _call(name, *args):
@@ -369,7 +368,7 @@ class ThreeBodyAdapter:
 
     def prepare(self, batch: GraphBatch) -> ThreeBodyInput:
         """Aliases of the batch and its line graph, the element index of every row (host check of
-        the species, outside any graph) and the two CSRs of the edge list."""
+        the species, outside any graph) and the CSR of the rows by sender."""
         if batch.positions is None or batch.edge_offsets is None or batch.edge_reverse is None:
             raise ValueError("the three-body model needs a fixed-capacity batch with its CSR")
         require_atom_rows(batch, "three-body")
@@ -384,7 +383,7 @@ class ThreeBodyAdapter:
             raise ValueError(f"the three-body model supports atomic numbers {list(self.module.config.elements)}")
         elem = table[species].to(torch.int32).contiguous()
         rows = batch.edge_index.shape[0]
-        return ThreeBodyInput(batch=batch, line=batch.line, elem=elem, csr_dst=Csr(batch.edge_offsets, None, rows),
+        return ThreeBodyInput(batch=batch, line=batch.line, elem=elem,
                               csr_src=Csr(batch.edge_offsets, batch.edge_reverse, rows))
 
     def node_energy(self, inputs: ThreeBodyInput, positions: Tensor, cell: Tensor) -> Tensor:

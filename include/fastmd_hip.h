@@ -263,7 +263,8 @@ int fmd_tb_bond_envelope_f32(float* geo, const uint8_t* short_flags, const int64
                              hipStream_t stream);
 /* out[s] (+)= scale * sum_{r in [offsets[s], offsets[s+1]) and r < rows} silu(z[r]) * w(r),
  * w(r) = w[r], w[index1[r]] or w[index1[r]] * w[index2[r]] (index rows of stride ld_index, w of
- * stride ldw); one wave per segment, rows in order. channels <= 256. */
+ * stride ldw); one wave per segment, rows in order. channels <= 256.
+ * (The model runs fmd_tb_edge_sum_f32, which forms z too; kept with its VJP as the general gated sum.) */
 int fmd_tb_gated_sum_f32(const float* z, int64_t ldz, int64_t rows, int32_t channels, const float* w, int64_t ldw,
                          const int32_t* index1, const int32_t* index2, int64_t ld_index, const int64_t* offsets,
                          int64_t n_segments, float scale, float* out, int64_t ldo, int32_t accumulate,
@@ -281,33 +282,23 @@ int fmd_tb_gated_sum_bwd_f32(const float* gout, int64_t ldg, const float* z, int
  * second bond the same run through second_perm), a fixed grid striding over the real bonds /
  * triplets, every sum in triplet order. The reference's triplet gather + segment sums
  * (fastmd/models/matris/op/triton_weighted_segment_sum.py, triton_csr_segment_sum.py:433-479).
- * Forward: eps[b] += scale * sum over b's triplets k of silu(z3[k]) s_b s_b2 (s = geo column 6). */
-int fmd_tb_bond_sum_f32(const float* z3, int64_t ldz, int32_t channels, const float* geo, const int64_t* short_offsets,
-                        const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
-                        int64_t n_atoms, int64_t t_cap, float scale, float* eps, int64_t lde, hipStream_t stream);
-/* VJP per triplet: gz3[k] = scale geps[b1] s_b1 s_b2 silu'(z3[k]) (0 past the real triplets) and
- * the envelope terms gsw [t_cap, 2] = (gw s_b2, gw s_b1), gw = sum_c scale geps[b1] silu(z3[k]). */
-int fmd_tb_triplet_bwd_f32(const float* geps, int64_t ldg, const float* z3, int64_t ldz, int32_t channels,
-                           const float* geo, const int32_t* line_graph, const int64_t* pair_offsets, int64_t n_atoms,
-                           int64_t t_cap, float scale, float* gz3, int64_t ldgz, float* gsw, hipStream_t stream);
-/* VJP per bond: geps[b] += sum over b's triplets as first bond of ga3[k, 0:C] + as second bond of
- * ga3[k, C:2C] (ga3 = gz3 [W_b1; W_b2]^T); gs[b] = (or += with accumulate_gs) the same sums of
- * gsw[k, 0] and gsw[k, 1]. Rows that are no bond are not written. */
-int fmd_tb_bond_reduce_f32(const float* ga3, int64_t lda, int32_t channels, const float* gsw,
-                           const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
-                           const int32_t* second_perm, int64_t n_atoms, int64_t t_cap, float* geps, int64_t ldg,
-                           float* gs, int32_t accumulate_gs, hipStream_t stream);
-/* fmd_tb_bond_sum_f32 with the pre-activation formed and stored on the way: z3[k] = u[b1] + v[b2] +
- * h[atom] + aw[k] over the real triplets (b1, b2, atom of line_graph; u, v rows of stride ldu). */
+ * Forward: eps[b] += scale * sum over b's triplets k of silu(z3[k]) s_b s_b2 (s = geo column 6), with
+ * the pre-activation formed and stored on the way: z3[k] = u[b1] + v[b2] + h[atom] + aw[k] over the real
+ * triplets (b1, b2, atom of line_graph; u, v rows of stride ldu). */
 int fmd_tb_bond_update_f32(const float* u, const float* v, int64_t ldu, const float* h, int64_t ldh, const float* aw,
                            int64_t lda, int32_t channels, const float* geo, const int64_t* short_offsets,
                            const int32_t* bond_rows, const int64_t* edge_triplet_offsets, const int32_t* line_graph,
                            int64_t n_atoms, int64_t t_cap, float scale, float* z3, int64_t ldz, float* eps, int64_t lde,
                            hipStream_t stream);
-/* The sums of a layer's VJP in one launch. Per bond those of fmd_tb_bond_reduce_f32 of gz3 [t_cap, C] itself,
- * kept apart: guv[b] = (sum as first bond | sum as second bond) [., 2 C], stored on every bond row; gs as there. Per
- * atom s_src[i] = sum of gz2 [e_cap, C] over the rows reverse[offsets[i] .. offsets[i + 1]) (negative entries
- * skipped) and s_tri[i] = sum of gz3 over its triplets. channels a multiple of 64; t_cap > 0; gz3, gz2, s_src,
+/* VJP per triplet: gz3[k] = scale geps[b1] s_b1 s_b2 silu'(z3[k]) (0 past the real triplets) and
+ * the envelope terms gsw [t_cap, 2] = (gw s_b2, gw s_b1), gw = sum_c scale geps[b1] silu(z3[k]). */
+int fmd_tb_triplet_bwd_f32(const float* geps, int64_t ldg, const float* z3, int64_t ldz, int32_t channels,
+                           const float* geo, const int32_t* line_graph, const int64_t* pair_offsets, int64_t n_atoms,
+                           int64_t t_cap, float scale, float* gz3, int64_t ldgz, float* gsw, hipStream_t stream);
+/* The sums of a layer's VJP in one launch. Per bond guv[b] = (sum of gz3 [t_cap, C] over b's triplets as first bond |
+ * as second bond) [., 2 C], stored on every bond row, and gs[b] = (or += with accumulate_gs) the same sums of gsw[k, 0]
+ * and gsw[k, 1]; rows that are no bond are not written. Per atom s_src[i] = sum of gz2 [e_cap, C] over the rows
+ * reverse[offsets[i] .. offsets[i + 1]) (negative entries skipped) and s_tri[i] = sum of gz3 over its triplets. channels a multiple of 64; t_cap > 0; gz3, gz2, s_src,
  * s_tri 16-byte aligned, strides multiples of 4. */
 int fmd_tb_vjp_sums_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
                         const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
@@ -351,7 +342,8 @@ int fmd_tb_readout_bwd_f32(const float* gE, float sign, const float* wr, int32_t
                            int64_t ldgh, hipStream_t stream);
 /* gvec [e_cap, 3] = gr u + (gu - (gu . u) u) / r per real row (0 on padding), gr = sum_n gef def +
  * gfc dfc + gs ds (each term nullable); with bond_flags (nullable) gu and gs are read on the flagged
- * rows only (the bonds of a line graph, the rows the three-body VJP writes). */
+ * rows only (the bonds of a line graph, the rows the three-body VJP writes). The row gradients that
+ * fmd_tb_edge_forces_f32 sums, and its reference in the tests. */
 int fmd_tb_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, const float* gef, int64_t ldgef,
                             const float* gu, int64_t ldgu, const float* gfc, const float* gs, const uint8_t* bond_flags,
                             const int64_t* n_edges, int64_t e_cap, float* gvec, hipStream_t stream);
@@ -670,7 +662,8 @@ int fmd_sum_f64(const void* x, int32_t x_is_f64, int64_t n, double* out, hipStre
 int fmd_edge_geometry_f32(const float* positions, const float* cell, const int32_t* system_of,
                           const int32_t* edge_index, const float* edge_image, const int64_t* n_edges, int64_t e_cap,
                           float rc, int32_t nb, float* geo, float* ef, float* def, hipStream_t stream);
-/* gvec[e] = dE/dvec from dE/def (up to two sources, row strides ld0/ld1) and dE/d(u, fcut) (ggeo [E,4]). */
+/* gvec[e] = dE/dvec from dE/def (up to two sources, row strides ld0/ld1) and dE/d(u, fcut) (ggeo [E,4]): the row
+ * gradients that fmd_edge_forces_f32 sums, and its reference in the tests. */
 int fmd_edge_geometry_bwd_f32(const float* geo, const float* def, int32_t nb, const float* gef0, int64_t ld0,
                               const float* gef1, int64_t ld1, const float* ggeo, const int64_t* n_edges,
                               int64_t e_cap, float* gvec, hipStream_t stream);
