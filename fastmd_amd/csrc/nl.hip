@@ -214,7 +214,7 @@ struct QueryArgs {
   uint8_t* capacity_valid;
   int64_t system_size;
   int64_t index_offset;
-  float full;  // (the sphere's volume / the share of the cell's cells within reach) / the wave form's keys
+  int32_t full;  // atoms in the cells within reach from which the wave form leaves an atom unsearched
 };
 
 // The slots of atom i that a search writes, [0, end): its candidates and then the pad value, up to
@@ -319,14 +319,24 @@ __device__ __forceinline__ void query_atom(const QueryArgs& a, int64_t i, uint64
   }
 }
 
-// The workgroup form for every atom, or (SPARSE) for those left over by the wave form, `per` atoms of a
-// workgroup in turn: at most 16, and few enough that kSparseGroups workgroups share them, since a slab or a cluster
-// in vacuum may hold nothing else. Slabs of 320 candidates per atom, refreshed: 4 000 atoms 1 190 us with 16 in
-// turn, 395 with one; 20 000 atoms 2 030 with 16, 1 640 with 9 (2 048 workgroups), 1 390 with 4. Workgroups with
-// nothing to do cost their launch (a crystal of 40 000 atoms 132 us with 16 in turn, 134 with 9).
+// The workgroup form for every atom, or (SPARSE) for those left over by the wave form where that does not search
+// them itself, `per` atoms of a workgroup in turn: at most 16, and few enough that kSparseGroups workgroups share
+// them, since a slab or a cluster in vacuum may hold nothing else. Refreshes of slabs of 320 candidates per atom: 4 000
+// atoms 1 190 us with 16 in turn, 390 with one; 20 000 atoms 2 030 with 16, 1 640 with 9, 1 400 with 4. Workgroups
+// with nothing to do cost their launch (a crystal of 40 000 atoms: 10 000 of them 1 us more than 2 500), so fewer share
+// them where the mean row (kSparseRow) makes rows past the keys unlikely: five a CU, all resident. In a cluster in
+// so much vacuum 40 000 atoms of 360 candidates take 2 290 us, 2 010 with 4 096 workgroups.
 constexpr int kWaveKeys = 256;  // candidate keys of a wave
 constexpr int kSparseAtoms = 16;
-constexpr int64_t kSparseGroups = 4096;
+constexpr int64_t kSparseGroups = 4096, kFewGroups = 1280;
+constexpr double kSparseRow = 64.;
+constexpr int kAtoms = 256 / FMD_WAVE;  // atoms of a workgroup of the wave form
+constexpr int kWaveLds = kAtoms * (kWaveKeys * 8 + 3 * FMD_WAVE * 4);
+// The wave form's workgroups search what they leave over themselves, without the second launch, up to so many atoms and
+// LDS keys: 135 atoms 32.2 -> 31 us of a refresh, 5 000 57.8 -> 57.4; 20 480 96 -> 99 (the workgroup's last
+// wave holds its LDS, which is half as large again), so not there.
+constexpr int64_t kRestAtoms = 8192;
+constexpr int kRestKeys = 2048;
 
 template <bool SPARSE>
 __global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a, int per) {
@@ -349,30 +359,25 @@ __global__ void __launch_bounds__(256) cells_query_kernel(const QueryArgs a, int
 // each lane finding its cell in the scanned counts, so that every lane tests an atom and the loads of
 // a pass go out together; candidate keys appended to the wave's LDS list by ballot. The list is put in
 // order by rank: a key's slot is the number of smaller keys (up to four keys per lane against the list,
-// read as LDS broadcasts), written straight to the row. More than kWaveKeys candidates, found or expected: the
-// search ends there, with a count above kWaveKeys for the workgroup form. Bound by the latency of its loads (27
-// cells, 320 atoms per atom at 40 000): 40 000 atoms 487 -> 65 us with the rows' unused slots no longer written.
-__global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a) {
-  __shared__ uint64_t s_keys[256 / FMD_WAVE][kWaveKeys];
-  __shared__ int32_t s_first[256 / FMD_WAVE][FMD_WAVE];  // scanned atom counts of the wave's 64 cells
-  __shared__ int32_t s_start[256 / FMD_WAVE][FMD_WAVE];
-  __shared__ uint32_t s_shift[256 / FMD_WAVE][FMD_WAVE];
+// read as LDS broadcasts), written straight to the row. More than kWaveKeys candidates: the count alone, for the
+// workgroup form, unsearched where the cells within reach are so full that it is to be expected. Bound by the
+// latency of its loads (27 cells, 320 atoms per atom at 40 000): 40 000 atoms 487 -> 65 us with the rows'
+// unused slots no longer written.
+// leave: whether num_neighbors tells of an atom left over; returns false for one.
+__device__ __forceinline__ bool query_wave(const QueryArgs& a, int64_t i, uint64_t* lds, bool leave) {
   const int lane = threadIdx.x & (FMD_WAVE - 1), wave = threadIdx.x / FMD_WAVE;
-  const int64_t i = (int64_t)blockIdx.x * (256 / FMD_WAVE) + wave;
-  if (i >= a.n) return;  // no barrier below: every wave works on its own share of the LDS
-  uint64_t* keys = s_keys[wave];
-  int32_t *first = s_first[wave], *start = s_start[wave];
-  uint32_t* shift = s_shift[wave];
+  // no barrier below: every wave works on its own share of the LDS
+  uint64_t* keys = lds + wave * kWaveKeys;
+  int32_t* first = reinterpret_cast<int32_t*>(lds + kAtoms * kWaveKeys) + wave * 3 * FMD_WAVE;  // scanned atom counts
+  int32_t* start = first + FMD_WAVE;                                                            // of 64 cells
+  uint32_t* shift = reinterpret_cast<uint32_t*>(start + FMD_WAVE);
   const Mat3 cm = load_mat3(a.cell);
   const float xi = a.wrapped[3 * i], yi = a.wrapped[3 * i + 1], zi = a.wrapped[3 * i + 2];
   const int c0 = cell_coord(a.frac[3 * i], a.n0), c1 = cell_coord(a.frac[3 * i + 1], a.n1),
             c2 = cell_coord(a.frac[3 * i + 2], a.n2);
   const int span1 = 2 * a.r1 + 1, span2 = 2 * a.r2 + 1, noff = (2 * a.r0 + 1) * span1 * span2;
-  const float volume = fabsf(cm.m[0] * (cm.m[4] * cm.m[8] - cm.m[5] * cm.m[7]) -
-                             cm.m[1] * (cm.m[3] * cm.m[8] - cm.m[5] * cm.m[6]) +
-                             cm.m[2] * (cm.m[3] * cm.m[7] - cm.m[4] * cm.m[6]));
   int count = 0;
-  for (int q0 = 0; q0 < noff && count <= kWaveKeys; q0 += FMD_WAVE) {
+  for (int q0 = 0; q0 < noff; q0 += FMD_WAVE) {
     const int q = q0 + lane;
     int from = 0, atoms = 0;
     uint32_t packed = 0;
@@ -402,12 +407,11 @@ __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const int total = __shfl(incl, FMD_WAVE - 1, FMD_WAVE);
-    // cells so full that the sphere's share of them passes the keys: left to the workgroup form unsearched
-    if (noff <= FMD_WAVE && (float)total * a.full > volume) {
+    if (total > a.full && noff <= FMD_WAVE) {
       count = kWaveKeys + 1;
       break;
     }
-    for (int f0 = 0; f0 < total && count <= kWaveKeys; f0 += FMD_WAVE) {
+    for (int f0 = 0; f0 < total; f0 += FMD_WAVE) {
       const int f = f0 + lane;
       bool hit = false;
       uint64_t key = 0;
@@ -470,9 +474,32 @@ __global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a
       srow[3 * s] = srow[3 * s + 1] = srow[3 * s + 2] = 0;
     }
   }
-  if (lane == 0) {
+  if (lane == 0 && (fits || leave)) {
     a.num_neighbors[i] = count;
     if (fits && count > a.bmax) a.capacity_valid[0] = 0;  // else the workgroup form's to say
+  }
+  return fits;
+}
+
+// REST: the atoms left over are searched by their workgroup at once.
+template <bool REST>
+__global__ void __launch_bounds__(256) cells_query_wave_kernel(const QueryArgs a) {
+  const int wave = threadIdx.x / FMD_WAVE;
+  const int64_t i0 = (int64_t)blockIdx.x * kAtoms;
+  if constexpr (!REST) {
+    __shared__ uint64_t lds[kWaveLds / 8];
+    if (i0 + wave < a.n) query_wave(a, i0 + wave, lds, true);
+    return;
+  }
+  extern __shared__ uint64_t keys[];
+  __shared__ int s_left[kAtoms];
+  const bool left = i0 + wave < a.n && !query_wave(a, i0 + wave, keys, false);
+  if ((threadIdx.x & (FMD_WAVE - 1)) == 0) s_left[wave] = left;
+  __syncthreads();
+  for (int k = 0; k < kAtoms; ++k) {
+    if (!s_left[k]) continue;
+    query_atom(a, i0 + k, keys);
+    __syncthreads();  // keys and counter are free
   }
 }
 
@@ -1376,23 +1403,32 @@ int fmd_nl_candidates_pad(const float* wrapped, const float* frac, const float* 
   FMD_CHECK_LAUNCH();
   QueryArgs a{wrapped, frac, cell, n_atoms, cutoff2, n0, n1, n2, r0, r1, r2, bmax, lcap, pad_mode, cell_start, cell_atoms,
               neighbor_matrix, neighbor_shifts, num_neighbors, capacity_valid, system_size, index_offset};
-  a.full = (float)(4.18879 * (double)cutoff2 * sqrt((double)cutoff2) * (double)ncell /
-                   ((2. * r0 + 1) * (2. * r1 + 1) * (2. * r2 + 1) * kWaveKeys));
   const size_t lds = (size_t)lcap * sizeof(uint64_t);
   // The wave form where three quarters of its keys hold a row at the mean density: the sphere has 4.19 cutoffs cubed,
   // and a cell is at least 1 / reach of a cutoff thick along an axis of one cell, the cutoff along others. An upper
   // bound at that density, since a cell is up to two cutoffs thick; the workgroup form above it, which searches
   // a long row once (a bound without the reach sent 40 atoms in a 9 A cell, 404 candidates within 12 A, through
   // both: 470 us, 46 now). Rows past the keys at a lower mean density go to the workgroup form after the wave form.
-  double row = 4.19 * (double)n_atoms / (double)ncell;
-  for (int k = 0; k < 3; ++k) row *= ncells[k] == 1 && reach[k] > 1 ? reach[k] : 1;
+  double sphere = 4.19, cells = 1.;  // in cells; the cells within reach
+  for (int k = 0; k < 3; ++k) {
+    sphere *= ncells[k] == 1 && reach[k] > 1 ? reach[k] : 1;
+    cells *= 2. * reach[k] + 1.;
+  }
+  const double row = sphere * (double)n_atoms / (double)ncell;
+  // the sphere's share of as many atoms passes the keys by a quarter (by less in thicker cells)
+  a.full = (int32_t)fmin(1.25 * kWaveKeys * cells / sphere, 2147483647.);
   if (row <= 0.75 * kWaveKeys) {
-    hipLaunchKernelGGL(cells_query_wave_kernel, dim3((unsigned)fmd_cdiv(n_atoms, 256 / FMD_WAVE)), dim3(256), 0, stream,
-                       a);
+    const dim3 grid((unsigned)fmd_cdiv(n_atoms, kAtoms));
+    if (lcap <= kRestKeys && n_atoms <= kRestAtoms) {
+      hipLaunchKernelGGL(cells_query_wave_kernel<true>, grid, dim3(256), lds > kWaveLds ? lds : kWaveLds, stream, a);
+      FMD_CHECK_LAUNCH();
+      return FMD_OK;
+    }
+    hipLaunchKernelGGL(cells_query_wave_kernel<false>, grid, dim3(256), 0, stream, a);
     FMD_CHECK_LAUNCH();
     a.pad_mode = pad_mode == FMD_NL_PAD_NONE ? FMD_NL_PAD_NONE : FMD_NL_PAD_ALL;  // the old counts are gone
-    const int64_t per = n_atoms / kSparseGroups < 1 ? 1 : n_atoms / kSparseGroups < kSparseAtoms ? n_atoms / kSparseGroups
-                                                                                                : kSparseAtoms;
+    const int64_t share = n_atoms / (row < kSparseRow ? kFewGroups : kSparseGroups);
+    const int64_t per = share < 1 ? 1 : share < kSparseAtoms ? share : kSparseAtoms;
     hipLaunchKernelGGL(cells_query_kernel<true>, dim3((unsigned)fmd_cdiv(n_atoms, per)), dim3(256), lds, stream, a,
                        (int)per);
   } else {
