@@ -24,8 +24,8 @@ from fastmd_amd._device import require_cuda, rows_view, stream
 _EPILOGUES = {None: 0, "none": 0, "silu": 1}
 
 
-# A float32 gemm splits its B into the bf16 planes beforehand (one launch, about 4 us for a weight of some 1 000 x 1 000)
-# and runs on the split-plane kernel with fp32 A:
+# A float32 gemm splits its B into the bf16 planes beforehand (one launch, 5 us for a weight of 1 000 x 1 000, 24 for 4 000
+# x 2 000) and runs on the split-plane kernel with fp32 A:
 # * b [K, N]: from 256 tiles of 128 x 128, as the b [N, K] kernel that splits both operands, where _planes_pay
 #   (the fp32 MFMA form takes 2 217 us at [160 000, 1 024] x [1 024, 520], this one 1 060, 153 against 100 us with
 #   10 000 rows; with 125 tiles, [16 000, 384] x [384, 128], 29 against 37);
@@ -45,12 +45,12 @@ def _takes_planes(m: int, n: int, k: int, b_layout: int) -> bool:
 
 
 def _planes_pay(m: int, n: int, k: int, b_layout: int) -> bool:
-    """Whether it is the faster form there. b [K, N] (us, fp32 MFMA against planes): from 512 tiles, where the fp32 form
-    goes over to tiles of 128 x 128, always ([70 000, 20] x [20, 40] 30 / 14) but for the fewest rows, which the
-    split costs more than it saves ([100, 264] x [264, 70 000] 0.8 of the time, [300, 64] x [64, 32 768] 1.2 times it).
+    """Whether it is the faster form there (r: the fp32 form's time over this one's). b [K, N]: from 512 tiles, where
+    the fp32 form goes over to tiles of 128 x 128, always (r = 2.1 for [70 000, 20] x [20, 40]) but for the fewest rows,
+    which the split costs more than it saves (r = 0.8 for [100, 264] x [264, 70 000], 1.2 for [300, 64] x [64, 32 768]).
     Between 256 and 511 tiles (64 x 64 there) the split's launch and a last column tile that is not whole blocks of
-    32 have to be earned: [32 836, K] x [K, 40] 8.4 / 12.5 at K = 20, 28.4 / 26.2 at 264; x [K, 136] 0.95 of the time at
-    K = 32, 1.11 at 48; x [K, 256] 1.16 at 20."""
+    32 have to be earned: [32 836, K] x [K, 40] r = 0.69 at K = 20, 1.06 at 264; [16 452, K] x [K, 136] 0.95 at K = 32, 1.11
+    at 48; [16 452, 20] x [20, 256] 1.16."""
     if b_layout == 0:
         return m >= PLANES_MIN_ROWS
     tiles = -(-m // 128) * -(-n // 128)

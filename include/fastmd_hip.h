@@ -298,8 +298,8 @@ int fmd_tb_triplet_bwd_f32(const float* geps, int64_t ldg, const float* z3, int6
 /* The sums of a layer's VJP in one launch. Per bond guv[b] = (sum of gz3 [t_cap, C] over b's triplets as first bond |
  * as second bond) [., 2 C], stored on every bond row, and gs[b] = (or += with accumulate_gs) the same sums of gsw[k, 0]
  * and gsw[k, 1]; rows that are no bond are not written. Per atom s_src[i] = sum of gz2 [e_cap, C] over the rows
- * reverse[offsets[i] .. offsets[i + 1]) (negative entries skipped) and s_tri[i] = sum of gz3 over its triplets. channels a multiple of 64; t_cap > 0; gz3, gz2, s_src,
- * s_tri 16-byte aligned, strides multiples of 4. */
+ * reverse[offsets[i] .. offsets[i + 1]) (negative entries skipped) and s_tri[i] = sum of gz3 over its triplets.
+ * channels a multiple of 64; t_cap > 0; gz3, gz2, s_src, s_tri 16-byte aligned, strides multiples of 4. */
 int fmd_tb_vjp_sums_f32(const float* gz3, int64_t ldz, int32_t channels, const float* gsw,
                         const int64_t* short_offsets, const int32_t* bond_rows, const int64_t* edge_triplet_offsets,
                         const int32_t* second_perm, const int64_t* pair_offsets, int64_t n_atoms, int64_t t_cap,
